@@ -569,10 +569,14 @@ extern "C" __global__ void __launch_bounds__(256) OutlierKnl(
   // thousand features of five tiles per workgroup took 69.6 us that way, 68.6 us with the
   // round trip in the open).  When every tile is drawn, the first ticket is asked for ahead
   // of the binding.
-  rfx::TailTickets *const d_tickets = d_outliers;
+  const rfx::TailDraw d_tickets{{d_outliers, xcd}};
   __shared__ int s_ticket[2];
+  // A workgroup's first tile is dealt in any case: it is there without a draw, and a batch of one
+  // pass or less draws nothing (every workgroup asking for a ticket to learn that there are no
+  // tiles left: 1 000 features, one sample 13.1 us, 37 samples 28.4; without 9.2 and 20.8 us).
   const int static_last = DRAWN_TAIL >= RFX_DRAWN_ALL ? 0 :
-      static_cast<int>(max(0ll, walk_last - static_cast<long long>(DRAWN_TAIL) * walk_step));
+      static_cast<int>(max(static_cast<long long>(min(walk_last, walk_step)),
+                           walk_last - static_cast<long long>(DRAWN_TAIL) * walk_step));
   int walk = walk_first, ticket_slot = 0, next_ticket = 0;
   bool drawing = false;
   for (;;) {{
@@ -582,6 +586,7 @@ extern "C" __global__ void __launch_bounds__(256) OutlierKnl(
         at = walk;
         walk += walk_step;
       }} else {{
+        if (static_last >= walk_last) break;
         drawing = true;
         if (threadIdx.x == 0)
           s_ticket[0] = DRAWN_TAIL >= RFX_DRAWN_ALL ? first_ticket : rfx::draw_tail_ticket(d_tickets, xcd);
@@ -590,7 +595,11 @@ extern "C" __global__ void __launch_bounds__(256) OutlierKnl(
     }} else {{
       __syncthreads();                         // the ticket is there, the previous tile is done
       at = static_last + s_ticket[ticket_slot];
-      if (at >= walk_last) break;
+      if (at >= walk_last) {{
+        // the counter's last ticket (walk_step workgroups share it): back to zero
+        if (threadIdx.x == 0 && at == walk_last + walk_step - 1) rfx::tail_tickets_done(d_tickets);
+        break;
+      }}
       if (threadIdx.x == 0) next_ticket = rfx::draw_tail_ticket(d_tickets, xcd);
       ticket_slot ^= 1;
     }}
@@ -605,10 +614,6 @@ extern "C" __global__ void __launch_bounds__(256) OutlierKnl(
     }}
 '''
             loop_tail = '''    if (drawing && threadIdx.x == 0) s_ticket[ticket_slot] = next_ticket;
-'''
-            outlier_end = '''
-  __syncthreads();
-  if (threadIdx.x == 0) rfx::tail_tickets_done(d_tickets);
 '''
         drain_func = f'''
 // Sums mid-size bags from the workgroup's list for as long as the calling wavefront gets one.

@@ -126,26 +126,37 @@ template <typename Space> __device__ __forceinline__ void outliers_done(Space *s
 // cheap tiles last (a model of a thousand small features, five tiles per workgroup: 70.2 ->
 // 67.8 us; alone, or on a model of 100 features with ten tiles per workgroup, nothing).  One
 // thread draws, the next ticket is requested before the current tile runs, the workgroup agrees
-// through LDS; the last workgroup to finish puts the counters back to zero.
+// through LDS.
+//
+// Who puts a counter back to zero for the next launch: every workgroup draws until a ticket lies
+// beyond the last tile, and exactly one of its tickets does.  A counter that W workgroups share
+// over N tiles therefore hands out the tickets 0 .. N + W - 1 and no others, and whoever holds
+// N + W - 1 knows that nobody draws any more.  (A counter of finished workgroups told the same
+// before: one device-scope add per workgroup to a single address, 11 ns each one after the
+// other, 14 us for 1 280 workgroups -- most of a small batch's kernel: 100 features, 8 samples
+// 22.7 us with it, 11.1 us without; 2 048 samples 126.0 and 123.2 us.)
 // ---------------------------------------------------------------------------------------------
 struct TailTickets {
   int next[8][32];                           // per XCD, each on a cache line of its own
-  int finished;                              // workgroups that are done
-  int pad[31];
 };
 
 __device__ __forceinline__ int draw_tail_ticket(TailTickets *t, const int xcd) {
   return __hip_atomic_fetch_add(&t->next[xcd][0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// by one thread of every workgroup when it has drawn its last ticket
-__device__ __forceinline__ void tail_tickets_done(TailTickets *t) {
-  const int done = __hip_atomic_fetch_add(&t->finished, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (done == static_cast<int>(gridDim.x) - 1) {
-    for (int x = 0; x < 8; ++x)
-      __hip_atomic_store(&t->next[x][0], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(&t->finished, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
+// the tickets as one workgroup sees them: it draws from one counter only
+struct TailDraw {
+  TailTickets *tickets;
+  int counter;
+};
+
+__device__ __forceinline__ int draw_tail_ticket(const TailDraw &d, const int xcd) {
+  return draw_tail_ticket(d.tickets, xcd);
+}
+
+// by one thread of the workgroup that holds the last ticket of its counter
+__device__ __forceinline__ void tail_tickets_done(const TailDraw &d) {
+  __hip_atomic_store(&d.tickets->next[d.counter][0], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 } // namespace rfx
