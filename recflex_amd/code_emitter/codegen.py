@@ -297,7 +297,9 @@ constexpr int MAX_LONG_DIM = {max_long_dim};
 constexpr int DRAWN_TAIL = RFX_DRAWN_TAIL;
 static_assert(!(OUTLIERS && DRAWN_TAIL > 0), "one or the other");
 using OutlierSpace = {"rfx::TailTickets" if drawn_tail else f"rfx::OutlierSpace<MAX_LONG_DIM, {outlier_capacity(num_feats)}>"};
-constexpr long long OUTLIER_BYTES = OUTLIERS || DRAWN_TAIL > 0 ? (long long)sizeof(OutlierSpace) : 0LL;
+// (the ticket counters of the outlier parts come right ahead of their list)
+constexpr long long TICKET_BYTES = OUTLIERS ? (long long)sizeof(rfx::OutlierTickets) : 0LL;
+constexpr long long OUTLIER_BYTES = OUTLIERS || DRAWN_TAIL > 0 ? TICKET_BYTES + (long long)sizeof(OutlierSpace) : 0LL;
 #define RFX_TILE_ORDER {1 if tile_order is not None else 0}
 // the binding table of a model that is bound once per launch (rfx::bind_once) comes last
 constexpr long long BOUND_OFFSET = (SPLIT_BYTES + OUTLIER_BYTES + 255) / 256 * 256;
@@ -471,8 +473,8 @@ extern "C" __global__ void __launch_bounds__(1024) BindKnl(
 ''' if bind_once else ''
 
         outlier_kernel = f'''
-// Finds the bags that are too long for their feature's schedule (one thread per bag).
-extern "C" __global__ void __launch_bounds__(256) OutlierKnl(
+// Finds the bags that are too long for their feature's schedule.
+extern "C" __global__ void __launch_bounds__(rfx::kFindThreads) OutlierKnl(
     const int64_t *__restrict__ d_io_ptrs, const char *__restrict__ d_arg_buffers,
     const int64_t *__restrict__ d_arg_buffer_offsets, const int batch,
     OutlierSpace *__restrict__ d_outliers) {{
@@ -483,7 +485,8 @@ extern "C" __global__ void __launch_bounds__(256) OutlierKnl(
 ''' if outliers else ''
         outlier_begin = f'''
   // the parts of the outlier bags of this batch (0: none, or more than the list holds)
-  const int outlier_tiles = rfx::outlier_parts(d_outliers);
+  const rfx::OutlierDraw outlier_draw = rfx::outlier_draw(d_outliers);
+  const int outlier_tiles = outlier_draw.parts;
   const int total_tiles = regular_tiles;
   // mid-size bags wait here for a wavefront of this workgroup
   __shared__ rfx::MidBagQueue s_mid_queue;
@@ -526,16 +529,23 @@ extern "C" __global__ void __launch_bounds__(256) OutlierKnl(
     else
       __builtin_amdgcn_s_sleep(8);
   }}
-  if (outlier_tiles > 0) {{
+  // (also for a list that overflowed and is not used: its header is put back to zero this way)
+  if (outlier_draw.listed) {{
     __shared__ int s_ticket[2];
     int slot = 0;
-    if (threadIdx.x == 0) s_ticket[0] = rfx::draw_outlier_part(d_outliers);
+    if (threadIdx.x == 0) s_ticket[0] = rfx::draw_outlier_ticket(outlier_draw);
     for (;;) {{
       __syncthreads();
-      const int tile = s_ticket[slot];
-      if (tile >= outlier_tiles) break;
+      const int ticket = s_ticket[slot];
+      const int tile = outlier_draw.part_of(ticket);
+      if (tile >= outlier_tiles) {{
+        if (threadIdx.x == 0 && outlier_draw.is_last(ticket) &&
+            rfx::outlier_counter_done(d_outliers, outlier_draw))
+          rfx::outliers_done(d_outliers);
+        break;
+      }}
       int next = 0;
-      if (threadIdx.x == 0) next = rfx::draw_outlier_part(d_outliers);
+      if (threadIdx.x == 0) next = rfx::draw_outlier_ticket(outlier_draw);
       const int entry = d_outliers->partmap[tile];
       const rfx::OutlierEntry e = d_outliers->entries[entry];
       const int part = tile - e.first;
@@ -549,9 +559,9 @@ extern "C" __global__ void __launch_bounds__(256) OutlierKnl(
       slot ^= 1;
       if (threadIdx.x == 0) s_ticket[slot] = next;
     }}
+  }} else if (blockIdx.x == 0 && threadIdx.x == 0) {{
+    rfx::no_outliers(d_outliers);
   }}
-  __syncthreads();
-  if (threadIdx.x == 0) rfx::outliers_done(d_outliers);
 ''' if outliers else ''
         drawn_begin = ''
         if drawn_tail:
@@ -735,7 +745,7 @@ static int launch_kernels(const recom_process_args *a, void *workspace) {
   const char *arg_buffers = static_cast<const char *>(a->d_arg_buffers);
   int batch = a->batch, tile_arg = tile_bytes, xcd_arg = xcd_segments;
   int stride_arg = static_cast<int>(row_stride);
-  void *outlier_space = OUTLIERS || DRAWN_TAIL > 0 ? static_cast<char *>(workspace) + SPLIT_BYTES : nullptr;
+  void *outlier_space = OUTLIERS || DRAWN_TAIL > 0 ? static_cast<char *>(workspace) + SPLIT_BYTES + TICKET_BYTES : nullptr;
   void *bound = BIND_ONCE ? static_cast<char *>(workspace) + BOUND_OFFSET : nullptr;
   // The caller's events take the begin of the call's first kernel and the end of its last
   // (the fused kernel): a library that launches a kernel ahead of the fused one is timed whole.
@@ -752,9 +762,11 @@ static int launch_kernels(const recom_process_args *a, void *workspace) {
   {
     void *outlier_args[] = {const_cast<int64_t **>(&a->d_io_ptrs), &arg_buffers,
                             const_cast<int64_t **>(&a->d_arg_buffer_offsets), &batch, &outlier_space};
-    const unsigned gx = static_cast<unsigned>((batch + 255) / 256 > 64 ? 64 : (batch + 255) / 256);
+    constexpr int kFindRound = rfx::kFindThreads * rfx::kFindBags;
+    const int rounds = batch / kFindRound + (batch % kFindRound ? 1 : 0);
+    const unsigned gx = static_cast<unsigned>(rounds > 64 ? 64 : rounds);
     const unsigned gy = static_cast<unsigned>(NUM_FEATS > 1024 ? 1024 : NUM_FEATS);
-    e = launch(reinterpret_cast<const void *>(OutlierKnl), dim3(gx, gy), dim3(256), outlier_args, 0, false);
+    e = launch(reinterpret_cast<const void *>(OutlierKnl), dim3(gx, gy), dim3(rfx::kFindThreads), outlier_args, 0, false);
     if (e != hipSuccess) return static_cast<int>(e);
   }
 #endif
@@ -825,7 +837,9 @@ extern "C" __global__ void __launch_bounds__(256) ScratchClearKnl(char *__restri
 #endif
 #if RFX_OUTLIERS
   if (blockIdx.y == 0) {
-    OutlierSpace *sp = reinterpret_cast<OutlierSpace *>(ws + SPLIT_BYTES);
+    int *tickets = reinterpret_cast<int *>(ws + SPLIT_BYTES);
+    for (int i = first; i < static_cast<int>(TICKET_BYTES / 4); i += step) tickets[i] = 0;
+    OutlierSpace *sp = reinterpret_cast<OutlierSpace *>(ws + SPLIT_BYTES + TICKET_BYTES);
     int *hdr = reinterpret_cast<int *>(&sp->hdr);
     for (int i = first; i < static_cast<int>(sizeof(rfx::OutlierHeader) / 4); i += step) hdr[i] = 0;
     for (int i = first; i < OutlierSpace::kCap; i += step) sp->counters[i] = 0;
