@@ -273,6 +273,15 @@ int recom_host_pack(int32_t num_features, int32_t batch, const int32_t *const *o
                     const int32_t *const *indices, const int64_t *num_indices, void *dst,
                     int64_t dst_capacity, int64_t *byte_offsets_out);
 
+/* recom_host_parse_lines of every feature followed by recom_host_pack, in one pass and on several
+ * threads: texts[f] / text_lens[f] hold the `batch` sample lines of feature f.  dst needs
+ * byte_offsets_out[F] bytes, which the sum of recom_host_packed_size(batch,
+ * recom_host_max_indices(text_lens[f])) bounds from above; num_indices_out[f] receives the
+ * number of feature f's indices.  An error is that of the first feature that has one. */
+int recom_host_parse_packed(int32_t num_features, int32_t batch, const char *const *texts,
+                            const int64_t *text_lens, void *dst, int64_t dst_capacity,
+                            int64_t *byte_offsets_out, int64_t *num_indices_out);
+
 #ifdef __cplusplus
 }
 #endif

@@ -35,7 +35,7 @@ class BasicBuilder:
         ]
         # e.g. RECFLEX_HIP_EXTRA_FLAGS="-DRFX_PREFETCH_GROUPS=0" for an experiment
         self.hip_flags += os.environ.get("RECFLEX_HIP_EXTRA_FLAGS", "").split()
-        self.host_flags: List[str] = ["-std=c++17", "-shared", "-fPIC", "-Wall"]
+        self.host_flags: List[str] = ["-std=c++17", "-shared", "-fPIC", "-Wall", "-pthread"]
 
     def device_headers(self) -> List[str]:
         """The headers every emitted ``process.hip`` is built from."""
@@ -52,7 +52,7 @@ class BasicBuilder:
         if force or not os.path.exists(lib):
             os.makedirs(os.path.dirname(lib), exist_ok=True)
             tmp = lib + f".tmp{os.getpid()}"
-            cmd = [self.cxx, *self.host_flags, "-O2", f"-I{self.abi_include}", self.host_source, "-o", tmp]
+            cmd = [self.cxx, *self.host_flags, "-O3", f"-I{self.abi_include}", self.host_source, "-o", tmp]
             subprocess.run(cmd, check=True)
             os.replace(tmp, lib)
         return lib

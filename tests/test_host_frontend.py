@@ -116,3 +116,34 @@ def test_preprocess_tuple_shape(host):
     assert scala == [3, 3, 3, 3]                      # (num_inputs, num_segments) per feature
     assert data[0].tolist() == [0, 2, 2, 3] and data[1].tolist() == [1, 2, 3]
     assert data[2].tolist() == [0, 1, 2, 3] and data[3].tolist() == [4, 5, 6]
+
+
+def _feature_lines(rng, batch, mean):
+    return [",".join(str(int(v)) for v in rng.integers(0, 2 ** 31 - 1, rng.poisson(mean))) for _ in range(batch)]
+
+
+@pytest.mark.parametrize("features, batch, mean", [(1, 0, 0.), (1, 1, 3.), (5, 33, 0.3), (3, 31, 12.),
+                                                   (40, 64, 60.), (2, 1500, 40.)])
+def test_joint_parse_equals_feature_by_feature(host, features, batch, mean):
+    """One thread and several (128 KiB of text each), offsets that end on a 128-byte boundary and not,
+    separators of other kinds, empty lines."""
+    rng = np.random.default_rng(features * 1000 + batch)
+    raw = [_feature_lines(rng, batch, mean) for _ in range(features)]
+    if batch > 8:
+        raw[0][:8] = ["", "1,,2", "9,", ",4", ";", "é5", "", "007"]
+    dbo, _, _, _, _, data, scala = host.preprocess(raw)
+    packed = host.packed.copy()
+    want_data, want_scala, want_offsets = host._parse_each(raw)
+    assert np.array_equal(packed, host.packed) and dbo == want_offsets.tolist() and scala == want_scala
+    assert len(data) == len(want_data) and all(
+        a.dtype == np.int32 and np.array_equal(a, b) for a, b in zip(data, want_data))
+
+
+@pytest.mark.parametrize("bad, message", [({2: "2147483648", 4: "1\n2"}, "int32"), ({3: "1\n2\n3", 4: "99999999999"}, "lines")])
+def test_joint_parse_reports_the_first_feature_that_fails(host, bad, message):
+    raw = [["1,2", "3"] for _ in range(6)]
+    for f, text in bad.items():
+        raw[f][0] = text
+    for parse in (host.preprocess, host._parse_each):
+        with pytest.raises(RecomHostError, match=message):
+            parse(raw)
