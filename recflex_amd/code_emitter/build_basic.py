@@ -56,3 +56,19 @@ class BasicBuilder:
             subprocess.run(cmd, check=True)
             os.replace(tmp, lib)
         return lib
+
+    def mlp_lib_path(self, dirname: str = "build") -> str:
+        return os.path.join(self.csrc_dir, dirname, "librecflex_mlp.so")
+
+    def build_mlp(self, dirname: str = "build", force: bool = False) -> str:
+        """Build ``librecflex_mlp.so`` (the kernels of ``RecomModel``'s MLP, model independent) if
+        missing (or ``force``); returns its path."""
+        lib = self.mlp_lib_path(dirname)
+        if force or not os.path.exists(lib):
+            os.makedirs(os.path.dirname(lib), exist_ok=True)
+            tmp = lib + f".tmp{os.getpid()}"
+            cmd = [self.hipcc, *self.hip_flags, "-O3", os.path.join(self.csrc_dir, "mlp", "recflex_mlp.hip"),
+                   "-o", tmp]
+            subprocess.run(cmd, check=True)
+            os.replace(tmp, lib)
+        return lib

@@ -1,0 +1,401 @@
+// The MLP behind the fused embedding (RecomModel): Linear + ReLU layers and a last Linear to one
+// unit with a sigmoid, all in fp32 on the matrix cores.
+//
+// Reference counterpart: the nn.Sequential of RecFlex/rec_modules.py:150-179.
+//
+// A batch of 512 through 4408 -> 1024 -> 256 -> 128 -> 1 is 5 GFLOP, 32 us at the rate a large fp32
+// product reaches here (154 TFLOP/s), and most of it the first layer.  Library products with
+// activations between them are eight launches and, one after the other in a graph, 73 us; batches
+// of 1, 37 and 256 take 50, 49 and 86 us.  Here they are three launches (four where the first
+// layer's K is split) and 67 us; 23, 29 and 49 us for the smaller batches:
+//   gemm_nt    a layer: X [M, K] times W [N, K] transposed, bias and ReLU on the way out;
+//   tail       the last hidden layer, its ReLU, the dot product with the last layer's row and
+//              the sigmoid, and ahead of them the sum of the K-splits of the layer before.
+// Where a layer has too few tiles for the device its K is split over workgroups; the splits' sums
+// go to a buffer and are added in order (tail, or reduce_splits for an earlier layer): the result
+// does not depend on which workgroup ends first.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "recflex_mlp.h"
+
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// x, or 0 where x is not positive; a NaN stays one
+__device__ __forceinline__ float relu(const float x) { return x <= 0.f ? 0.f : x; }
+
+// ---------------------------------------------------------------------------------------------
+// gemm_nt: a workgroup of eight wavefronts computes a tile of 32 or 64 rows x 64 units.  Bound by the
+// matrix cores: 2 048 cycles of them per chunk (32 rows, 128 of K, or 64 rows, 64 of K) for 48 or 32 KB
+// read, of the 128 KB that the L2 delivers to a CU meanwhile.  They are busy 62 to 68 % of the time
+// (batch 512, K 23 980: 105 TFLOP/s; the library's kernel 72 %); tiles of 64 x 64 and 128 x 64 by four
+// or eight wavefronts, chunks of 32 to 128 and one to eight splits all end within 7 % of each other.
+// The tiles are small for the number of them: a batch of 512 and 1 024 units give 256 tiles of 32
+// rows, one per CU.  Such a CU has two wavefronts per SIMD and nothing else to run while they wait,
+// so the wavefronts split the K of a chunk among them, meet once per chunk, and a chunk is asked for
+// two ahead: it goes to LDS while the matrix cores work on the one before.
+// ---------------------------------------------------------------------------------------------
+constexpr int kTileN = 64, kThreads = 512;
+
+// TM x 64 tile: a wavefront sums WM blocks of 32 x 32 over its share of a chunk's K
+template <int TM, int KC, int WM> struct Tile {
+  static constexpr int kM = TM, kChunk = KC;
+  static constexpr int kRow = KC + 4;          // LDS row, in floats: 16-byte reads of 8 rows spread over all banks
+  static constexpr int kRows = TM + kTileN;
+  static constexpr int kVecs = KC / 4;         // 16-byte vectors of a row
+  static constexpr int kRowsPerLoad = kThreads / kVecs;
+  static constexpr int kLoads = kRows / kRowsPerLoad;
+  static constexpr int kKGroups = kThreads / 64 / (TM / 32 / WM * 2);       // wavefronts that share a tile's K
+  static constexpr int kRedRow = kTileN + 4;
+  static_assert(TM % kRowsPerLoad == 0 && kTileN % kRowsPerLoad == 0, "a load instruction stays within X or within W");
+  static_assert(kKGroups * TM * kRedRow <= 2 * kRows * kRow, "the sums fit where the chunks were");
+};
+
+template <int TM, int KC, int WM>
+__global__ void __launch_bounds__(kThreads)
+gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
+        float *__restrict__ out, const int M, const int N, const int K, const int splits) {
+  using T = Tile<TM, KC, WM>;
+  __shared__ float lds[2 * T::kRows * T::kRow];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tiles_n = (N + kTileN - 1) / kTileN;
+  const int tiles = tiles_n * ((M + TM - 1) / TM);
+  const int split = blockIdx.x / tiles, tile = blockIdx.x - split * tiles;
+  // consecutive workgroups (one XCD each) take the units of the same rows: an XCD keeps to an
+  // eighth of the weights, the larger operand
+  const int m0 = tile / tiles_n * TM, n0 = tile % tiles_n * kTileN;
+  const int chunks = (K + KC - 1) / KC;
+  const int per_split = (chunks + splits - 1) / splits;
+  const int first = split * per_split, last = min(chunks, first + per_split);
+
+  // rows beyond M or N repeat the last one (their sums are not stored); K beyond the end reads 0
+  const int col = tid % T::kVecs * 4;
+  const float *src[T::kLoads];
+#pragma unroll
+  for (int i = 0; i < T::kLoads; ++i) {
+    const int row = i * T::kRowsPerLoad + tid / T::kVecs;
+    src[i] = (i * T::kRowsPerLoad < TM
+                  ? x + static_cast<int64_t>(min(m0 + row, M - 1)) * K
+                  : w + static_cast<int64_t>(min(n0 + row - TM, N - 1)) * K) + col;
+  }
+  f32x4 next[T::kLoads];
+  auto request = [&](const int c) {
+    const int k = min(c * KC, K - 4 - col);      // stays within the row
+#pragma unroll
+    for (int i = 0; i < T::kLoads; ++i) next[i] = *reinterpret_cast<const f32x4 *>(src[i] + k);
+  };
+  auto put = [&](float *buf, const int c) {
+    if (c * KC + KC > K) {                       // the last chunk's surplus
+      const bool in = c * KC + col < K;
+#pragma unroll
+      for (int i = 0; i < T::kLoads; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) next[i][j] = in ? next[i][j] : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < T::kLoads; ++i)
+      *reinterpret_cast<f32x4 *>(buf + (i * T::kRowsPerLoad + tid / T::kVecs) * T::kRow + col) = next[i];
+  };
+
+  f32x16 acc[WM];
+#pragma unroll
+  for (int v = 0; v < WM; ++v)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[v][r] = 0.f;
+  const int half_n = wave & 1, part_m = (wave >> 1) % (TM / 32 / WM), kgroup = wave / (TM / 32 / WM * 2);
+  // lane (i, h) of a 32x32x2 product holds row i at two values of k, one per h; which two does not
+  // matter as long as both operands agree, so a lane reads four consecutive ones at once
+  const int frag = (lane & 31) * T::kRow + kgroup * (KC / T::kKGroups) + (lane >> 5) * 4;
+  if (first < last) {
+    request(first);
+    put(lds, first);
+    if (first + 1 < last) request(first + 1);
+  }
+  __syncthreads();
+  for (int c = first; c < last; ++c) {
+    // chunk c + 1, requested a chunk ago, goes to the other buffer (every wavefront is past the
+    // barrier behind its last reads of it) while the matrix cores are busy with chunk c
+    if (c + 1 < last) put(lds + ((c + 1 - first) & 1) * (T::kRows * T::kRow), c + 1);
+    if (c + 2 < last) request(c + 2);
+    const float *buf = lds + ((c - first) & 1) * (T::kRows * T::kRow);
+    const float *xs = buf + part_m * 32 * WM * T::kRow + frag, *ws = buf + (TM + half_n * 32) * T::kRow + frag;
+#pragma unroll
+    for (int s = 0; s < KC / T::kKGroups / 8; ++s) {
+      f32x4 a[WM];
+#pragma unroll
+      for (int v = 0; v < WM; ++v) a[v] = *reinterpret_cast<const f32x4 *>(xs + v * 32 * T::kRow + s * 8);
+      const f32x4 b = *reinterpret_cast<const f32x4 *>(ws + s * 8);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int v = 0; v < WM; ++v)
+          acc[v] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[v][j], b[j], acc[v], 0, 0, 0);
+    }
+    __syncthreads();
+  }
+
+  // the wavefronts' shares of K, added in order
+#pragma unroll
+  for (int v = 0; v < WM; ++v)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int row = (part_m * WM + v) * 32 + 8 * (r / 4) + 4 * (lane >> 5) + r % 4;
+      lds[(kgroup * TM + row) * T::kRedRow + half_n * 32 + (lane & 31)] = acc[v][r];
+    }
+  __syncthreads();
+  for (int at = tid; at < TM * (kTileN / 4); at += kThreads) {
+    const int row = at / (kTileN / 4), unit = at % (kTileN / 4) * 4;
+    f32x4 sum = *reinterpret_cast<const f32x4 *>(lds + row * T::kRedRow + unit);
+#pragma unroll
+    for (int g = 1; g < T::kKGroups; ++g)
+      sum += *reinterpret_cast<const f32x4 *>(lds + (g * TM + row) * T::kRedRow + unit);
+    if (m0 + row >= M || n0 + unit >= N) continue;
+    float *dst = out + (static_cast<int64_t>(split) * M + m0 + row) * N + n0 + unit;
+    if (bias) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sum[j] = relu(sum[j] + bias[min(n0 + unit + j, N - 1)]);
+    }
+    if (N % 4 == 0) {
+      *reinterpret_cast<f32x4 *>(dst) = sum;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (n0 + unit + j < N) dst[j] = sum[j];
+    }
+  }
+}
+
+// out = ReLU(bias + the splits' sums, in order)
+__global__ void __launch_bounds__(256)
+reduce_splits(const float *__restrict__ parts, const float *__restrict__ bias, float *__restrict__ out,
+              const int64_t count, const int N, const int splits) {
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < count;
+       i += static_cast<int64_t>(gridDim.x) * 256) {
+    float v = parts[i];
+    for (int s = 1; s < splits; ++s) v += parts[s * count + i];
+    out[i] = relu(v + bias[i % N]);
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
+// tail: 16 rows a workgroup.  Its input (K <= kTailMaxK) stays in LDS, the last hidden layer's
+// weights (N <= kTailMaxN units) come through LDS in chunks, wavefront w computes the units
+// 16 w .. 16 w + 15, and what leaves is one number per row.  A matter of latencies -- 32 workgroups
+// for a batch of 512 --, worth it because its three steps would be three launches.
+// ---------------------------------------------------------------------------------------------
+constexpr int kTailRows = 16, kTailMaxN = RECFLEX_MLP_TAIL_MAX_UNITS, kTailMaxK = RECFLEX_MLP_TAIL_MAX_INPUTS;
+constexpr int kTailChunk = 128, kTailRow = kTailChunk + 4;
+constexpr int kTailLoads = kTailMaxN * (kTailChunk / 4) / kThreads;
+static_assert(kTailMaxN == kThreads / 64 * 16, "16 units per wavefront");
+
+__global__ void __launch_bounds__(kThreads)
+tail(const float *__restrict__ parts, const int splits, const float *__restrict__ bias0,
+     float *__restrict__ hidden0, const float *__restrict__ w, const float *__restrict__ bias,
+     float *__restrict__ hidden, const float *__restrict__ w_last, const float *__restrict__ b_last,
+     float *__restrict__ out, const int M, const int N, const int K) {
+  __shared__ float xs[kTailRows * (kTailMaxK + 4)];
+  __shared__ float ws[kTailMaxN * kTailRow];
+  __shared__ float dots[kThreads / 64][kTailRows];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m0 = blockIdx.x * kTailRows;
+  const int padded = (K + kTailChunk - 1) / kTailChunk * kTailChunk;   // <= kTailMaxK
+  const int stride = padded + 4;
+
+  f32x4 next[kTailLoads];
+  auto request = [&](const int k0) {
+#pragma unroll
+    for (int i = 0; i < kTailLoads; ++i) {
+      const int at = i * kThreads + tid, row = at / (kTailChunk / 4), k = k0 + at % (kTailChunk / 4) * 4;
+      f32x4 v = {0.f, 0.f, 0.f, 0.f};
+      if (k < K) v = *reinterpret_cast<const f32x4 *>(w + static_cast<int64_t>(min(row, N - 1)) * K + k);
+      next[i] = v;
+    }
+  };
+  request(0);
+
+  // the input: the splits of the layer before, its bias and ReLU
+  const int64_t count = static_cast<int64_t>(M) * K;
+  for (int at = tid; at < kTailRows * (padded / 4); at += kThreads) {
+    const int row = at / (padded / 4), k = (at - row * (padded / 4)) * 4;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (m0 + row < M && k < K) {
+      const int64_t i = static_cast<int64_t>(m0 + row) * K + k;
+      v = *reinterpret_cast<const f32x4 *>(parts + i);
+      for (int s = 1; s < splits; ++s) v += *reinterpret_cast<const f32x4 *>(parts + s * count + i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = relu(v[j] + bias0[k + j]);
+      if (hidden0) *reinterpret_cast<f32x4 *>(hidden0 + i) = v;
+    }
+    *reinterpret_cast<f32x4 *>(xs + row * stride + k) = v;
+  }
+
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < padded; k0 += kTailChunk) {
+#pragma unroll
+    for (int i = 0; i < kTailLoads; ++i) {
+      const int at = i * kThreads + tid;
+      *reinterpret_cast<f32x4 *>(ws + at / (kTailChunk / 4) * kTailRow + at % (kTailChunk / 4) * 4) = next[i];
+    }
+    __syncthreads();
+    if (k0 + kTailChunk < padded) request(k0 + kTailChunk);
+    const float *xf = xs + (lane & 15) * stride + k0 + (lane >> 4) * 4;
+    const float *wf = ws + (wave * 16 + (lane & 15)) * kTailRow + (lane >> 4) * 4;
+#pragma unroll
+    for (int s = 0; s < kTailChunk / 16; ++s) {
+      const f32x4 a = *reinterpret_cast<const f32x4 *>(xf + s * 16);
+      const f32x4 b = *reinterpret_cast<const f32x4 *>(wf + s * 16);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], acc, 0, 0, 0);
+    }
+    __syncthreads();                            // before the next chunk takes this one's place
+  }
+
+  // lane: unit wave * 16 + lane % 16, rows (lane / 16) * 4 + r
+  const int unit = wave * 16 + (lane & 15);
+  const float b = unit < N ? bias[unit] : 0.f, wl = unit < N ? w_last[unit] : 0.f;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = (lane >> 4) * 4 + r;
+    const float h = relu(acc[r] + b);
+    if (hidden && unit < N && m0 + row < M) hidden[static_cast<int64_t>(m0 + row) * N + unit] = h;
+    float d = unit < N ? h * wl : 0.f;
+    d += __shfl_xor(d, 8, 64);
+    d += __shfl_xor(d, 4, 64);
+    d += __shfl_xor(d, 2, 64);
+    d += __shfl_xor(d, 1, 64);
+    if ((lane & 15) == 0) dots[wave][row] = d;
+  }
+  __syncthreads();
+  if (tid < kTailRows && m0 + tid < M) {
+    float z = dots[0][tid];
+#pragma unroll
+    for (int v = 1; v < kThreads / 64; ++v) z += dots[v][tid];
+    out[m0 + tid] = 1.f / (1.f + expf(-(z + b_last[0])));
+  }
+}
+
+int ceil_div(const int64_t a, const int64_t b) { return static_cast<int>((a + b - 1) / b); }
+
+// How a layer is cut: tiles of 32 or 64 rows, and its K into splits.  What a CU takes for a chunk was
+// measured at a batch of 512 and K 23 980: 1.35 us (32 rows), 1.25 us (64 rows, one workgroup on the
+// CU) and 1.18 us (64 rows, two); two more chunks' time for the first loads and the last sums.  Splits
+// cost their traffic and, ahead of any layer but the tail, a kernel that adds them up.
+struct Plan { int rows, splits; };
+Plan plan_of(const int M, const int N, const int K, const int cus, const bool feeds_tail) {
+  Plan best{32, 1};
+  double best_us = 1e30;
+  for (int rows = 32; rows <= 64; rows += 32) {
+    const int64_t tiles = static_cast<int64_t>(ceil_div(M, rows)) * ceil_div(N, kTileN);
+    const int chunks = ceil_div(K, rows == 32 ? 128 : 64);
+    for (int s = 1; s <= RECFLEX_MLP_MAX_SPLITS && s <= chunks; ++s) {
+      const int per_split = ceil_div(chunks, s);
+      if (static_cast<int64_t>(per_split) * (s - 1) >= chunks) continue;            // an empty split
+      const double chunk_us = rows == 32 ? 1.35 : (tiles * s > cus ? 1.18 : 1.25);
+      double us = chunk_us * ceil_div(tiles * s, cus) * (per_split + 2);
+      if (s > 1) us += (feeds_tail ? 0. : 3.) + 2. * s * M * N * 4 / 4e6;
+      if (us < best_us * 0.98) { best = {rows, s}; best_us = us; }
+    }
+  }
+  return best;
+}
+
+struct Device { int id, cus; };
+hipError_t current_device(Device *d) {
+  static int cus[64];                           // written with the same value by whoever is first
+  hipError_t e = hipGetDevice(&d->id);
+  if (e != hipSuccess) return e;
+  if (d->id < 0 || d->id >= 64) return hipErrorInvalidDevice;
+  int n = __atomic_load_n(&cus[d->id], __ATOMIC_RELAXED);
+  if (n <= 0) {
+    e = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, d->id);
+    if (e != hipSuccess) return e;
+    __atomic_store_n(&cus[d->id], n, __ATOMIC_RELAXED);
+  }
+  d->cus = n;
+  return hipSuccess;
+}
+
+bool valid(const recflex_mlp_args *a) {
+  if (!a || a->batch < 0 || a->layers < 2 || a->layers > RECFLEX_MLP_MAX_LAYERS || !a->x) return false;
+  for (int l = 0; l <= a->layers; ++l) {
+    if (a->units[l] <= 0 || !a->weights[l] || !a->biases[l]) return false;
+    if (l < a->layers && (a->units[l] % 4 || reinterpret_cast<uintptr_t>(a->weights[l]) % 16)) return false;
+  }
+  return reinterpret_cast<uintptr_t>(a->x) % 16 == 0 &&
+         a->units[a->layers] <= kTailMaxN && a->units[a->layers - 1] <= kTailMaxK;
+}
+
+} // namespace
+
+extern "C" int recflex_mlp_workspace_floats(const recflex_mlp_args *a, int64_t *floats) {
+  if (!valid(a) || !floats) return static_cast<int>(hipErrorInvalidValue);
+  Device d;
+  const hipError_t e = current_device(&d);
+  if (e != hipSuccess) return static_cast<int>(e);
+  int64_t most = 0;
+  for (int l = 0; l + 1 < a->layers; ++l) {
+    const int s = plan_of(a->batch, a->units[l + 1], a->units[l], d.cus, l + 2 == a->layers).splits;
+    const int64_t need = static_cast<int64_t>(s) * a->batch * a->units[l + 1];
+    if ((s > 1 || l + 2 == a->layers) && need > most) most = need;
+  }
+  *floats = most;
+  return 0;
+}
+
+extern "C" int recflex_mlp_forward(const recflex_mlp_args *a) {
+  if (!valid(a) || !a->out || !a->workspace || reinterpret_cast<uintptr_t>(a->workspace) % 16)
+    return static_cast<int>(hipErrorInvalidValue);
+  for (int l = 0; l + 2 < a->layers; ++l)       // the tail's input needs no buffer of its own
+    if (!a->hidden[l] || reinterpret_cast<uintptr_t>(a->hidden[l]) % 16) return static_cast<int>(hipErrorInvalidValue);
+  if (reinterpret_cast<uintptr_t>(a->hidden[a->layers - 2]) % 16) return static_cast<int>(hipErrorInvalidValue);
+  if (a->batch == 0) return 0;
+  Device d;
+  hipError_t e = current_device(&d);
+  if (e != hipSuccess) return static_cast<int>(e);
+  hipStream_t stream = static_cast<hipStream_t>(a->stream);
+  auto launch = [&](const void *kernel, int64_t blocks, int threads, void **args) {
+    if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
+    return hipLaunchKernel(kernel, dim3(static_cast<unsigned>(blocks)), dim3(threads), args, 0, stream);
+  };
+  int M = a->batch;
+  const float *x = a->x;
+  int splits = 1;
+  for (int l = 0; l + 1 < a->layers; ++l) {
+    int K = a->units[l], N = a->units[l + 1];
+    const bool feeds_tail = l + 2 == a->layers;
+    const Plan plan = plan_of(M, N, K, d.cus, feeds_tail);
+    splits = plan.splits;
+    const bool direct = splits == 1 && !feeds_tail;
+    const float *w = a->weights[l], *bias = direct ? a->biases[l] : nullptr;
+    float *out = direct ? a->hidden[l] : a->workspace;
+    void *args[] = {&x, &w, &bias, &out, &M, &N, &K, &splits};
+    const int64_t tiles = static_cast<int64_t>(ceil_div(M, plan.rows)) * ceil_div(N, kTileN);
+    const void *kernel = plan.rows == 32 ? reinterpret_cast<const void *>(&gemm_nt<32, 128, 1>)
+                                         : reinterpret_cast<const void *>(&gemm_nt<64, 64, 2>);
+    e = launch(kernel, tiles * splits, kThreads, args);
+    if (e != hipSuccess) return static_cast<int>(e);
+    if (!direct && !feeds_tail) {
+      int64_t count = static_cast<int64_t>(M) * N;
+      const float *parts = a->workspace;
+      bias = a->biases[l];
+      out = a->hidden[l];
+      void *rargs[] = {&parts, &bias, &out, &count, &N, &splits};
+      const int64_t blocks = (count + 255) / 256;
+      e = launch(reinterpret_cast<const void *>(reduce_splits), blocks > 4096 ? 4096 : blocks, 256, rargs);
+      if (e != hipSuccess) return static_cast<int>(e);
+    }
+    x = feeds_tail ? a->workspace : a->hidden[l];
+  }
+  const int t = a->layers - 1;                  // the last hidden layer
+  int K = a->units[t], N = a->units[t + 1];
+  const float *bias0 = a->biases[t - 1], *w = a->weights[t], *bias = a->biases[t];
+  const float *w_last = a->weights[t + 1], *b_last = a->biases[t + 1];
+  float *hidden0 = a->hidden[t - 1], *hidden = a->hidden[t], *out = a->out;
+  void *args[] = {&x, &splits, &bias0, &hidden0, &w, &bias, &hidden, &w_last, &b_last, &out, &M, &N, &K};
+  return static_cast<int>(launch(reinterpret_cast<const void *>(tail), ceil_div(M, kTailRows), kThreads, args));
+}

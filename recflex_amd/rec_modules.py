@@ -26,6 +26,7 @@ import numpy as np
 import torch
 import torch.nn as nn
 
+from . import mlp as mlp_kernels
 from .librecom import RecomLib
 from .quant import random_int8_table
 
@@ -372,6 +373,7 @@ class RecomModel(nn.Module):
             layers.append(nn.Linear(unit_nums[i], unit_nums[i + 1], bias=True, device=self.embed_layer.device))
             layers.append(nn.Sigmoid() if i + 2 == len(unit_nums) else nn.ReLU())
         self.mlp = nn.Sequential(*layers)
+        mlp_kernels.load_library()
 
     def forward(self, arg_buffers: torch.Tensor, data_buffer_offsets: torch.Tensor,
                 scala_args: torch.Tensor, extra_buffers: torch.Tensor, extra_buffer_offsets: torch.Tensor,
@@ -381,4 +383,5 @@ class RecomModel(nn.Module):
             arg_buffers, data_buffer_offsets, scala_args, extra_buffers, extra_buffer_offsets,
             task_mapping, task_tiles, task_barriers, embed_output_size)
         embed_output = torch.reshape(embed_output, [-1, self.embed_layer.output_units])
-        return self.mlp(embed_output)
+        out = mlp_kernels.forward(self.mlp, embed_output)
+        return self.mlp(embed_output) if out is None else out

@@ -1,0 +1,133 @@
+"""The kernels of ``RecomModel``'s MLP against the same layers in 64 bits, and the module they stand
+in for wherever they step aside."""
+
+import pytest
+import torch
+import torch.nn as nn
+
+from recflex_amd import mlp as kernels
+
+pytestmark = pytest.mark.gpu
+
+# fp32 sums in blocks of at most 128 terms, blocks and splits added in order: errors of a few eps per
+# layer in the 2-norm
+REL = 1e-6
+
+
+def build(units, device="cuda", seed=0):
+    torch.manual_seed(seed)
+    sizes = list(units) + [1]
+    mods = []
+    for i, (a, b) in enumerate(zip(sizes, sizes[1:])):
+        mods += [nn.Linear(a, b), nn.Sigmoid() if i + 2 == len(sizes) else nn.ReLU()]
+    return nn.Sequential(*mods).to(device)
+
+
+def rel(got, want):
+    return float((got.double().cpu() - want.double().cpu()).norm() / want.double().cpu().norm())
+
+
+# edges of the tiles (32 and 64 rows, 64 units), of a chunk of K (128), of the tail (16 rows, 128 units,
+# 1 024 inputs), odd unit counts where they are allowed, many layers, many splits of K
+@pytest.mark.parametrize("units, batch", [
+    ((4, 4, 1), 1), ((20, 36, 100, 8), 17), ((128, 64, 128), 16), ((132, 68, 127), 33),
+    ((64, 1024, 3), 31), ((512, 1020, 128), 65), ((4408, 1024, 256, 128), 37),
+    ((4408, 1024, 256, 128), 512), ((12, 8, 8, 8, 8, 8, 8, 8, 8), 5), ((23980, 64, 128), 3),
+    ((1000, 200, 64, 16), 449),
+])
+def test_mlp_forward_and_gradients(units, batch):
+    print("[case] mlp", units, batch, flush=True)
+    mlp = build(units)
+    exact = build(units).double()
+    exact.load_state_dict({k: v.double() for k, v in mlp.state_dict().items()})
+    x = torch.randn(batch, units[0], device="cuda", requires_grad=True)
+    xd = x.detach().double().requires_grad_()
+    want = exact(xd)
+    with torch.no_grad():
+        got = kernels.forward(mlp, x.detach())
+    assert got is not None and got.shape == (batch, 1) and not got.requires_grad
+    assert rel(got, want.detach()) < REL
+    out = kernels.forward(mlp, x)
+    assert torch.equal(out.detach(), got)
+    weight = torch.linspace(0.5, 1.5, batch, device="cuda")[:, None]
+    (out * weight).sum().backward()
+    # against the modules: the gradients of the kernels' path are stock products on the kernels' activations.
+    # A unit within rounding of zero may be on for one and off for the other: fp32 rounding of a few
+    # hundred terms puts one unit in a million there, and one such unit of n is sqrt(1 / n) of a norm.
+    stock = build(units)
+    stock.load_state_dict(mlp.state_dict())
+    xs = x.detach().clone().requires_grad_()
+    (stock(xs) * weight).sum().backward()
+    assert rel(x.grad, xs.grad) < 0.02
+    for a, b in zip(mlp.parameters(), stock.parameters()):
+        assert a.grad.shape == b.grad.shape and rel(a.grad, b.grad) < 0.02
+
+
+def test_mlp_repeats_bits_and_passes_nan_on():
+    mlp = build((256, 96, 32))
+    x = torch.randn(70, 256, device="cuda")
+    with torch.no_grad():
+        first = kernels.forward(mlp, x)
+        assert all(torch.equal(kernels.forward(mlp, x), first) for _ in range(3))
+        x[5, 7], x[6, 9] = float("nan"), float("inf")
+        got, want = kernels.forward(mlp, x), mlp(x)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and bool(torch.isnan(got[5]))
+    assert torch.equal(got[7:], first[7:])
+
+
+def test_mlp_second_derivatives():
+    """Through the hidden layers' outputs too: the gradient's gradient equals the modules'."""
+    units = (16, 12, 8, 4)
+    mlp, stock = build(units), build(units)
+    x = torch.randn(9, 16, device="cuda")
+    got = []
+    for net, run in ((mlp, lambda v: kernels.forward(mlp, v)), (stock, stock)):
+        v = x.clone().requires_grad_()
+        (g,) = torch.autograd.grad(run(v).sum(), v, create_graph=True)
+        got.append(torch.autograd.grad((g * g).sum(), [v] + [p for p in net.parameters() if p.dim() == 2]))
+    for a, b in zip(*got):
+        assert torch.allclose(a, b, rtol=1e-3, atol=1e-7)
+
+
+def test_mlp_graph_replays():
+    mlp = build((200, 64, 32))
+    x = torch.randn(50, 200, device="cuda")
+    side = torch.cuda.Stream()
+    with torch.no_grad():
+        kernels.forward(mlp, x)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            out = kernels.forward(mlp, x)
+        for seed in range(3):
+            torch.manual_seed(seed)
+            x.copy_(torch.randn(50, 200, device="cuda"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, kernels.forward(mlp, x))
+
+
+def test_mlp_steps_aside():
+    """Whatever wants to see the layers gets them."""
+    mlp = build((64, 32, 16))
+    x = torch.randn(8, 64, device="cuda")
+    assert kernels.forward(mlp, x) is not None
+    handle = mlp[2].register_forward_hook(lambda *a: None)
+    assert kernels.forward(mlp, x) is None
+    handle.remove()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert kernels.forward(mlp, x) is None
+    seen = []
+    torch.func.vmap(lambda row: seen.append(kernels.forward(mlp, row[None])) or row)(x)
+    assert seen == [None]
+    with torch.autograd.forward_ad.dual_level():
+        assert kernels.forward(mlp, x) is None
+    for other in (build((64, 32, 16)).double(), build((62, 32, 16)), build((64, 16)), build((64, 32, 132)),
+                  build((64, 1028, 16)), build((64, 32, 16), device="cpu")):
+        v = torch.randn(8, other[0].in_features, device=other[0].weight.device, dtype=other[0].weight.dtype)
+        assert kernels.forward(other, v) is None
+    assert kernels.forward(mlp, x.t().contiguous().t()) is None
+    assert kernels.forward(mlp, torch.randn(kernels.MAX_BATCH + 1, 64, device="cuda")) is None
+    assert kernels.forward(mlp, x[:0]) is None
+    mlp[0].bias = None
+    assert kernels.forward(mlp, x) is None
