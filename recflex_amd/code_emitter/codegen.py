@@ -736,7 +736,9 @@ static int launch_kernels(const recom_process_args *a, void *workspace) {
   if (e != hipSuccess) return static_cast<int>(e);
   const int grid = a->grid_blocks > 0 ? a->grid_blocks : st->cus * st->occupancy;
   if (grid <= 0) return static_cast<int>(hipErrorInvalidConfiguration);
-  const int tile_bytes = a->tile_bytes > 0 ? a->tile_bytes : TILE_BYTES;
+  // the caller's tile size as it is; the library's own is for full batches (rfx::capped_tile_size)
+  const int tile_bytes = a->tile_bytes > 0 ? a->tile_bytes
+                                           : (TILE_BYTES > rfx::kAutoTileMin ? -TILE_BYTES : TILE_BYTES);
   const int xcd_segments = a->xcd_segments > 0 ? a->xcd_segments
                                                : (a->xcd_segments < 0 ? 0 : XCD_SEGMENTS);
 

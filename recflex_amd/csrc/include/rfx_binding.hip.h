@@ -170,6 +170,22 @@ __host__ __device__ inline int auto_tile_size(const long long total, const int g
   return static_cast<int>(t) & ~1023;
 }
 
+// The tile size of a library that was built with one beyond kAutoTileMin (tile_bytes = -size): it was
+// chosen on full batches, and a batch of less than kCappedTilesPerWorkgroup such tiles per workgroup
+// gets smaller ones, so that its end is not a matter of whole tiles, down to kAutoTileMin.  (Below that
+// tiles come apart into less than a workgroup's pass and teams idle: 400 fp16 features, 16 samples, 43
+// us with 64 KiB, 61 with 32.  A size of 64 KiB or less stays: cut in half it gave 100 and 1 000
+// features 3 % at some batches and cost 3 % at others.)  Measured, in us, with the size as built and
+// this one: 200 int8 features (128 KiB) 64 / 300 / 1 000 samples 24.5 / 66.6 / 138 and 20.8 / 55.4 /
+// 133; 400 fp16 features (256 KiB) 4 / 16 / 64 samples 39.3 / 51.0 / 105 and 36.5 / 47.6 / 100.
+constexpr int kCappedTilesPerWorkgroup = 5;
+
+__host__ __device__ inline int capped_tile_size(const int built, const long long total, const int grid_blocks) {
+  const long long t = total / ((grid_blocks > 0 ? grid_blocks : 1) * static_cast<long long>(kCappedTilesPerWorkgroup));
+  if (t >= built || kAutoTileMin >= built) return built;
+  return t > kAutoTileMin ? static_cast<int>(t) & ~1023 : kAutoTileMin;
+}
+
 // Inclusive prefix sum over the 64 lanes of a wavefront with DPP moves (no LDS traffic): shifts
 // by 1, 2, 4 and 8 inside each row of 16 lanes (lanes shifted in from outside the row read 0),
 // then lane 15 of a row broadcast to the next row (rows 1 and 3), then lane 31 to rows 2 and 3.
@@ -204,8 +220,8 @@ __device__ __forceinline__ float wave_sum(float v) {
 // production build, the whole candidate list in a tuning build); choice[f] (clamped; 0 if
 // choice is null) selects the one this launch runs, and cand_gran[] gives the bags a workgroup
 // of that schedule handles per pass (tiles are whole multiples of it unless a pass is too large).
-// tile_bytes: traffic a tile should carry; <= 0 lets the workgroup size the tiles from the batch
-// (see kAutoTilesPerWorkgroup above).
+// tile_bytes: traffic a tile should carry; 0 lets the workgroup size the tiles from the batch
+// (see kAutoTilesPerWorkgroup above), -size does so up to that size (see capped_tile_size).
 // fixed_tiles: if non-null, the tile count per feature is taken from it instead of from the
 // live offsets (static thread binding, for the ablation).
 // grid_blocks: workgroups of the fused kernel's grid (for the automatic tile size).
@@ -344,8 +360,9 @@ bind_tiles(BindingStorage<F> &s, const IoView &io, const int tile_bytes,
   // Step 2 (only where the tile size or the split unit depend on it): the batch's traffic, in
   // single precision -- it sizes tiles in steps of kilobytes.
   const bool automatic = tile_bytes <= 0 && !fixed_tiles;
-  const bool need_total = automatic || (SPLIT && !fixed_tiles);
-  int tile_size = tile_bytes;
+  // (one sample: a tile per feature whatever its size)
+  const bool need_total = (automatic && B > 1) || (SPLIT && !fixed_tiles);
+  int tile_size = automatic ? kAutoTileMin : tile_bytes;
   long long split_unit = 0;
   if (need_total) {
     float total = wave_sum(traffic);
@@ -359,7 +376,8 @@ bind_tiles(BindingStorage<F> &s, const IoView &io, const int tile_bytes,
     // the same in every lane: what follows from it is scalar arithmetic
     total = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(total)));
     const long long total_bytes = static_cast<long long>(total);
-    if (automatic) tile_size = auto_tile_size(total_bytes, grid_blocks);
+    if (automatic) tile_size = tile_bytes < 0 ? capped_tile_size(-tile_bytes, total_bytes, grid_blocks)
+                                              : auto_tile_size(total_bytes, grid_blocks);
     if (SPLIT) {
       const long long grid = grid_blocks > 0 ? grid_blocks : 1;
       split_unit = total_bytes / (4ll * grid);

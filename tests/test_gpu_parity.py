@@ -679,3 +679,29 @@ def test_kernel_events_take_the_dispatch_time_and_change_nothing(name):
     print(f"   dispatch {min(inside):.2f} us, event records around it {min(around):.2f} us", flush=True)
     assert all(0.0 < t < 1e5 for t in inside)
     assert min(inside) <= min(around) * 1.05
+
+
+@pytest.mark.parametrize("batch", [1, 3, 64, 300, 1100])
+def test_smaller_tiles_of_small_batches_change_no_bit(batch):
+    """A library built with tiles of 128 KiB cuts a small batch into smaller ones, down to 64 KiB (its
+    own choice); the tiles as built, smaller ones and the library's choice give the same bits."""
+    import torch
+    from recflex_amd import prebuilt
+    from recflex_amd.rec_modules import FeatEmbed
+    from recflex_amd.workloads import gen_inputs, gen_tables
+    wl = prebuilt.model_spec("c5_tuned").workload
+    wl = wl._replace(batch=batch, table_values="integer",
+                     features=tuple(f._replace(rows=min(f.rows, 3000)) for f in wl.features))
+    print("[case] c5_tuned, batch", batch, flush=True)
+    dev = torch.device("cuda", 0)
+    tables = gen_tables(wl, dev)
+    indices, offsets = gen_inputs(wl)
+    layer = FeatEmbed(dev, embed_tables=tables, librecom=require_lib("c5_tuned"))
+    assert layer.lib.info.tile_bytes > 64 * 1024
+    bound = layer.bind_inputs([torch.from_numpy(i).to(dev) for i in indices],
+                              [torch.from_numpy(o).to(dev) for o in offsets])
+    got = layer.forward_indices(bound)
+    want = oracle_output(wl, [t.cpu().numpy() for t in tables], indices, offsets)
+    assert np.array_equal(got.cpu().numpy(), want)
+    for tile_bytes in (layer.lib.info.tile_bytes, 32768):
+        assert torch.equal(layer.forward_indices(bound, tile_bytes=tile_bytes), got)
