@@ -106,6 +106,13 @@ constexpr int kSplitMinUnit = 256 * 1024;
 // 256 KiB are 1.4 tiles per workgroup, i.e. two rounds with the second a third full, 94 us;
 // 3 872 parts of 199 KiB are 1.9, 88 us).
 constexpr int kSplitFloorUnit = 128 * 1024;
+// Models of up to kSplitSearchFeats features count the tiles that a part size would give, and take the
+// size whose tiles fill a whole number of rounds of the grid (rfx::search_split_unit).  (16 x 20 000
+// lookups, 2 048 workgroups, in us: 3 712 parts of 200 KiB 85, 2 176 of 340 KiB 104, 1 984 of 384 KiB
+// 74, 1 696 of 440 KiB 80; 128 x 2 500: 2 304 tiles 99, 2 048 of them 77.)  Counting takes a few
+// instructions per feature in every workgroup, hence the limit.
+constexpr int kSplitSearchFeats = 16;
+constexpr int kSplitPartCost = 35 * 1024;      // a part's round trips, in traffic
 constexpr int kSplitGran = -1;
 constexpr int kBindMaxParts = 64;
 constexpr int kBindMaxSplitTiles = 2048;
@@ -214,6 +221,21 @@ __device__ __forceinline__ float wave_sum(float v) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
+// Least v over the wavefront, the same value in every lane (a lane without a source keeps its own).
+template <int CTRL, int ROW_MASK> __device__ __forceinline__ float min_dpp(const float v) {
+  const int i = __float_as_int(v);
+  return fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(i, i, CTRL, ROW_MASK, 0xf, false)));
+}
+__device__ __forceinline__ float wave_min(float v) {
+  v = min_dpp<0x111, 0xf>(v);
+  v = min_dpp<0x112, 0xf>(v);
+  v = min_dpp<0x114, 0xf>(v);
+  v = min_dpp<0x118, 0xf>(v);
+  v = min_dpp<0x142, 0xa>(v);
+  v = min_dpp<0x143, 0xc>(v);
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
 // lookup_bytes[f]: bytes fetched per lookup (row + index); bag_bytes[f]: bytes per bag that do
 // not depend on its length (output row slice + offset).
 // Feature f owns the candidate schedules cand_begin[f] .. cand_begin[f+1]-1 (exactly one in a
@@ -251,6 +273,52 @@ __device__ __forceinline__ int div_small(const int a, const int b) {
 }
 // batches up to which div_small serves (its dividends stay below twice the batch)
 constexpr int kSmallDivBatch = 1 << 21;
+
+// Parts a bag of bag_cost bytes (the feature's mean) is cut into at part size 1 / inv_unit; 1: left
+// whole.  A bag is split from 1.25 units on (128 x 2 500 lookups: 102.8 us with bags of 1.7 units left
+// whole beside split ones, 89.3 us with those in two parts).  most: split_parts_most of the batch.
+__device__ __forceinline__ float parts_of_bag(const float bag_cost, const float inv_unit, const float most) {
+  const float units = bag_cost * inv_unit;
+  return units > 1.25f ? fmaxf(fminf(ceilf(units), most), 1.f) : 1.f;
+}
+// the most parts a bag may have in a batch of this size
+__device__ __forceinline__ float split_parts_most(const int batch) {
+  const int slots = kBindMaxSplitTiles / (batch > 0 ? batch : 1);
+  return static_cast<float>(slots < kBindMaxParts ? slots : kBindMaxParts);
+}
+
+// The part size of a model of few features, by its first wavefront (lane f < F: feature f's traffic
+// and schedule): every lane takes one candidate, a workgroup's share of the batch in 1 to 4 rounds,
+// enlarged by 0 to 15 sixteenths, and counts its tiles; of those that fit their rounds the one with
+// the least rounds * (part + kSplitPartCost) wins.  0: none fits.  The same value in every lane.
+template <int F>
+__device__ __forceinline__ int
+search_split_unit(const float cost, const int gran, const int B, const int tile_size, const float total,
+                  const float grid) {
+  const int lane = threadIdx.x & 63;
+  const float rounds = static_cast<float>(1 + (lane >> 4));
+  const float unit = total * __builtin_amdgcn_rcpf(rounds * grid) * (1.f + 0.0625f * static_cast<float>(lane & 15));
+  const float inv_unit = __builtin_amdgcn_rcpf(unit), most = split_parts_most(B);
+  const float batch = static_cast<float>(B);
+  const float bag = gran == kSplitGran && B > 0 ? cost * __builtin_amdgcn_rcpf(batch) : 0.f;
+  // what the features that don't split come to, in tiles of the regular size
+  const float whole = gran == kSplitGran ? 0.f : fmaxf(1.f, ceilf(cost * __builtin_amdgcn_rcpf(static_cast<float>(tile_size))));
+  float tiles = 0.f, part = 0.f;                // ... and the longest part
+#pragma unroll
+  for (int f = 0; f < F; ++f) {
+    const float bag_f = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bag), f));
+    const float whole_f = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(whole), f));
+    const float parts = parts_of_bag(bag_f, inv_unit, most);
+    tiles += whole_f > 0.f ? whole_f : batch * parts;
+    part = fmaxf(part, bag_f * __builtin_amdgcn_rcpf(parts));
+  }
+  const bool fits = tiles <= rounds * grid && unit >= static_cast<float>(kSplitFloorUnit) &&
+                    unit >= static_cast<float>(tile_size);
+  const float price = fits ? rounds * (part + static_cast<float>(kSplitPartCost)) : 3.4e38f;
+  const float least = wave_min(price);
+  const unsigned long long best = __builtin_amdgcn_ballot_w64(fits && price == least);
+  return best ? __builtin_amdgcn_readlane(static_cast<int>(unit), __builtin_ctzll(best)) : 0;
+}
 
 template <int F, int BT, bool SPLIT = false, bool ONE_CAND = false>
 __device__ __forceinline__ int
@@ -391,6 +459,13 @@ bind_tiles(BindingStorage<F> &s, const IoView &io, const int tile_bytes,
         if (split_unit > kSplitMinUnit) split_unit = kSplitMinUnit;
         if (split_unit < kSplitFloorUnit) split_unit = kSplitFloorUnit;
         if (split_unit < tile_size) split_unit = tile_size;
+        if constexpr (F <= kSplitSearchFeats) {
+          // one round of parts of kSplitMinUnit or less is what the rule above gives by itself
+          if (tid < 64 && total_bytes > grid * kSplitMinUnit) {
+            const int searched = search_split_unit<F>(cost[0], gran[0], B, tile_size, total, static_cast<float>(grid));
+            if (searched > 0) split_unit = searched;
+          }
+        }
       }
     }
   }
@@ -425,12 +500,8 @@ bind_tiles(BindingStorage<F> &s, const IoView &io, const int tile_bytes,
     }
     int bpt = 0;
     int parts = 1;
-    // a bag is split from 1.25 units on (128 x 2 500 lookups: 102.8 us with bags of 1.7 units left
-    // whole beside split ones, 89.3 us with those in two parts)
-    if (SPLIT && may_split && B > 0 && split_unit > 0 && 4.f * bag_cost > 5.f * split_unit_f) {
-      parts = static_cast<int>(fminf(ceilf(bag_cost / split_unit_f), static_cast<float>(kBindMaxParts)));
-      if (static_cast<long long>(parts) * B > kBindMaxSplitTiles) parts = kBindMaxSplitTiles / B;
-    }
+    if (SPLIT && may_split && split_unit > 0)
+      parts = static_cast<int>(parts_of_bag(bag_cost, __builtin_amdgcn_rcpf(split_unit_f), split_parts_most(B)));
     if (parts > 1) {
       tiles = B * parts;
       bpt = -parts;

@@ -705,3 +705,31 @@ def test_smaller_tiles_of_small_batches_change_no_bit(batch):
     assert np.array_equal(got.cpu().numpy(), want)
     for tile_bytes in (layer.lib.info.tile_bytes, 32768):
         assert torch.equal(layer.forward_indices(bound, tile_bytes=tile_bytes), got)
+
+
+@pytest.mark.parametrize("bags, mean, grid", [(16, 4000, 64), (150, 300, 40), (3, 9000, 7), (48, 900, 0),
+                                              (1, 30000, 3), (2049, 40, 12), (33, 2000, 16)])
+def test_part_sizes_that_fill_rounds_of_the_grid(bags, mean, grid):
+    """Models of up to 16 features choose the part size whose tiles fill whole rounds of the grid,
+    where a workgroup's share of the batch is beyond 256 KiB: small grids bring small batches there.
+    Bags of unequal length, empty ones among them; integer-valued tables, so any split gives the same
+    bits; two launches, since the arrival counters must be back at zero."""
+    import torch
+    from recflex_amd import prebuilt
+    from recflex_amd.rec_modules import FeatEmbed
+    from recflex_amd.workloads import gen_inputs, gen_tables
+    wl = prebuilt.model_spec("fewbags").workload
+    wl = wl._replace(batch=bags, table_values="integer", features=tuple(
+        f._replace(rows=5000, mean_bag=float(mean), len_sigma=0.7 if k % 2 else 0.0, empty_frac=0.1)
+        for k, f in enumerate(wl.features)))
+    print("[case] fewbags", bags, mean, grid, flush=True)
+    dev = torch.device("cuda", 0)
+    tables = gen_tables(wl, dev)
+    indices, offsets = gen_inputs(wl)
+    layer = FeatEmbed(dev, embed_tables=tables, librecom=require_lib("fewbags"))
+    bound = layer.bind_inputs([torch.from_numpy(i).to(dev) for i in indices],
+                              [torch.from_numpy(o).to(dev) for o in offsets])
+    want = oracle_output(wl, [t.cpu().numpy() for t in tables], indices, offsets)
+    for _ in range(2):
+        got = layer.forward_indices(bound, grid_blocks=grid).cpu().numpy()
+        assert np.array_equal(got, want)
