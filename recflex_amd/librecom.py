@@ -8,6 +8,7 @@ any number of emitted kernels can be used in one process.
 
 import ctypes
 import os
+import struct
 from typing import List
 
 _I32P = ctypes.POINTER(ctypes.c_int32)
@@ -64,6 +65,11 @@ class RecomProcessArgs(ctypes.Structure):
         ("d_lookup_counts", ctypes.c_void_p),
     ]
 
+# the same, packed by one call (a ctypes structure converts field by field, a third of a small
+# call's time on the host)
+_PROCESS_ARGS = struct.Struct("@5Q4i3Qq1Qq3Q")
+assert _PROCESS_ARGS.size == ctypes.sizeof(RecomProcessArgs)
+
 
 RECOM_ABI_VERSION = 6
 RECOM_STATIC_WORKSPACE_MAX_BYTES = 32 * 1024 * 1024
@@ -98,6 +104,9 @@ class RecomLib:
         self.lib.recom_get_max_concurrent_blocks.argtypes = [_I32P]
         self.lib.recom_process.restype = ctypes.c_int
         self.lib.recom_process.argtypes = [ctypes.POINTER(RecomProcessArgs)]
+        self._process_packed = self.lib["recom_process"]      # a function object of its own
+        self._process_packed.restype = ctypes.c_int
+        self._process_packed.argtypes = [ctypes.c_char_p]
         self.lib.recom_process_static_workspace.restype = ctypes.c_int
         self.lib.recom_process_static_workspace.argtypes = [ctypes.POINTER(RecomProcessArgs)]
 
@@ -202,12 +211,17 @@ class RecomLib:
             return
         if not workspace and self.workspace_bytes:
             workspace, workspace_bytes = self.default_workspace(), self.workspace_bytes
-        args = RecomProcessArgs(table_ptrs or None, io_ptrs or None, arg_buffers or None,
-                                arg_buffer_offsets or None, output or None, batch, tile_bytes,
-                                grid_blocks, xcd_segments, schedule_choice or None, times or None,
-                                stream or None, output_row_stride, workspace or None,
-                                workspace_bytes, start_event or None, stop_event or None,
-                                lookup_counts or None)
-        rc = self.lib.recom_process(ctypes.byref(args))
+        try:
+            packed = _PROCESS_ARGS.pack(
+                table_ptrs, io_ptrs, arg_buffers, arg_buffer_offsets, output, batch, tile_bytes, grid_blocks,
+                xcd_segments, schedule_choice, times, stream, output_row_stride, workspace, workspace_bytes,
+                start_event, stop_event, lookup_counts)
+        except struct.error:                    # None for 0, numbers beyond their field: as ctypes takes them
+            packed = bytes(RecomProcessArgs(
+                table_ptrs or None, io_ptrs or None, arg_buffers or None, arg_buffer_offsets or None,
+                output or None, batch, tile_bytes, grid_blocks, xcd_segments, schedule_choice or None,
+                times or None, stream or None, output_row_stride, workspace or None, workspace_bytes,
+                start_event or None, stop_event or None, lookup_counts or None))
+        rc = self._process_packed(packed)
         if rc != 0:
             raise RecomError("recom_process", rc)

@@ -174,7 +174,7 @@ class FeatEmbed(nn.Module):
                 raise TypeError(f"out must be an fp32 device tensor of "
                                 f"{batch * self.output_units} elements")
             if out.is_contiguous():
-                output = out.view(-1)
+                output = out                    # (the callers shape the result)
             elif out.dim() == 2 and out.shape == (batch, self.output_units) and out.stride(1) == 1:
                 # a column slab of a wider buffer: the library writes rows out.stride(0) apart
                 output, row_stride = out, out.stride(0)
@@ -195,7 +195,8 @@ class FeatEmbed(nn.Module):
                     or schedule_choice.device.type != "cuda":
                 raise TypeError("schedule_choice must be an int32 device tensor with one entry per feature")
             inputs["schedule_choice"] = schedule_choice.data_ptr()
-        stream = torch.cuda.current_stream(self.device).cuda_stream
+        index = self.device.index
+        stream = torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
         if kernel_events is not None:
             inputs.update(start_event=kernel_events[0].handle, stop_event=kernel_events[1].handle)
         if self.workspace is not None:
