@@ -32,6 +32,7 @@ from .quant import random_int8_table
 
 _current_lib: Optional[RecomLib] = None
 
+_ADDRESS = torch.Tensor.data_ptr        # mapped over lists: half the time of a call per element
 _TORCH_DTYPES = {0: torch.float32, 1: torch.float16, 2: torch.uint8}
 
 
@@ -247,7 +248,7 @@ class FeatEmbed(nn.Module):
         batch = offsets[0].numel() - 1
         for f in range(n):
             for name, t in (("indices", indices[f]), ("offsets", offsets[f])):
-                if t.dtype != torch.int32 or not t.is_contiguous() or t.device.type != "cuda":
+                if t.dtype != torch.int32 or not t.is_contiguous() or not t.is_cuda:
                     raise TypeError(f"{name}[{f}] must be a contiguous int32 device tensor")
             if offsets[f].numel() != batch + 1:
                 raise ValueError("all features must share one batch size")
@@ -301,8 +302,7 @@ class FeatEmbed(nn.Module):
             n = len(self.embed_tables)
             if offsets is None or len(indices) != n or len(offsets) != n:
                 raise ValueError(f"expected {n} index and offset tensors")
-            key = tuple(t.data_ptr() for t in indices) + tuple(t.data_ptr() for t in offsets) \
-                + (offsets[0].numel(),)
+            key = (*map(_ADDRESS, indices), *map(_ADDRESS, offsets), offsets[0].numel())
             if key != self._io_cache_key:
                 # new input tensors: validate them and upload their addresses
                 self._io_bound = self.bind_inputs(indices, offsets)
