@@ -22,8 +22,8 @@ TAIL_MAX_UNITS = 128                # RECFLEX_MLP_TAIL_MAX_UNITS
 TAIL_MAX_INPUTS = 1024              # RECFLEX_MLP_TAIL_MAX_INPUTS
 # Beyond this many rows the layers are library products: the first layer alone keeps the device busy,
 # and the library's kernel for large products reaches 140 TFLOP/s where these reach 105.  MLP of
-# 1024, 256 and 128 units on 4 408 / 23 980 inputs, kernels against library, in us: 256 rows 49 / 153
-# against 86 / 383, 512 rows 67 / 250 against 73 / 250, 700 rows 100 / 398 against 90 / 682, 1 024
+# 1024, 256 and 128 units on 4 408 / 23 980 inputs, kernels against library, in us: 256 rows 44 / 140
+# against 86 / 383, 512 rows 65 / 238 against 74 / 250, 700 rows 100 / 398 against 90 / 682, 1 024
 # rows 105 / 517 against 106 / 380.
 MAX_BATCH = 512
 
