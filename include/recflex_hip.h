@@ -146,7 +146,8 @@ typedef struct recom_process_args {
   float *d_output;
   int32_t batch;
   /* memory traffic per tile for the run-time binding; 0 = the emitted default
-   * (recom_info.tile_bytes; if that is 0 too, the device sizes the tiles from the batch:
+   * (recom_info.tile_bytes, or less, down to 64 KiB, for a batch of fewer than five such tiles per
+   * workgroup; if that is 0 too, the device sizes the tiles from the batch:
    * total traffic / (64 tiles per workgroup of the grid), within 64..256 KiB) */
   int32_t tile_bytes;
   /* persistent grid size; 0 = recom_get_max_concurrent_blocks() */
