@@ -69,6 +69,7 @@ class RecomProcessArgs(ctypes.Structure):
 # call's time on the host)
 _PROCESS_ARGS = struct.Struct("@5Q4i3Qq1Qq3Q")
 assert _PROCESS_ARGS.size == ctypes.sizeof(RecomProcessArgs)
+_ADDRESS_TYPES = {int}
 
 
 RECOM_ABI_VERSION = 6
@@ -211,12 +212,20 @@ class RecomLib:
             return
         if not workspace and self.workspace_bytes:
             workspace, workspace_bytes = self.default_workspace(), self.workspace_bytes
-        try:
-            packed = _PROCESS_ARGS.pack(
-                table_ptrs, io_ptrs, arg_buffers, arg_buffer_offsets, output, batch, tile_bytes, grid_blocks,
-                xcd_segments, schedule_choice, times, stream, output_row_stride, workspace, workspace_bytes,
-                start_event, stop_event, lookup_counts)
-        except struct.error:                    # None for 0, numbers beyond their field: as ctypes takes them
+        packed = None
+        # (struct takes anything with an __index__, a one-element tensor in place of its address
+        # among them; ctypes wants an address to be an int)
+        if {type(table_ptrs), type(io_ptrs), type(arg_buffers), type(arg_buffer_offsets), type(output),
+                type(schedule_choice), type(times), type(stream), type(workspace), type(start_event),
+                type(stop_event), type(lookup_counts)} == _ADDRESS_TYPES:
+            try:
+                packed = _PROCESS_ARGS.pack(
+                    table_ptrs, io_ptrs, arg_buffers, arg_buffer_offsets, output, batch, tile_bytes, grid_blocks,
+                    xcd_segments, schedule_choice, times, stream, output_row_stride, workspace, workspace_bytes,
+                    start_event, stop_event, lookup_counts)
+            except struct.error:                # numbers beyond their field: as ctypes takes them
+                pass
+        if packed is None:
             packed = bytes(RecomProcessArgs(
                 table_ptrs or None, io_ptrs or None, arg_buffers or None, arg_buffer_offsets or None,
                 output or None, batch, tile_bytes, grid_blocks, xcd_segments, schedule_choice or None,

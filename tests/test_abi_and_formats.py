@@ -52,6 +52,31 @@ def test_host_library_exports_every_host_symbol():
             assert hasattr(lib, name), name
 
 
+def test_process_takes_addresses_that_are_ints_only():
+    """A tensor or a numpy number in the place of an address is refused before anything runs (a
+    one-element tensor would pass for the address it holds); numbers and ``None`` are packed as
+    the ctypes structure packs them."""
+    import torch
+    lib = RecomLib(prebuilt.ensure_built("c1"))
+    packed = []
+    lib._process_packed = lambda args: packed.append(args) or 0
+    for bad in (torch.tensor([1 << 20]), np.int64(1 << 20), 1.0):
+        for name in ("io_ptrs", "arg_buffers", "arg_buffer_offsets", "schedule_choice", "times", "stream",
+                     "workspace", "start_event", "stop_event", "lookup_counts"):
+            with pytest.raises(TypeError):
+                lib.process(1 << 20, 1 << 21, 4, **{name: bad})
+        with pytest.raises(TypeError):
+            lib.process(bad, 1 << 21, 4)
+        with pytest.raises(TypeError):
+            lib.process(1 << 20, bad, 4)
+    assert not packed
+    lib.process(1 << 20, 1 << 40, 4, io_ptrs=1 << 21, tile_bytes=-1, output_row_stride=7, stream=None)
+    lib.process(1 << 20, 1 << 40, np.int32(4), io_ptrs=1 << 21, tile_bytes=-1, output_row_stride=7)
+    want = bytes(RecomProcessArgs(d_embed_table_ptrs=1 << 20, d_io_ptrs=1 << 21, d_output=1 << 40, batch=4,
+                                  tile_bytes=-1, output_row_stride=7))
+    assert packed == [want, want]
+
+
 def test_ctypes_structs_match_header_layout():
     # recom_info: 11 named int32 + 5 reserved; recom_process_args: 5 pointers, 4 int32,
     # 3 pointers, an int64, a pointer and an int64 on LP64
