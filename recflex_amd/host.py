@@ -121,12 +121,13 @@ class RecomHost:
 
     # -------------------------------------------------------------------------------------
 
-    def _parse_packed(self, raw_data: List[List[str]]) -> Tuple[List[np.ndarray], List[int], np.ndarray]:
-        """Sets ``self.packed``; returns ``data``, ``scala_data`` and the packed buffer's byte
-        offsets.  One native call for all features (``recom_host_parse_packed``: several threads,
-        each feature parsed straight into its place); a thousand features of 64 lines, 7.7 MB of
-        text, take 5 ms on eight cores that way and 33 ms with a parse, three allocations and two
-        copies per feature."""
+    def _parse_packed(self, raw_data: List[List[str]], with_data: bool
+                      ) -> Tuple[List[np.ndarray], List[int], np.ndarray]:
+        """Sets ``self.packed``; returns ``data`` (empty unless asked for), ``scala_data`` and the
+        packed buffer's byte offsets.  One native call for all features
+        (``recom_host_parse_packed``: several threads, each feature parsed straight into its
+        place); a thousand features of 64 lines, 7.7 MB of text, take 5 ms on eight cores that way
+        and 33 ms with a parse, three allocations and two copies per feature."""
         num_feats = len(raw_data)
         batches = {len(lines) for lines in raw_data}
         if len(batches) != 1 or not hasattr(self.lib, "recom_host_parse_packed"):
@@ -146,13 +147,16 @@ class RecomHost:
                                               counts.ctypes.data_as(_I64P))
         if rc != 0:
             raise RecomHostError(f"recom_host_parse_lines: {_ERRORS.get(rc, rc)}")
-        self.packed = dst[:int(byte_offsets[-1]) // 4]
+        dst.resize(int(byte_offsets[-1]) // 4, refcheck=False)      # gives the rest of the room back
+        self.packed = dst
+        scala_data = np.stack([counts, np.full(num_feats, batch)], 1).ravel().tolist()  # num_inputs, num_segments
         data: List[np.ndarray] = []
-        scala_data: List[int] = []
-        for at, n in zip((byte_offsets[:-1] // 4).tolist(), counts.tolist()):
-            first = at + off_bytes // 4
-            data += [dst[at:at + batch + 1], dst[first:first + n]]
-            scala_data += [n, batch]                      # num_inputs, num_segments
+        if with_data:
+            # arrays of their own: a caller may change them without changing what goes to the GPU,
+            # and one that is kept keeps nothing else alive
+            for at, n in zip((byte_offsets[:-1] // 4).tolist(), counts.tolist()):
+                first = at + off_bytes // 4
+                data += [dst[at:at + batch + 1].copy(), dst[first:first + n].copy()]
         return data, scala_data, byte_offsets
 
     def _parse_each(self, raw_data: List[List[str]]) -> Tuple[List[np.ndarray], List[int], np.ndarray]:
@@ -171,11 +175,15 @@ class RecomHost:
         return data, scala_data, byte_offsets
 
     def preprocess(self, raw_data: List[List[str]], max_concurrent_blocks: int = 0):
+        return self._preprocess(raw_data, True)
+
+    def _preprocess(self, raw_data: List[List[str]], with_data: bool):
+        """``preprocess``, without the arrays of ``data`` where nobody looks at them."""
         num_feats = len(raw_data)
         if self.num_features is not None and num_feats != self.num_features:
             raise ValueError(f"this host library was generated for {self.num_features} features, "
                              f"got {num_feats}")
-        data, scala_data, byte_offsets = self._parse_packed(raw_data)
+        data, scala_data, byte_offsets = self._parse_packed(raw_data, with_data)
         data_buffer_offsets = byte_offsets.tolist()
         # byte offsets of each feature's slab of pooled output (prefix sum of batch * dim * 4,
         # reference: codegen.py:144-147); the generic library does not know the dims and

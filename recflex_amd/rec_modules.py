@@ -27,6 +27,7 @@ import torch
 import torch.nn as nn
 
 from . import mlp as mlp_kernels
+from .host import RecomHost
 from .librecom import RecomLib
 from .quant import random_int8_table
 
@@ -63,8 +64,11 @@ class FeatPreprocess(nn.Module):
         self.output_units = output_units
 
     def forward(self, raw_data: List[List[str]], max_concurrent_blocks: int = 0):
-        (data_buffer_offsets, output_offsets, extra_buffer_offsets, task_mapping, task_tiles,
-         data, scala_data) = self.recom_host.preprocess(raw_data, max_concurrent_blocks)
+        # (a RecomHost as it is hands the packed buffer over: the arrays of data are not needed)
+        host = self.recom_host
+        whole = type(host) is not RecomHost or "preprocess" in vars(host)
+        (data_buffer_offsets, output_offsets, extra_buffer_offsets, task_mapping, task_tiles, data,
+         scala_data) = host.preprocess(raw_data, max_concurrent_blocks) if whole else host._preprocess(raw_data, False)
 
         output_size: int = output_offsets[-1]
         if output_size == 0 and self.output_units and len(raw_data) > 0:

@@ -139,6 +139,49 @@ def test_joint_parse_equals_feature_by_feature(host, features, batch, mean):
         a.dtype == np.int32 and np.array_equal(a, b) for a, b in zip(data, want_data))
 
 
+@pytest.mark.parametrize("features, batch", [(3, 31), (1, 1), (12, 64)])
+def test_preprocess_data_are_arrays_of_their_own(host, features, batch):
+    """Changing ``data`` changes neither the packed buffer nor one another, and none of them, nor
+    the packed buffer, holds on to more memory than its own."""
+    rng = np.random.default_rng(5)
+    raw = [_feature_lines(rng, batch, 9.) for _ in range(features)]
+    data = host.preprocess(raw)[5]
+    packed, before = host.packed, host.packed.copy()
+    assert packed.base is None and packed.flags.owndata
+    for k, a in enumerate(data):
+        assert a.base is None and a.flags.owndata and a.flags.writeable
+        a[:] = -1 - k
+    assert np.array_equal(packed, before)
+    assert all((a == -1 - k).all() for k, a in enumerate(data))
+
+
+def test_feat_preprocess_takes_any_host(host):
+    """The host as it is, a subclass and an instance with a ``preprocess`` of their own: the same
+    tensors, and the caller's ``preprocess`` runs."""
+    import torch
+    from recflex_amd.host import RecomHost
+    from recflex_amd.rec_modules import FeatPreprocess
+
+    class Own(RecomHost):
+        def preprocess(self, raw_data, max_concurrent_blocks=0):
+            calls.append(max_concurrent_blocks)
+            return super().preprocess(raw_data, max_concurrent_blocks)
+
+    calls = []
+    rng = np.random.default_rng(6)
+    raw = [_feature_lines(rng, 21, 7.) for _ in range(4)]
+    own, patched = Own(), RecomHost()
+    patched.preprocess = own.preprocess
+    patched.packed = None
+    want = FeatPreprocess(RecomHost(), torch.device("cpu"), output_units=8)(raw, 5)
+    got = FeatPreprocess(own, torch.device("cpu"), output_units=8)(raw, 5)
+    data = FeatPreprocess(patched, torch.device("cpu"), output_units=8)(raw, 6)[0]
+    assert calls == [5, 6] and len(want) == len(got) == 9 and want[-1] == got[-1] == 21 * 8 * 4
+    assert all(torch.equal(a, b) for a, b in zip(want[:-1], got[:-1]))
+    # no packed buffer: the arrays of data, one after the other
+    assert data.tolist() == np.concatenate(own.preprocess(raw)[5]).tolist()
+
+
 @pytest.mark.parametrize("bad, message", [({2: "2147483648", 4: "1\n2"}, "int32"), ({3: "1\n2\n3", 4: "99999999999"}, "lines")])
 def test_joint_parse_reports_the_first_feature_that_fails(host, bad, message):
     raw = [["1,2", "3"] for _ in range(6)]
