@@ -4,13 +4,15 @@ eight of the same ``nn.Sequential`` run layer by layer.
 
 ``forward(mlp, x)`` returns ``None`` where the kernels don't apply, and the caller then runs the
 modules: other layers than ``RecomModel`` builds, hooks on any of them, parameters that are not
-plain fp32 tensors on the current device, sizes outside the kernels' range, and whatever wants to
+plain fp32 tensors on the current device, sizes outside the kernels' range, no library and no
+compiler to build it, and whatever wants to
 see the single operations (autocast, tracing, compiling, vmap and the other function transforms,
 forward-mode derivatives, dispatch and function modes).
 """
 
 import ctypes
-import os
+import subprocess
+import warnings
 from typing import List, Optional
 
 import torch
@@ -38,6 +40,7 @@ class _Args(ctypes.Structure):
 
 
 _lib = None
+_missing = False                    # it could not be loaded, nor built: the modules run
 
 
 def load_library() -> ctypes.CDLL:
@@ -52,6 +55,19 @@ def load_library() -> ctypes.CDLL:
         lib.recflex_mlp_workspace_floats.argtypes = [ctypes.POINTER(_Args), ctypes.POINTER(ctypes.c_int64)]
         _lib = lib
     return _lib
+
+
+def try_load_library() -> bool:
+    """Load the library, with a warning where that fails: the modules serve without it."""
+    global _missing
+    try:
+        load_library()
+        _missing = False
+    except (OSError, subprocess.SubprocessError) as e:      # no file and no compiler, nowhere to write, ...
+        _missing = True
+        warnings.warn(f"the MLP kernels could not be loaded or built, RecomModel runs its layers one by one: {e}",
+                      RuntimeWarning, stacklevel=3)
+    return not _missing
 
 
 def _hooked(m: nn.Module) -> bool:
@@ -168,6 +184,8 @@ def forward(mlp: nn.Module, x: torch.Tensor) -> Optional[torch.Tensor]:
             return None
         params += [w, b]
         fan_in = w.shape[0]
+    if _lib is None and (_missing or not try_load_library()):
+        return None
     if linears[-1].weight.shape[1] > TAIL_MAX_UNITS or linears[-2].weight.shape[1] > TAIL_MAX_INPUTS:
         return None
     if torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in params)):

@@ -378,7 +378,7 @@ class RecomModel(nn.Module):
             layers.append(nn.Linear(unit_nums[i], unit_nums[i + 1], bias=True, device=self.embed_layer.device))
             layers.append(nn.Sigmoid() if i + 2 == len(unit_nums) else nn.ReLU())
         self.mlp = nn.Sequential(*layers)
-        mlp_kernels.load_library()
+        mlp_kernels.try_load_library()
 
     def forward(self, arg_buffers: torch.Tensor, data_buffer_offsets: torch.Tensor,
                 scala_args: torch.Tensor, extra_buffers: torch.Tensor, extra_buffer_offsets: torch.Tensor,
