@@ -7,6 +7,7 @@ CMakeLists).  Here the device side is header-only (``csrc/include/*.hip.h``), so
 text front end is a prebuilt library.
 """
 
+import hashlib
 import os
 import shutil
 import subprocess
@@ -61,14 +62,28 @@ class BasicBuilder:
         return os.path.join(self.csrc_dir, dirname, "librecflex_mlp.so")
 
     def build_mlp(self, dirname: str = "build", force: bool = False) -> str:
-        """Build ``librecflex_mlp.so`` (the kernels of ``RecomModel``'s MLP, model independent) if
-        missing (or ``force``); returns its path."""
+        """Build ``librecflex_mlp.so`` (the kernels of ``RecomModel``'s MLP, model independent) if it is
+        missing or was built from another source or with other flags (or ``force``); returns its path."""
         lib = self.mlp_lib_path(dirname)
-        if force or not os.path.exists(lib):
+        sources = [os.path.join(self.csrc_dir, "mlp", n) for n in ("recflex_mlp.hip", "recflex_mlp.h")]
+        if not force and os.path.exists(lib) and not all(map(os.path.exists, sources)):
+            return lib                              # a package without its sources
+        flags = [*self.hip_flags, "-O3"]
+        key = hashlib.sha256(" ".join(flags).encode())
+        for path in sources:
+            with open(path, "rb") as f:
+                key.update(f.read())
+        built_from = lib + ".from"                  # what the library beside it was built from
+        current = ""
+        if os.path.exists(lib) and os.path.exists(built_from):
+            with open(built_from) as f:
+                current = f.read()
+        if force or current != key.hexdigest():
             os.makedirs(os.path.dirname(lib), exist_ok=True)
             tmp = lib + f".tmp{os.getpid()}"
-            cmd = [self.hipcc, *self.hip_flags, "-O3", os.path.join(self.csrc_dir, "mlp", "recflex_mlp.hip"),
-                   "-o", tmp]
-            subprocess.run(cmd, check=True)
+            subprocess.run([self.hipcc, *flags, sources[0], "-o", tmp], check=True)
             os.replace(tmp, lib)
+            with open(tmp, "w") as f:
+                f.write(key.hexdigest())
+            os.replace(tmp, built_from)
         return lib

@@ -1,5 +1,7 @@
 """What ``RecomModel`` does around its MLP kernels, as far as that needs no GPU."""
 
+import shutil
+
 import pytest
 import torch
 import torch.nn as nn
@@ -42,3 +44,29 @@ def test_model_without_the_mlp_library_runs_its_modules(no_library):
     assert torch.equal(model(x, *[None] * 8), model.mlp(x))
     # asked for without a model: once, not on every call
     assert kernels._missing and kernels._lib is None
+
+
+def test_mlp_library_follows_its_source(monkeypatch, tmp_path):
+    """Built when it is missing, kept as long as source and flags are what it was built from."""
+    builder = BasicBuilder()
+    (tmp_path / "mlp").mkdir()
+    for name in ("recflex_mlp.hip", "recflex_mlp.h"):
+        shutil.copy(f"{builder.csrc_dir}/mlp/{name}", tmp_path / "mlp" / name)
+    builder.csrc_dir = str(tmp_path)
+    builds = []
+
+    def compile_(cmd, check):
+        builds.append(cmd)
+        with open(cmd[-1], "w") as f:
+            f.write("library %d" % len(builds))
+
+    monkeypatch.setattr("subprocess.run", compile_)
+    for source, flags, want in (("", [], 1), ("", [], 1), ("\n// edited\n", [], 2), ("", [], 2), ("", ["-DX"], 3)):
+        with open(tmp_path / "mlp" / "recflex_mlp.hip", "a") as f:
+            f.write(source)
+        builder.hip_flags = builder.hip_flags + [x for x in flags if x not in builder.hip_flags]
+        with open(builder.build_mlp()) as f:
+            assert f.read() == "library %d" % want
+    assert builder.build_mlp(force=True) and len(builds) == 4
+    (tmp_path / "mlp" / "recflex_mlp.h").unlink()       # a package without its sources keeps its library
+    assert builder.build_mlp() and len(builds) == 4
