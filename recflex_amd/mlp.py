@@ -17,7 +17,17 @@ from typing import List, Optional
 
 import torch
 import torch.nn as nn
-from torch.nn.modules.module import _has_any_global_hook
+
+# What wants to see the single operations, as far as torch has no public name for it.  In a torch
+# without one of these the modules run.
+try:
+    from torch.nn.modules.module import _has_any_global_hook
+    _transforms = torch._C._functorch.peek_interpreter_stack
+    _dispatch_modes = torch._C._len_torch_dispatch_stack
+    _function_modes = torch._C._len_torch_function_stack
+    _KNOWS_OBSERVERS = isinstance(torch.autograd.forward_ad._current_level, int)
+except (ImportError, AttributeError):
+    _KNOWS_OBSERVERS = False
 
 MAX_LAYERS = 8                      # RECFLEX_MLP_MAX_LAYERS
 TAIL_MAX_UNITS = 128                # RECFLEX_MLP_TAIL_MAX_UNITS
@@ -97,9 +107,8 @@ def _plain(t, shape, x) -> bool:
 def _observed() -> bool:
     """Something wants to see every operation."""
     return torch.is_autocast_enabled("cuda") or torch.jit.is_tracing() or torch.compiler.is_compiling() \
-        or torch._C._functorch.peek_interpreter_stack() is not None \
-        or torch.autograd.forward_ad._current_level >= 0 \
-        or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0
+        or _transforms() is not None or torch.autograd.forward_ad._current_level >= 0 \
+        or _dispatch_modes() > 0 or _function_modes() > 0
 
 
 def _run(x: torch.Tensor, weights, biases, keep_hidden: bool):
@@ -166,6 +175,8 @@ class _Mlp(torch.autograd.Function):
 
 
 def forward(mlp: nn.Module, x: torch.Tensor) -> Optional[torch.Tensor]:
+    if not _KNOWS_OBSERVERS:
+        return None
     linears = _linears(mlp)
     if linears is None or _observed():
         return None

@@ -34,6 +34,8 @@ from .quant import random_int8_table
 _current_lib: Optional[RecomLib] = None
 
 _ADDRESS = torch.Tensor.data_ptr        # mapped over lists: half the time of a call per element
+# the current stream's handle without the torch.cuda.Stream around it, in a torch that has a name for it
+_RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 _TORCH_DTYPES = {0: torch.float32, 1: torch.float16, 2: torch.uint8}
 
 
@@ -54,6 +56,12 @@ def _resolve_lib(librecom: Union[None, str, RecomLib]) -> RecomLib:
         raise RuntimeError("no fused-kernel library loaded: pass librecom=... or call "
                            "recflex_amd.rec_modules.load_library(path) first")
     return _current_lib
+
+
+def _stream_of(device: torch.device) -> int:
+    if _RAW_STREAM is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _RAW_STREAM(torch.cuda.current_device() if device.index is None else device.index)
 
 
 class FeatPreprocess(nn.Module):
@@ -200,8 +208,7 @@ class FeatEmbed(nn.Module):
                     or schedule_choice.device.type != "cuda":
                 raise TypeError("schedule_choice must be an int32 device tensor with one entry per feature")
             inputs["schedule_choice"] = schedule_choice.data_ptr()
-        index = self.device.index
-        stream = torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+        stream = _stream_of(self.device)
         if kernel_events is not None:
             inputs.update(start_event=kernel_events[0].handle, stop_event=kernel_events[1].handle)
         if self.workspace is not None:

@@ -1,11 +1,14 @@
 """What ``RecomModel`` does around its MLP kernels, as far as that needs no GPU."""
 
 import shutil
+import subprocess
+import sys
 
 import pytest
 import torch
 import torch.nn as nn
 
+from helpers import ROOT
 from recflex_amd import mlp as kernels
 from recflex_amd import rec_modules
 from recflex_amd.code_emitter.build_basic import BasicBuilder
@@ -70,3 +73,24 @@ def test_mlp_library_follows_its_source(monkeypatch, tmp_path):
     assert builder.build_mlp(force=True) and len(builds) == 4
     (tmp_path / "mlp" / "recflex_mlp.h").unlink()       # a package without its sources keeps its library
     assert builder.build_mlp() and len(builds) == 4
+
+
+@pytest.mark.parametrize("name", ["torch._C._cuda_getCurrentRawStream", "torch._C._functorch.peek_interpreter_stack",
+                                  "torch._C._len_torch_dispatch_stack", "torch._C._len_torch_function_stack",
+                                  "torch.autograd.forward_ad._current_level",
+                                  "torch.nn.modules.module._has_any_global_hook"])
+def test_a_torch_without_a_private_name(name):
+    """The public call, or the modules, take its place."""
+    script = f'''
+import torch, types
+import torch.utils._python_dispatch, torch.overrides
+del {name}
+from recflex_amd import mlp, rec_modules
+torch.cuda.current_stream = lambda device: types.SimpleNamespace(cuda_stream=77)
+if "RawStream" in "{name}":
+    assert mlp._KNOWS_OBSERVERS and rec_modules._stream_of(torch.device("cuda", 0)) == 77
+else:
+    assert rec_modules._RAW_STREAM is not None
+    assert mlp.forward(None, None) is None
+'''
+    subprocess.run([sys.executable, "-c", script], check=True, cwd=ROOT, timeout=120)
