@@ -16,6 +16,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "rfx_tile_sizes.h"
+
 namespace rfx {
 
 // A device address read from memory, as a pointer the compiler knows to be global memory (so
@@ -81,42 +83,6 @@ struct IoView {
   __device__ __forceinline__ const int *indices(int f) const { return global_ptr<int>(indices_addr(f)); }
 };
 
-// Schedules that split a bag over several workgroups (rfx::split_bags) announce themselves with
-// a granularity of kSplitGran.  A bag is worth splitting when it alone would keep its workgroup
-// busy for a good part of the kernel: the unit is a quarter of a workgroup's fair share of the
-// batch's traffic (total / grid), at least one tile and kSplitMinUnit; when the mean bag of such a feature
-// carries more than 1.25 units, the feature gets batch * parts tiles, parts = bag / unit, tile t
-// being part t % parts of bag t / parts, and bags_per_tile holds -parts.  (A part costs some
-// 6 us of dependent memory round trips besides its rows, and with two to five tiles per
-// workgroup the time moves in steps of whole tiles: a unit of half a share gave 150 / 162 /
-// 161 us where a quarter gives 177 / 109 / 160 us on 16 x 20 000, 64 x 4 000 and 128 x 2 500
-// lookups; the finer one is kept, it also evens out bags of unequal length.)
-// Always parts <= kBindMaxParts and batch * parts <= kBindMaxSplitTiles (the slots of the feature's
-// workspace region).  Otherwise -- many bags, or a small grid -- the feature is bound like any
-// other with one bag per workgroup pass.  (Measured on 8 features of 16 bags of 20 000 lookups:
-// 968 us unsplit, 177 us split; 64 bags of 4 000: 204 and 109 us; 512 bags of 1 000 stay
-// unsplit at 185 us.)
-// Smallest part: 256 KiB of traffic (with 128 KiB parts the three shapes above take 175 / 108 /
-// 161 us at four workgroups per CU, with 256 KiB parts 142 / 103 / 122 us; at eight workgroups
-// per CU, which these light kernels allow, 138 / 76 / 83 us and 107 / 83 / 96 us).
-constexpr int kSplitMinUnit = 256 * 1024;
-// ... unless the batch is so small that parts of that size leave the workgroups with one or two
-// tiles each: then the part size is chosen so that the tiles come out as a whole number per
-// workgroup, down to kSplitFloorUnit (16 x 20 000 lookups on 2 048 workgroups: 2 880 parts of
-// 256 KiB are 1.4 tiles per workgroup, i.e. two rounds with the second a third full, 94 us;
-// 3 872 parts of 199 KiB are 1.9, 88 us).
-constexpr int kSplitFloorUnit = 128 * 1024;
-// Models of up to kSplitSearchFeats features count the tiles that a part size would give, and take the
-// size whose tiles fill a whole number of rounds of the grid (rfx::search_split_unit).  (16 x 20 000
-// lookups, 2 048 workgroups, in us: 3 712 parts of 200 KiB 85, 2 176 of 340 KiB 104, 1 984 of 384 KiB
-// 74, 1 696 of 440 KiB 80; 128 x 2 500: 2 304 tiles 99, 2 048 of them 77.)  Counting takes a few
-// instructions per feature in every workgroup, hence the limit.
-constexpr int kSplitSearchFeats = 16;
-constexpr int kSplitPartCost = 35 * 1024;      // a part's round trips, in traffic
-constexpr int kSplitGran = -1;
-constexpr int kBindMaxParts = 64;
-constexpr int kBindMaxSplitTiles = 2048;
-
 // a tile is rounded up to one whole workgroup pass of its schedule only if that pass carries at
 // most this many times the target traffic per tile
 constexpr int kMaxTileFactor = 8;
@@ -150,47 +116,6 @@ __device__ __forceinline__ int64_t uniform64(const int64_t v) {
   const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<int>(v));
   const unsigned hi = __builtin_amdgcn_readfirstlane(static_cast<int>(v >> 32));
   return static_cast<int64_t>((static_cast<unsigned long long>(hi) << 32) | lo);
-}
-
-// Automatic tile size (tile_bytes <= 0): the batch's traffic divided by kAutoTilesPerWorkgroup
-// tiles for each workgroup of the grid, within [kAutoTileMin, kAutoTileMax], in steps of 4 KiB.
-// Small batches keep 64 KiB tiles; a batch of tens of GB with bags of hundreds of wide rows gets
-// 256 KiB, several bags per tile instead of one (measured on the 400-feature fp16 model with its
-// default schedules: 7.1 ms with 64 KiB tiles, 5.0 ms with 256 KiB).
-// A batch too small for that (less than kAutoTileMin of traffic per workgroup of the grid) gets
-// about two tiles per workgroup instead, down to kAutoTileFloor: its launch is a matter of
-// latencies -- every pass of a workgroup over a tile is a chain of dependent round trips to
-// memory -- so the passes are spread over all workgroups as evenly as their number allows
-// (measured on 26 features x 4 096 one-lookup bags, 1 024 workgroups: 9.0 us with 54 KiB tiles
-// of two passes each, 8.3 us with 32 KiB tiles of one).
-constexpr int kAutoTilesPerWorkgroup = 64;
-constexpr int kAutoTileMin = 64 * 1024;
-constexpr int kAutoTileMax = 256 * 1024;
-constexpr int kAutoTileFloor = 4 * 1024;
-
-__host__ __device__ inline int auto_tile_size(const long long total, const int grid_blocks) {
-  const long long grid = grid_blocks > 0 ? grid_blocks : 1;
-  long long t = total / (grid * kAutoTilesPerWorkgroup);
-  if (t >= kAutoTileMin) return static_cast<int>(t > kAutoTileMax ? kAutoTileMax : t) & ~4095;
-  t = total / (2 * grid);
-  t = t < kAutoTileFloor ? kAutoTileFloor : (t > kAutoTileMin ? kAutoTileMin : t);
-  return static_cast<int>(t) & ~1023;
-}
-
-// The tile size of a library that was built with one beyond kAutoTileMin (tile_bytes = -size): it was
-// chosen on full batches, and a batch of less than kCappedTilesPerWorkgroup such tiles per workgroup
-// gets smaller ones, so that its end is not a matter of whole tiles, down to kAutoTileMin.  (Below that
-// tiles come apart into less than a workgroup's pass and teams idle: 400 fp16 features, 16 samples, 43
-// us with 64 KiB, 61 with 32.  A size of 64 KiB or less stays: cut in half it gave 100 and 1 000
-// features 3 % at some batches and cost 3 % at others.)  Measured, in us, with the size as built and
-// this one: 200 int8 features (128 KiB) 64 / 300 / 1 000 samples 24.5 / 66.6 / 138 and 20.8 / 55.4 /
-// 133; 400 fp16 features (256 KiB) 4 / 16 / 64 samples 39.3 / 51.0 / 105 and 36.5 / 47.6 / 100.
-constexpr int kCappedTilesPerWorkgroup = 5;
-
-__host__ __device__ inline int capped_tile_size(const int built, const long long total, const int grid_blocks) {
-  const long long t = total / ((grid_blocks > 0 ? grid_blocks : 1) * static_cast<long long>(kCappedTilesPerWorkgroup));
-  if (t >= built || kAutoTileMin >= built) return built;
-  return t > kAutoTileMin ? static_cast<int>(t) & ~1023 : kAutoTileMin;
 }
 
 // Inclusive prefix sum over the 64 lanes of a wavefront with DPP moves (no LDS traffic): shifts
@@ -274,50 +199,31 @@ __device__ __forceinline__ int div_small(const int a, const int b) {
 // batches up to which div_small serves (its dividends stay below twice the batch)
 constexpr int kSmallDivBatch = 1 << 21;
 
-// Parts a bag of bag_cost bytes (the feature's mean) is cut into at part size 1 / inv_unit; 1: left
-// whole.  A bag is split from 1.25 units on (128 x 2 500 lookups: 102.8 us with bags of 1.7 units left
-// whole beside split ones, 89.3 us with those in two parts).  most: split_parts_most of the batch.
-__device__ __forceinline__ float parts_of_bag(const float bag_cost, const float inv_unit, const float most) {
-  const float units = bag_cost * inv_unit;
-  return units > 1.25f ? fmaxf(fminf(ceilf(units), most), 1.f) : 1.f;
-}
-// the most parts a bag may have in a batch of this size
-__device__ __forceinline__ float split_parts_most(const int batch) {
-  const int slots = kBindMaxSplitTiles / (batch > 0 ? batch : 1);
-  return static_cast<float>(slots < kBindMaxParts ? slots : kBindMaxParts);
-}
+struct DeviceRcp {
+  static __device__ __forceinline__ float rcp(const float x) { return __builtin_amdgcn_rcpf(x); }
+};
 
-// The part size of a model of few features, by its first wavefront (lane f < F: feature f's traffic
-// and schedule): every lane takes one candidate, a workgroup's share of the batch in 1 to 4 rounds,
-// enlarged by 0 to 15 sixteenths, and counts its tiles; of those that fit their rounds the one with
-// the least rounds * (part + kSplitPartCost) wins.  0: none fits.  The same value in every lane.
+// The part size of a model of few features, by its first wavefront.  Lane f < F holds, of feature f:
+// the mean traffic of a bag (0 if its schedule does not split), and the tiles it has as long as its
+// bags are left whole.  Every lane takes one candidate and counts its tiles; of those that fit their
+// rounds the one with the least rounds * (part + kSplitPartCost) wins.  0: none fits.  The same value
+// in every lane.
 template <int F>
 __device__ __forceinline__ int
-search_split_unit(const float cost, const int gran, const int B, const int tile_size, const float total,
-                  const float grid) {
+search_split_unit(const float bag, const int whole_tiles, const int B, const int tile_size, const float total,
+                  const int grid) {
   const int lane = threadIdx.x & 63;
-  const float rounds = static_cast<float>(1 + (lane >> 4));
-  const float unit = total * __builtin_amdgcn_rcpf(rounds * grid) * (1.f + 0.0625f * static_cast<float>(lane & 15));
-  const float inv_unit = __builtin_amdgcn_rcpf(unit), most = split_parts_most(B);
-  const float batch = static_cast<float>(B);
-  const float bag = gran == kSplitGran && B > 0 ? cost * __builtin_amdgcn_rcpf(batch) : 0.f;
-  // what the features that don't split come to, in tiles of the regular size
-  const float whole = gran == kSplitGran ? 0.f : fmaxf(1.f, ceilf(cost * __builtin_amdgcn_rcpf(static_cast<float>(tile_size))));
-  float tiles = 0.f, part = 0.f;                // ... and the longest part
+  const int unit = split_unit_candidate<DeviceRcp>(lane, total, grid);
+  const float inv_unit = DeviceRcp::rcp(static_cast<float>(unit)), most = split_parts_most(B);
+  SplitTally tally;
 #pragma unroll
-  for (int f = 0; f < F; ++f) {
-    const float bag_f = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bag), f));
-    const float whole_f = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(whole), f));
-    const float parts = parts_of_bag(bag_f, inv_unit, most);
-    tiles += whole_f > 0.f ? whole_f : batch * parts;
-    part = fmaxf(part, bag_f * __builtin_amdgcn_rcpf(parts));
-  }
-  const bool fits = tiles <= rounds * grid && unit >= static_cast<float>(kSplitFloorUnit) &&
-                    unit >= static_cast<float>(tile_size);
-  const float price = fits ? rounds * (part + static_cast<float>(kSplitPartCost)) : 3.4e38f;
+  for (int f = 0; f < F; ++f)
+    tally.add<DeviceRcp>(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(bag), f)),
+                         __builtin_amdgcn_readlane(whole_tiles, f), B, inv_unit, most);
+  const float price = tally.price(unit, tile_size, grid, split_unit_rounds(lane));
   const float least = wave_min(price);
-  const unsigned long long best = __builtin_amdgcn_ballot_w64(fits && price == least);
-  return best ? __builtin_amdgcn_readlane(static_cast<int>(unit), __builtin_ctzll(best)) : 0;
+  const unsigned long long best = __builtin_amdgcn_ballot_w64(price == least);
+  return least < 3e38f ? __builtin_amdgcn_readlane(unit, __builtin_ctzll(best)) : 0;
 }
 
 template <int F, int BT, bool SPLIT = false, bool ONE_CAND = false>
@@ -431,7 +337,7 @@ bind_tiles(BindingStorage<F> &s, const IoView &io, const int tile_bytes,
   // (one sample: a tile per feature whatever its size)
   const bool need_total = (automatic && B > 1) || (SPLIT && !fixed_tiles);
   int tile_size = automatic ? kAutoTileMin : tile_bytes;
-  long long split_unit = 0;
+  float total_traffic = 0.f;
   if (need_total) {
     float total = wave_sum(traffic);
     if constexpr (!ONE_WAVE) {
@@ -446,47 +352,24 @@ bind_tiles(BindingStorage<F> &s, const IoView &io, const int tile_bytes,
     const long long total_bytes = static_cast<long long>(total);
     if (automatic) tile_size = tile_bytes < 0 ? capped_tile_size(-tile_bytes, total_bytes, grid_blocks)
                                               : auto_tile_size(total_bytes, grid_blocks);
-    if (SPLIT) {
-      const long long grid = grid_blocks > 0 ? grid_blocks : 1;
-      split_unit = total_bytes / (4ll * grid);
-      if (split_unit < tile_size) split_unit = tile_size;
-      if (split_unit < kSplitMinUnit) {
-        // whole tiles per workgroup at about the minimum part size, and 6 % of slack for the
-        // rounding up of every feature's parts per bag
-        const long long per_workgroup = (total_bytes + grid * kSplitMinUnit - 1) / (grid * kSplitMinUnit);
-        split_unit = total_bytes / (grid * (per_workgroup > 0 ? per_workgroup : 1));
-        split_unit += split_unit >> 4;
-        if (split_unit > kSplitMinUnit) split_unit = kSplitMinUnit;
-        if (split_unit < kSplitFloorUnit) split_unit = kSplitFloorUnit;
-        if (split_unit < tile_size) split_unit = tile_size;
-        if constexpr (F <= kSplitSearchFeats) {
-          // one round of parts of kSplitMinUnit or less is what the rule above gives by itself
-          if (tid < 64 && total_bytes > grid * kSplitMinUnit) {
-            const int searched = search_split_unit<F>(cost[0], gran[0], B, tile_size, total, static_cast<float>(grid));
-            if (searched > 0) split_unit = searched;
-          }
-        }
-      }
-    }
+    total_traffic = total;
   }
 
-  // Step 3: tiles of every feature, from registers.  Traffic figures in single precision;
-  // the quotients that decide which bags a tile holds exact.
+  // Step 3: tiles of every feature, from registers, its bags left whole.  Traffic figures in single
+  // precision; the quotients that decide which bags a tile holds exact.
   const float tile_f = static_cast<float>(tile_size);
   const float inv_tile = __builtin_amdgcn_rcpf(tile_f);
   const float inv_batch = B > 0 ? __builtin_amdgcn_rcpf(static_cast<float>(B)) : 0.f;
-  const float split_unit_f = static_cast<float>(split_unit);
   const bool small = B < kSmallDivBatch;
   // "tiles in plenty" below: (B / g) * F >= kPlentyTilesPerWorkgroup * grid  <=>  B >= g * need
   const int plenty_need = grid_blocks > 0
       ? static_cast<int>((static_cast<long long>(kPlentyTilesPerWorkgroup) * grid_blocks + F - 1) / F) : 0;
-  int tiles_of[K];
+  int tiles_of[K], bags_of[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const bool real = tid + k * BT < F;
     const int f = min(tid + k * BT, F - 1);
     int g = gran[k];
-    const bool may_split = g == kSplitGran && !fixed_tiles;
     if (g == kSplitGran) g = 1;
     // mean traffic of one bag of this feature
     const float bag_cost = cost[k] * inv_batch;
@@ -499,13 +382,7 @@ bind_tiles(BindingStorage<F> &s, const IoView &io, const int tile_bytes,
       tiles = static_cast<int>(fminf(fmaxf(want, 1.f), static_cast<float>(B)));
     }
     int bpt = 0;
-    int parts = 1;
-    if (SPLIT && may_split && split_unit > 0)
-      parts = static_cast<int>(parts_of_bag(bag_cost, __builtin_amdgcn_rcpf(split_unit_f), split_parts_most(B)));
-    if (parts > 1) {
-      tiles = B * parts;
-      bpt = -parts;
-    } else if (B > 0) {
+    if (B > 0) {
       bpt = small ? div_small(B + tiles - 1, tiles) : (B + tiles - 1) / tiles;
       // Tiles are whole workgroup passes (g bags) -- unless one pass of this schedule is more
       // than kMaxTileFactor times the traffic a tile should carry AND whole passes would leave
@@ -526,10 +403,36 @@ bind_tiles(BindingStorage<F> &s, const IoView &io, const int tile_bytes,
     } else {
       tiles = 0;
     }
-    // (a surplus thread may have sized its tiles from another wavefront's view of the total)
-    if (real) s.bags_per_tile[f] = bpt;
+    bags_of[k] = bpt;
     tiles_of[k] = real ? tiles : 0;
   }
+  // ... and where a bag is worth splitting, the parts of all its bags.
+  if (SPLIT && !fixed_tiles) {
+    const int grid = grid_blocks > 0 ? grid_blocks : 1;
+    const long long total_bytes = static_cast<long long>(total_traffic);
+    long long split_unit = split_unit_rule(total_bytes, grid, tile_size);
+    if constexpr (F <= kSplitSearchFeats) {
+      if (tid < 64 && search_is_due(total_bytes, grid, tile_size)) {
+        const int searched = search_split_unit<F>(gran[0] == kSplitGran ? cost[0] * inv_batch : 0.f, tiles_of[0], B,
+                                                  tile_size, total_traffic, grid);
+        if (searched > 0) split_unit = searched;
+      }
+    }
+    const float inv_unit = DeviceRcp::rcp(static_cast<float>(split_unit)), most = split_parts_most(B);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const float bag = gran[k] == kSplitGran ? cost[k] * inv_batch : 0.f;
+      const int parts = static_cast<int>(parts_of_bag(bag, inv_unit, most));
+      if (parts > 1) {
+        bags_of[k] = -parts;
+        tiles_of[k] = tid + k * BT < F ? B * parts : 0;
+      }
+    }
+  }
+  // (a surplus thread may have sized its tiles from another wavefront's view of the total)
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    if (tid + k * BT < F) s.bags_per_tile[tid + k * BT] = bags_of[k];
 
   // Step 4: prefix[f] = first tile of feature f.
   if constexpr (ONE_WAVE) {

@@ -40,6 +40,7 @@ its library is missing.  Names:
                    ``fewbags_unsplit``: the same with one workgroup per bag, for comparison;
                    ``fewbags64`` / ``fewbags128`` / ``fewbags512``: the same lookups as 64 x 4 000,
                    128 x 2 500 and 512 x 1 000
+``fewbags_even``   8 like features x 16 samples x exactly 20 000 lookups, bound once per launch
 ``manysplit``      17 fp16 features of dim 256 under the split-bag schedule: 36 MB of workspace,
                    more than the static array of ``recom_process_static_workspace`` may hold
 ``refa``, ``reff4`` models shaped like the reference's example models A and a quarter of F (1 000 and
@@ -277,6 +278,15 @@ def _few_bags(split: bool, bags: int = 16, lookups: float = 20000.0) -> ModelSpe
     return ModelSpec(wl, fs, 8)
 
 
+def _few_even_bags() -> ModelSpec:
+    """Few bags of one and the same cost, in eight like features: as many parts as the grid has
+    workgroups, or just more.  Bound once per launch, so that the workspace tells the tiles."""
+    feats = tuple(FeatureSpec(5000, 64, "float", 20000.0, True, 0.0, 1.0) for _ in range(8))
+    wl = Workload("fewbags_even", 16, 78, feats, "integer")
+    fs = default_feat_schedules(metas_of(wl), [f.mean_bag for f in feats], BLOCK_THREADS)
+    return ModelSpec(wl, fs, 8, dict(bind_once=True))
+
+
 def _many_split() -> ModelSpec:
     """More split-bag workspace than a library's static device array may hold (32 MiB)."""
     feats = tuple(FeatureSpec(5000 + f, 256, "half", 3000.0, False, 0.0, 1.0) for f in range(17))
@@ -380,6 +390,7 @@ _SPECS: Dict[str, Callable[[], ModelSpec]] = {
     "fewbags_unsplit": lambda: _few_bags(False),
     "fewbags64": lambda: _few_bags(True, 64, 4000.0),
     "fewbags128": lambda: _few_bags(True, 128, 2500.0),
+    "fewbags_even": _few_even_bags,
     "fewbags512": lambda: _few_bags(True, 512, 1000.0),
     "manysplit": _many_split,
     "wide": _wide,

@@ -733,3 +733,31 @@ def test_part_sizes_that_fill_rounds_of_the_grid(bags, mean, grid):
     for _ in range(2):
         got = layer.forward_indices(bound, grid_blocks=grid).cpu().numpy()
         assert np.array_equal(got, want)
+
+
+def _bound_tiles(layer):
+    """Tiles per feature of the last launch of a library that is bound once per launch: the binding
+    kernel's table (prefix[F + 1], bags_per_tile[F], cand[F]) ends the workspace."""
+    n = layer.lib.num_features
+    table = layer.workspace.cpu().numpy()[-(3 * n + 1):]
+    return np.diff(table[:n + 1])
+
+
+def test_bags_of_one_cost_fill_one_round_of_the_grid():
+    """8 features of 16 bags of 20 000 lookups on 2 048 workgroups: 16 parts a bag are one tile per
+    workgroup, and a part size that is off by a byte makes 17 of them, two rounds."""
+    import torch
+    from recflex_amd import prebuilt
+    from recflex_amd.rec_modules import FeatEmbed
+    from recflex_amd.workloads import gen_inputs, gen_tables
+    wl = prebuilt.model_spec("fewbags_even").workload
+    print("[case] fewbags_even, 2 048 workgroups", flush=True)
+    dev = torch.device("cuda", 0)
+    tables = gen_tables(wl, dev)
+    indices, offsets = gen_inputs(wl)
+    layer = FeatEmbed(dev, embed_tables=tables, librecom=require_lib("fewbags_even"))
+    bound = layer.bind_inputs([torch.from_numpy(i).to(dev) for i in indices],
+                              [torch.from_numpy(o).to(dev) for o in offsets])
+    got = layer.forward_indices(bound, grid_blocks=2048).cpu().numpy()
+    assert np.array_equal(got, oracle_output(wl, [t.cpu().numpy() for t in tables], indices, offsets))
+    assert _bound_tiles(layer).tolist() == [16 * 16] * 8

@@ -1,0 +1,87 @@
+"""CPU: the part sizes of split bags (``rfx_tile_sizes.h``, the functions the device runs): what a size
+is counted with is what the batch is cut into, and models of equal features fill their rounds of
+the grid."""
+
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from helpers import ROOT
+
+PART_COST = 35 * 1024           # rfx::kSplitPartCost
+MIN_UNIT = 256 * 1024           # rfx::kSplitMinUnit
+
+
+@pytest.fixture(scope="module")
+def model(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("tile_sizes") / "model.so")
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-shared", "-fPIC", "-ffp-contract=off",
+                    f"-I{ROOT}/recflex_amd/csrc/include", os.path.join(ROOT, "tests", "cpu", "tile_sizes_model.cpp"),
+                    "-o", lib], check=True)
+    return ctypes.CDLL(lib)
+
+
+def bind(model, cost, gran, batch, grid, tile_size):
+    n = len(cost)
+    cost, gran = np.asarray(cost, np.float32), np.asarray(gran, np.int32)
+    tiles, rule_tiles, out = np.zeros(n, np.int32), np.zeros(n, np.int32), np.zeros(3, np.int64)
+    longest, rule_longest = np.zeros(1, np.float32), np.zeros(1, np.float32)
+    ptr = [a.ctypes.data_as(ctypes.c_void_p) for a in (cost, gran, tiles, longest, rule_tiles, rule_longest, out)]
+    model.model_bind(n, batch, grid, tile_size, *ptr)
+    price = [-(-int(t.sum()) // grid) * (float(l[0]) + PART_COST)
+             for t, l in ((tiles, longest), (rule_tiles, rule_longest))]
+    return dict(unit=int(out[0]), counted=int(out[1]), rule=int(out[2]), tiles=tiles, price=price[0],
+                rule_price=price[1])
+
+
+def split_cost(batch, lookups, dim):
+    """Traffic of a feature as the emitter counts it: rows and indices, output rows and offsets."""
+    return batch * lookups * (4.0 * dim + 4) + batch * (4.0 * dim + 4)
+
+
+@pytest.mark.parametrize("features, dim, batch, lookups", [
+    (8, 64, 16, 20000), (4, 128, 16, 20000), (2, 256, 16, 20000), (16, 64, 16, 20000), (8, 64, 64, 5000),
+    (8, 64, 32, 10000), (1, 128, 16, 100000), (16, 32, 8, 40000), (3, 64, 100, 2222), (7, 96, 48, 4321)])
+@pytest.mark.parametrize("grid", [2048, 1280, 1024, 304, 100])
+def test_equal_features_fill_their_rounds(model, features, dim, batch, lookups, grid):
+    """Bags of one cost: the parts of a round are at most ``grid // bags`` per bag, and no size leaves
+    a round that a share of the batch in that many rounds would fill."""
+    got = bind(model, [split_cost(batch, lookups, dim)] * features, [-1] * features, batch, grid, 65536)
+    if got["counted"] < 0:
+        assert got["unit"] == got["rule"]
+        return
+    bags, bag = features * batch, split_cost(batch, lookups, dim) / batch
+    assert got["counted"] == got["tiles"].sum()
+    best = min(-(-bags * p // grid) * (bag / p + PART_COST)
+               for r in range(1, 5) for p in [max(1, min(64, 2048 // batch, grid * r // bags))]
+               if bag / p >= 131072 and (p == 1 or p > 1.25) and bag / p >= 65536)
+    # at least as good as the most parts that one, two, three or four rounds hold
+    assert got["price"] <= best * (1 + 1e-5), got
+
+
+def test_random_models_count_what_they_bind(model):
+    rng = np.random.default_rng(1)
+    searched = 0
+    for _ in range(20000):
+        n = int(rng.integers(1, 17))
+        grid = int(rng.choice([2048, 1280, 1024, 304, int(rng.integers(1, 4096))]))
+        batch = int(np.exp(rng.uniform(0, np.log(4096))))
+        tile_size = int(rng.choice([4096, 32768, 65536, 131072, 262144, 300000]))
+        # around the window in which sizes are searched: 256 KiB to 1 MiB of traffic per workgroup
+        share = np.exp(rng.uniform(np.log(128 * 1024), np.log(2 << 20)))
+        weight = rng.random(n) + 0.05 if rng.random() < 0.7 else np.ones(n)
+        cost = share * grid * weight / weight.sum()
+        gran = np.where(rng.random(n) < 0.75, -1, rng.choice([1, 4, 16, 64], n))
+        got = bind(model, cost, gran, batch, grid, tile_size)
+        case = (n, grid, batch, tile_size, cost.tolist(), gran.tolist(), got)
+        if got["counted"] < 0:
+            assert got["unit"] == got["rule"], case
+            continue
+        searched += 1
+        assert got["counted"] == got["tiles"].sum(), case
+        assert all(t <= 2048 for t, g in zip(got["tiles"], gran) if g == -1 and t > batch), case
+    assert searched > 5000
+
