@@ -205,25 +205,25 @@ struct DeviceRcp {
 
 // The part size of a model of few features, by its first wavefront.  Lane f < F holds, of feature f:
 // the mean traffic of a bag (0 if its schedule does not split), and the tiles it has as long as its
-// bags are left whole.  Every lane takes one candidate and counts its tiles; of those that fit their
-// rounds the one with the least rounds * (part + kSplitPartCost) wins.  0: none fits.  The same value
-// in every lane.
+// bags are left whole and the traffic of one of them.  Every lane takes one candidate and counts; the
+// same value in every lane.
 template <int F>
 __device__ __forceinline__ int
-search_split_unit(const float bag, const int whole_tiles, const int B, const int tile_size, const float total,
-                  const int grid) {
-  const int lane = threadIdx.x & 63;
-  const int unit = split_unit_candidate<DeviceRcp>(lane, total, grid);
+search_split_unit(const float bag, const int whole_tiles, const float whole_tile, const int B,
+                  const int tile_size, const float total, const int grid, const int rule) {
+  const int unit = split_unit_candidate<DeviceRcp>(threadIdx.x & 63, total, grid, rule);
   const float inv_unit = DeviceRcp::rcp(static_cast<float>(unit)), most = split_parts_most(B);
   SplitTally tally;
 #pragma unroll
   for (int f = 0; f < F; ++f)
     tally.add<DeviceRcp>(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(bag), f)),
-                         __builtin_amdgcn_readlane(whole_tiles, f), B, inv_unit, most);
-  const float price = tally.price(unit, tile_size, grid, split_unit_rounds(lane));
+                         __builtin_amdgcn_readlane(whole_tiles, f),
+                         __int_as_float(__builtin_amdgcn_readlane(__float_as_int(whole_tile), f)), B, inv_unit, most);
+  const float price = tally.price(unit, tile_size, grid);
   const float least = wave_min(price);
+  // (never empty: the rule's own size has a price)
   const unsigned long long best = __builtin_amdgcn_ballot_w64(price == least);
-  return least < 3e38f ? __builtin_amdgcn_readlane(unit, __builtin_ctzll(best)) : 0;
+  return best ? __builtin_amdgcn_readlane(unit, __builtin_ctzll(best)) : rule;
 }
 
 template <int F, int BT, bool SPLIT = false, bool ONE_CAND = false>
@@ -365,74 +365,79 @@ bind_tiles(BindingStorage<F> &s, const IoView &io, const int tile_bytes,
   const int plenty_need = grid_blocks > 0
       ? static_cast<int>((static_cast<long long>(kPlentyTilesPerWorkgroup) * grid_blocks + F - 1) / F) : 0;
   int tiles_of[K], bags_of[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const bool real = tid + k * BT < F;
-    const int f = min(tid + k * BT, F - 1);
-    int g = gran[k];
-    if (g == kSplitGran) g = 1;
-    // mean traffic of one bag of this feature
-    const float bag_cost = cost[k] * inv_batch;
-    int tiles;
-    if (fixed_tiles) {
-      const int want = fixed_tiles[f];
-      tiles = want < 1 ? 1 : (want > B ? B : want);
-    } else {
-      const float want = ceilf(cost[k] * inv_tile);
-      tiles = static_cast<int>(fminf(fmaxf(want, 1.f), static_cast<float>(B)));
-    }
-    int bpt = 0;
-    if (B > 0) {
-      bpt = small ? div_small(B + tiles - 1, tiles) : (B + tiles - 1) / tiles;
-      // Tiles are whole workgroup passes (g bags) -- unless one pass of this schedule is more
-      // than kMaxTileFactor times the traffic a tile should carry AND whole passes would leave
-      // the grid short of tiles: then the tile keeps its share of the traffic and some of the
-      // schedule's teams idle (a small batch is spread over more workgroups that way).  With
-      // tiles in plenty -- this feature's whole passes times the number of features is at
-      // least kPlentyTilesPerWorkgroup tiles per workgroup of the grid -- idle teams are a pure
-      // loss: a batch whose bags are twice as long as the tile size was chosen for ran 262 us
-      // with a quarter of the wavefronts busy in the long-bag features, 197 us with whole passes.
-      const int passes = small ? div_small(bpt + g - 1, g) : (bpt + g - 1) / g;
-      const int whole = passes * g;
-      const bool plenty = grid_blocks > 0 &&
-                          static_cast<long long>(B) >= static_cast<long long>(g) * plenty_need;
-      if (fixed_tiles || bpt >= g || plenty ||
-          static_cast<float>(whole) * bag_cost <= static_cast<float>(kMaxTileFactor) * tile_f)
-        bpt = whole;
-      tiles = small ? div_small(B + bpt - 1, bpt) : (B + bpt - 1) / bpt;
-    } else {
-      tiles = 0;
-    }
-    bags_of[k] = bpt;
-    tiles_of[k] = real ? tiles : 0;
-  }
-  // ... and where a bag is worth splitting, the parts of all its bags.
-  if (SPLIT && !fixed_tiles) {
-    const int grid = grid_blocks > 0 ? grid_blocks : 1;
-    const long long total_bytes = static_cast<long long>(total_traffic);
-    long long split_unit = split_unit_rule(total_bytes, grid, tile_size);
-    if constexpr (F <= kSplitSearchFeats) {
-      if (tid < 64 && search_is_due(total_bytes, grid, tile_size)) {
-        const int searched = search_split_unit<F>(gran[0] == kSplitGran ? cost[0] * inv_batch : 0.f, tiles_of[0], B,
-                                                  tile_size, total_traffic, grid);
-        if (searched > 0) split_unit = searched;
-      }
-    }
-    const float inv_unit = DeviceRcp::rcp(static_cast<float>(split_unit)), most = split_parts_most(B);
+  // (up to 64 features: by the first wavefront, the others have none; with eight workgroups on a CU
+  // the other three made the binding 0.4 us longer)
+  if (!ONE_WAVE || tid < 64) {
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-      const float bag = gran[k] == kSplitGran ? cost[k] * inv_batch : 0.f;
-      const int parts = static_cast<int>(parts_of_bag(bag, inv_unit, most));
-      if (parts > 1) {
-        bags_of[k] = -parts;
-        tiles_of[k] = tid + k * BT < F ? B * parts : 0;
+      const bool real = tid + k * BT < F;
+      const int f = min(tid + k * BT, F - 1);
+      int g = gran[k];
+      if (g == kSplitGran) g = 1;
+      // mean traffic of one bag of this feature
+      const float bag_cost = cost[k] * inv_batch;
+      int tiles;
+      if (fixed_tiles) {
+        const int want = fixed_tiles[f];
+        tiles = want < 1 ? 1 : (want > B ? B : want);
+      } else {
+        const float want = ceilf(cost[k] * inv_tile);
+        tiles = static_cast<int>(fminf(fmaxf(want, 1.f), static_cast<float>(B)));
+      }
+      int bpt = 0;
+      if (B > 0) {
+        bpt = small ? div_small(B + tiles - 1, tiles) : (B + tiles - 1) / tiles;
+        // Tiles are whole workgroup passes (g bags) -- unless one pass of this schedule is more
+        // than kMaxTileFactor times the traffic a tile should carry AND whole passes would leave
+        // the grid short of tiles: then the tile keeps its share of the traffic and some of the
+        // schedule's teams idle (a small batch is spread over more workgroups that way).  With
+        // tiles in plenty -- this feature's whole passes times the number of features is at
+        // least kPlentyTilesPerWorkgroup tiles per workgroup of the grid -- idle teams are a pure
+        // loss: a batch whose bags are twice as long as the tile size was chosen for ran 262 us
+        // with a quarter of the wavefronts busy in the long-bag features, 197 us with whole passes.
+        const int passes = small ? div_small(bpt + g - 1, g) : (bpt + g - 1) / g;
+        const int whole = passes * g;
+        const bool plenty = grid_blocks > 0 &&
+                            static_cast<long long>(B) >= static_cast<long long>(g) * plenty_need;
+        if (fixed_tiles || bpt >= g || plenty ||
+            static_cast<float>(whole) * bag_cost <= static_cast<float>(kMaxTileFactor) * tile_f)
+          bpt = whole;
+        tiles = small ? div_small(B + bpt - 1, bpt) : (B + bpt - 1) / bpt;
+      } else {
+        tiles = 0;
+      }
+      bags_of[k] = bpt;
+      tiles_of[k] = real ? tiles : 0;
+    }
+    // ... and where a bag is worth splitting, the parts of all its bags.
+    if (SPLIT && !fixed_tiles) {
+      const int grid = grid_blocks > 0 ? grid_blocks : 1;
+      const long long total_bytes = static_cast<long long>(total_traffic);
+      long long split_unit = split_unit_rule(total_bytes, grid, tile_size);
+      if constexpr (F <= kSplitSearchFeats) {
+        if (search_is_due(total_bytes, grid, tile_size)) {
+          const float bag = cost[0] * inv_batch;
+          split_unit = search_split_unit<F>(gran[0] == kSplitGran ? bag : 0.f, tiles_of[0],
+                                            static_cast<float>(bags_of[0]) * bag, B, tile_size, total_traffic, grid,
+                                            static_cast<int>(split_unit));
+        }
+      }
+      const float inv_unit = DeviceRcp::rcp(static_cast<float>(split_unit)), most = split_parts_most(B);
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const float bag = gran[k] == kSplitGran ? cost[k] * inv_batch : 0.f;
+        const int parts = static_cast<int>(parts_of_bag(bag, inv_unit, most));
+        if (parts > 1) {
+          bags_of[k] = -parts;
+          tiles_of[k] = tid + k * BT < F ? B * parts : 0;
+        }
       }
     }
-  }
-  // (a surplus thread may have sized its tiles from another wavefront's view of the total)
+    // (a surplus thread may have sized its tiles from another wavefront's view of the total)
 #pragma unroll
-  for (int k = 0; k < K; ++k)
-    if (tid + k * BT < F) s.bags_per_tile[tid + k * BT] = bags_of[k];
+    for (int k = 0; k < K; ++k)
+      if (tid + k * BT < F) s.bags_per_tile[tid + k * BT] = bags_of[k];
+  }
 
   // Step 4: prefix[f] = first tile of feature f.
   if constexpr (ONE_WAVE) {

@@ -76,11 +76,12 @@ constexpr int kSplitMinUnit = 256 * 1024;
 // 256 KiB are 1.4 tiles per workgroup, i.e. two rounds with the second a third full, 94 us;
 // 3 872 parts of 199 KiB are 1.9, 88 us).
 constexpr int kSplitFloorUnit = 128 * 1024;
-// Models of up to kSplitSearchFeats features count the tiles that a part size would give, and take the
-// size whose tiles fill a whole number of rounds of the grid (rfx::search_split_unit).  (16 x 20 000
-// lookups, 2 048 workgroups, in us: 3 712 parts of 200 KiB 85, 2 176 of 340 KiB 104, 1 984 of 384 KiB
-// 74, 1 696 of 440 KiB 80; 128 x 2 500: 2 304 tiles 99, 2 048 of them 77.)  Counting takes a few
-// instructions per feature in every workgroup, hence the limit.
+// Models of up to kSplitSearchFeats features go by more than that rule: they count the tiles that a part
+// size would give, the rule's among 64 of them, and take the size whose rounds of the grid, each as
+// long as the longest tile, are over first.  (16 x 20 000 lookups, 2 048 workgroups, in us: 3 712
+// parts of 200 KiB 85, 2 176 of 340 KiB 104, 1 984 of 384 KiB 74, 1 696 of 440 KiB 80; 128 x 2 500:
+// 2 304 tiles 99, 2 048 of them 77.)  Counting takes a few instructions per feature in every
+// workgroup, hence the limit.
 constexpr int kSplitSearchFeats = 16;
 constexpr int kSplitPartCost = 35 * 1024;      // a part's round trips, in traffic
 constexpr int kSplitGran = -1;
@@ -125,36 +126,40 @@ RFX_SIZES_FN bool search_is_due(const long long total, const int grid, const int
 }
 
 // The part size that lane 0 .. 63 looks at: a workgroup's share of the batch in 1 to 4 rounds, enlarged
-// by 0 to 15 sixteenths.
+// by 0 to 15 sixteenths -- and the rule's, so that nothing is chosen that is dearer by the same count
+// (8 features of 878 bags of 600 / 900 lookups, 2 048 workgroups: 128.6 / 186.8 us where any size that
+// filled one to four rounds was taken, 116.7 / 168.8 us where the rule's more and shorter rounds count).
 // A whole number, since what is counted with it has to be what the tiles are made with, and beyond the
 // share by at least one byte, more than the figures' rounding errors of a few 2^-24 come to at shares
 // of up to 1 MiB: bags of equal cost come out at the number of parts that fills the round, not at one
 // more (8 features of 16 x 20 000 lookups, dim 64: 2 048 tiles on 2 048 workgroups, 63.7 us, where a size
 // cut off to the byte below made 2 176, two rounds, 86.4 us; 4 of dim 128 64.3 and 86.3, 16 of dim 64
 // 127.1 and 170.5).
-RFX_SIZES_FN int split_unit_rounds(const int lane) { return 1 + (lane >> 4); }
 template <typename M>
-RFX_SIZES_FN int split_unit_candidate(const int lane, const float total, const int grid) {
-  const float share = total * M::rcp(static_cast<float>(split_unit_rounds(lane)) * static_cast<float>(grid));
+RFX_SIZES_FN int split_unit_candidate(const int lane, const float total, const int grid, const int rule) {
+  if (lane == 63) return rule;
+  const float share = total * M::rcp(static_cast<float>(1 + (lane >> 4)) * static_cast<float>(grid));
   return static_cast<int>(share * (1.f + 0.0625f * static_cast<float>(lane & 15))) + 2;
 }
 
 // What a part size comes to, feature by feature.
 struct SplitTally {
   int tiles = 0;
-  float longest = 0.f;                          // the longest part
+  float longest = 0.f;                          // traffic of the longest tile
 
-  // bag: mean traffic of one of the feature's bags (0: its schedule does not split); whole_tiles: its
-  // tiles with the bags left whole
+  // bag: mean traffic of one of the feature's bags (0: its schedule does not split); whole_tiles and
+  // whole_tile: its tiles with the bags left whole, and the traffic of one
   template <typename M>
-  RFX_SIZES_FN void add(const float bag, const int whole_tiles, const int batch, const float inv_unit, const float most) {
+  RFX_SIZES_FN void add(const float bag, const int whole_tiles, const float whole_tile, const int batch,
+                        const float inv_unit, const float most) {
     const float parts = parts_of_bag(bag, inv_unit, most);
-    tiles += parts > 1.f ? batch * static_cast<int>(parts) : whole_tiles;
-    longest = __builtin_fmaxf(longest, bag * M::rcp(parts));
+    const bool split = parts > 1.f;
+    tiles += split ? batch * static_cast<int>(parts) : whole_tiles;
+    longest = __builtin_fmaxf(longest, split ? bag * M::rcp(parts) : whole_tile);
   }
-  // of a size whose tiles fit into `rounds` of the grid
-  RFX_SIZES_FN float price(const int unit, const int tile_size, const int grid, const int rounds) const {
-    if (unit < kSplitFloorUnit || unit < tile_size || tiles > rounds * grid) return 3.4e38f;
+  RFX_SIZES_FN float price(const int unit, const int tile_size, const int grid) const {
+    if (unit < kSplitFloorUnit || unit < tile_size) return 3.4e38f;
+    const int rounds = (tiles + grid - 1) / grid;
     return static_cast<float>(rounds) * (longest + static_cast<float>(kSplitPartCost));
   }
 };

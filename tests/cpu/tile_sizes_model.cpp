@@ -40,7 +40,7 @@ static void apply(int F, int B, int grid, int tile_size, const float *cost, cons
   }
 }
 
-// out: {part size chosen, tiles it was counted with (-1: none was), the rule's part size}; tiles[f]
+// out: {part size chosen, tiles it was counted with (-1: no search), the rule's part size}; tiles[f]
 // and longest as they are bound, rule_tiles / rule_longest as the rule alone would
 void model_bind(int F, int B, int grid, int tile_size, const float *cost, const int *gran, int *tiles,
                 float *longest, int *rule_tiles, float *rule_longest, long long *out) {
@@ -52,18 +52,20 @@ void model_bind(int F, int B, int grid, int tile_size, const float *cost, const 
   apply(F, B, grid, tile_size, cost, gran, static_cast<float>(unit), rule_tiles, rule_longest);
   if (F <= rfx::kSplitSearchFeats && rfx::search_is_due(static_cast<long long>(total), grid, tile_size)) {
     int whole[rfx::kSplitSearchFeats];
-    float ignored, best = 3e38f;
+    float ignored, best = 0.f;
     apply(F, B, grid, tile_size, cost, gran, 3e38f, whole, &ignored);        // no bag is worth splitting
+    const int rule = static_cast<int>(unit);
     for (int lane = 0; lane < 64; ++lane) {
-      const int candidate = rfx::split_unit_candidate<Rcp>(lane, total, grid);
+      const int candidate = rfx::split_unit_candidate<Rcp>(lane, total, grid, rule);
       rfx::SplitTally tally;
       for (int f = 0; f < F; ++f) {
         const float bag = cost[f] * (1.f / static_cast<float>(B));
-        tally.add<Rcp>(gran[f] == rfx::kSplitGran ? bag : 0.f, whole[f], B, 1.f / static_cast<float>(candidate),
-                       rfx::split_parts_most(B));
+        const int bpt = (B + whole[f] - 1) / whole[f];
+        tally.add<Rcp>(gran[f] == rfx::kSplitGran ? bag : 0.f, whole[f], static_cast<float>(bpt) * bag, B,
+                       1.f / static_cast<float>(candidate), rfx::split_parts_most(B));
       }
-      const float price = tally.price(candidate, tile_size, grid, rfx::split_unit_rounds(lane));
-      if (price < best) {
+      const float price = tally.price(candidate, tile_size, grid);
+      if (lane == 0 || price < best) {
         best = price;
         unit = candidate;
         out[1] = tally.tiles;

@@ -1,6 +1,6 @@
 """CPU: the part sizes of split bags (``rfx_tile_sizes.h``, the functions the device runs): what a size
-is counted with is what the batch is cut into, and models of equal features fill their rounds of
-the grid."""
+is counted with is what the batch is cut into, models of equal features fill their rounds of the
+grid, and no size is chosen that is dearer, by the same count, than the plain rule's."""
 
 import ctypes
 import os
@@ -62,7 +62,7 @@ def test_equal_features_fill_their_rounds(model, features, dim, batch, lookups, 
     assert got["price"] <= best * (1 + 1e-5), got
 
 
-def test_random_models_count_what_they_bind(model):
+def test_random_models_count_what_they_bind_and_never_lose(model):
     rng = np.random.default_rng(1)
     searched = 0
     for _ in range(20000):
@@ -82,6 +82,14 @@ def test_random_models_count_what_they_bind(model):
             continue
         searched += 1
         assert got["counted"] == got["tiles"].sum(), case
+        assert got["price"] <= got["rule_price"] * (1 + 1e-6), case
         assert all(t <= 2048 for t, g in zip(got["tiles"], gran) if g == -1 and t > batch), case
     assert searched > 5000
 
+
+def test_bags_just_below_the_split_limit_do_not_cost_rounds(model):
+    """878 bags of a quarter of a megabyte in eight features: left whole in four rounds of 527 KB by a
+    search that does not price the plain rule, five rounds of 263 KB by the rule."""
+    for mean in range(1000, 2200, 50):
+        got = bind(model, [split_cost(878, mean, 64)] * 8, [-1] * 8, 878, 2048, 65536)
+        assert got["price"] <= got["rule_price"] * (1 + 1e-6)
