@@ -130,14 +130,14 @@ def _frozen_binding(spec: ModelSpec) -> ModelSpec:
     """The model with the tiles per feature frozen at emit time to what the run-time binding
     chooses for the workload's own (seeded) batch: the fixed-thread-binding ablation."""
     from .code_emitter.codegen import BAG_FIXED_BYTES, DEFAULT_TILE_BYTES, INDEX_BYTES
-    from .tuning.measure import tiles_per_feature
+    from .tuning.measure import emitted_tile_bytes, tiles_per_feature
     from .workloads import gen_inputs
     _, offsets = gen_inputs(spec.workload)
     metas = [s.meta for s, _ in spec.feat_schedules]
     counts = tiles_per_feature(offsets, [m.row_bytes + INDEX_BYTES for m in metas],
                                [m.embed_dim * 4 + BAG_FIXED_BYTES for m in metas],
                                [s.TileGranularity(p) for s, p in spec.feat_schedules],
-                               spec.emit_kwargs.get("tile_bytes") or DEFAULT_TILE_BYTES,
+                               emitted_tile_bytes(spec.emit_kwargs.get("tile_bytes") or DEFAULT_TILE_BYTES),
                                grid_blocks=TUNE_FIXTURE_SM_COUNT * (spec.occupancy or DEFAULT_OCCUPANCY))
     return spec._replace(emit_kwargs=dict(_plain_walk(spec.emit_kwargs),
                                           fixed_task_block_nums=[max(1, c) for c in counts]))

@@ -529,6 +529,32 @@ PLENTY_TILES_PER_WORKGROUP = 2                      # rfx::kPlentyTilesPerWorkgr
 AUTO_TILES_PER_WORKGROUP = 64                       # rfx::kAutoTilesPerWorkgroup
 AUTO_TILE_MIN, AUTO_TILE_MAX = 64 * 1024, 256 * 1024    # rfx::kAutoTileMin / kAutoTileMax
 AUTO_TILE_FLOOR = 4 * 1024                              # rfx::kAutoTileFloor
+CAPPED_TILES_PER_WORKGROUP = 5                          # rfx::kCappedTilesPerWorkgroup
+
+
+def batch_traffic(offsets: Sequence[np.ndarray], lookup_bytes: Sequence[int], bag_bytes: Sequence[int]) -> int:
+    """The traffic of a batch as the binding counts it."""
+    total = 0
+    for off, lb, bb in zip(offsets, lookup_bytes, bag_bytes):
+        batch = len(off) - 1
+        if batch > 0:
+            total += int(off[-1] - off[0]) * lb + batch * bb
+    return total
+
+
+def capped_tile_bytes(built: int, total: int, grid_blocks: int) -> int:
+    """Host restatement of the tile size that a library emitted with ``built`` beyond 64 KiB runs a
+    batch of ``total`` bytes of traffic with (``rfx::capped_tile_size``): smaller, down to 64 KiB,
+    for a batch of fewer than five such tiles per workgroup."""
+    t = total // (max(1, grid_blocks) * CAPPED_TILES_PER_WORKGROUP)
+    if t >= built or built <= AUTO_TILE_MIN:
+        return built
+    return t & ~1023 if t > AUTO_TILE_MIN else AUTO_TILE_MIN
+
+
+def emitted_tile_bytes(tile_bytes: int) -> int:
+    """What ``tiles_per_feature`` takes for a library emitted with ``tile_bytes``."""
+    return -tile_bytes if tile_bytes > AUTO_TILE_MIN else tile_bytes
 
 
 def auto_tile_bytes(offsets: Sequence[np.ndarray], lookup_bytes: Sequence[int],
@@ -537,11 +563,7 @@ def auto_tile_bytes(offsets: Sequence[np.ndarray], lookup_bytes: Sequence[int],
     (``rfx::auto_tile_size``): the batch's traffic over 64 tiles per workgroup of the grid, within
     64..256 KiB, in steps of 4 KiB; a batch of less than 64 KiB per workgroup gets about two tiles
     per workgroup, at least 4 KiB, in steps of 1 KiB."""
-    total = 0
-    for off, lb, bb in zip(offsets, lookup_bytes, bag_bytes):
-        batch = len(off) - 1
-        if batch > 0:
-            total += int(off[-1] - off[0]) * lb + batch * bb
+    total = batch_traffic(offsets, lookup_bytes, bag_bytes)
     grid = max(1, grid_blocks)
     t = total // (grid * AUTO_TILES_PER_WORKGROUP)
     if t >= AUTO_TILE_MIN:
@@ -557,10 +579,14 @@ def tiles_per_feature(offsets: Sequence[np.ndarray], lookup_bytes: Sequence[int]
     for this batch on a grid of ``grid_blocks`` workgroups (0: unknown, taken as too large for
     the whole-pass rule of plentiful tiles to apply).  A schedule that can split bags over
     workgroups (granularity -1) counts as one bag per workgroup pass: a binding frozen at emit
-    time never splits.  ``tile_bytes`` <= 0: the size the device picks for this batch."""
+    time never splits.  ``tile_bytes``: a size given with the launch, 0 the one the device picks for
+    this batch, below 0 what becomes of the size a library was emitted with (``emitted_tile_bytes``)."""
     out = []
     num_feats = len(offsets)
-    if tile_bytes <= 0:
+    if tile_bytes < 0:
+        # (one sample: a tile per feature whatever its size)
+        tile_bytes = capped_tile_bytes(-tile_bytes, batch_traffic(offsets, lookup_bytes, bag_bytes), grid_blocks)
+    elif tile_bytes == 0:
         tile_bytes = auto_tile_bytes(offsets, lookup_bytes, bag_bytes, grid_blocks)
     for off, lb, bb, g in zip(offsets, lookup_bytes, bag_bytes, gran):
         g = 1 if g < 0 else g

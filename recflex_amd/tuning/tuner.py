@@ -41,7 +41,7 @@ from recflex_amd.parser import (parse_raw_data_batches, parse_table_shapes, pars
                                 parse_schedule_types, parse_knl_total_time, parse_knl_batch_times)
 
 from .measure import (measure_single_feat, rocprof_profile, measure_task_blocks, measure_feature_ticks,
-                      tiles_per_feature,
+                      emitted_tile_bytes, tiles_per_feature,
                       measure_naive_candidate, measure_kernel_events, measure_tournament,
                       save_batches, KernelTimer, PROFILE_PASSES, PROFILE_WARMUP_PASSES)
 
@@ -1014,7 +1014,7 @@ class Tuner:
                                        [m.row_bytes + INDEX_BYTES for m in metas],
                                        [m.embed_dim * 4 + BAG_FIXED_BYTES for m in metas],
                                        [s.TileGranularity(p) for s, p in sched_params],
-                                       tile_bytes or tune_config.tile_bytes,
+                                       emitted_tile_bytes(tile_bytes or tune_config.tile_bytes),
                                        grid_blocks=tune_config.sm_count * occupancy)
         return tiles
 
@@ -1639,7 +1639,7 @@ class Tuner:
                                 [m.row_bytes + INDEX_BYTES for m in metas],
                                 [m.embed_dim * 4 + BAG_FIXED_BYTES for m in metas],
                                 [s.TileGranularity(p) for s, p in opt_sched_params],
-                                tune_config.tile_bytes, fixed_blocks_path,
+                                emitted_tile_bytes(tune_config.tile_bytes), fixed_blocks_path,
                                 grid_blocks=tune_config.sm_count * (occupancy or self.natural_occupancy_guess()))
 
         task_block_batches: List[List[int]] = []

@@ -93,3 +93,51 @@ def test_bags_just_below_the_split_limit_do_not_cost_rounds(model):
     for mean in range(1000, 2200, 50):
         got = bind(model, [split_cost(878, mean, 64)] * 8, [-1] * 8, 878, 2048, 65536)
         assert got["price"] <= got["rule_price"] * (1 + 1e-6)
+
+
+def test_host_restatements_of_the_tile_sizes(model):
+    """What the tuner computes on the host is what the device does: the size picked for a batch, and
+    what becomes of a size that a library was emitted with."""
+    from recflex_amd.tuning import measure
+    rng = np.random.default_rng(2)
+    cut = 0
+    for _ in range(5000):
+        total, grid = int(np.exp(rng.uniform(0, np.log(1e11)))), int(rng.integers(0, 4096))
+        built = int(rng.choice([4096, 65536, 65537, 131072, 262144, 1 << 20]))
+        want = model.model_capped_tile_size(built, ctypes.c_longlong(total), grid)
+        assert measure.capped_tile_bytes(built, total, grid) == want
+        cut += want < built
+        # one bag of one lookup, `total` bytes in all
+        off = np.array([0, 1], np.int64)
+        auto = model.model_auto_tile_size(ctypes.c_longlong(total), grid)
+        assert measure.auto_tile_bytes([off], [total - 1], [1], grid) == auto
+    assert cut > 500
+
+
+def test_tiles_of_a_library_emitted_with_large_tiles():
+    """The walk stage's tile counts and the frozen bindings are those of the library that runs: one
+    emitted with 256 KiB gives a batch of a few such tiles per workgroup smaller ones."""
+    from recflex_amd.tuning.measure import emitted_tile_bytes, tiles_per_feature
+    from recflex_amd.tuning.tuner import Tuner, TuneConfig
+    off = np.arange(0, 16385 * 10, 10, dtype=np.int64)      # 16 384 bags of 10 lookups
+    args = ([off] * 4, [516] * 4, [516] * 4, [4] * 4)       # 89 MiB each
+    # 355 MiB on 256 workgroups: 5.5 tiles of 256 KiB each; on 1 280: 64 KiB and more
+    assert tiles_per_feature(*args, emitted_tile_bytes(262144), grid_blocks=256) == \
+        tiles_per_feature(*args, 262144, grid_blocks=256)
+    assert tiles_per_feature(*args, emitted_tile_bytes(262144), grid_blocks=1280) == \
+        tiles_per_feature(*args, 65536, grid_blocks=1280) != tiles_per_feature(*args, 262144, grid_blocks=1280)
+    assert emitted_tile_bytes(65536) == 65536 and emitted_tile_bytes(0) == 0
+
+    class Sched:
+        class meta:
+            row_bytes, embed_dim = 512, 128
+
+        @staticmethod
+        def TileGranularity(params):
+            return 4
+
+    tuner = Tuner.__new__(Tuner)
+    tuner.num_feats, tuner.batches = 4, [[(None, off)] for _ in range(4)]
+    cfg = TuneConfig(occupancies=[5], gpu_ids=[0], sm_count=256)
+    tiles = tuner.sample_tiles([(Sched, None)] * 4, 5, 262144, cfg)
+    assert tiles.tolist() == tiles_per_feature(*args, 65536, grid_blocks=1280)
