@@ -366,7 +366,8 @@ def measure_kernel_events(librecom_path: str, table_shapes: Sequence[Tuple[int, 
                           tile_bytes: int = 0, xcd_segments: int = 0, repeats: int = 7, warmup: int = 10,
                           gpu_id: int = None) -> Optional[float]:
     """Total FusedKnl time in ns over all batches (median of ``repeats`` launches per batch),
-    measured with events on the launch stream; written to ``output_path``."""
+    measured with events on the launch stream; written to ``output_path``.  ``tile_bytes``: as if
+    the library had been emitted with it (0: as it was)."""
     try:
         _pin_gpu(gpu_id)
         import torch
@@ -382,11 +383,11 @@ def measure_kernel_events(librecom_path: str, table_shapes: Sequence[Tuple[int, 
             d_off = [torch.from_numpy(b[k][1]).to(dev) for b in per_feat]
             out = layer.forward_indices(d_idx, d_off)       # its buffer is reused below
             bound = layer.bind_inputs(d_idx, d_off)         # no per-feature host work when timed
+            tile = launch_tile_bytes(layer.lib, [b[k][1] for b in per_feat], tile_bytes)
             for _ in range(warmup):                         # let the clocks settle
-                layer.forward_indices(bound, out=out, tile_bytes=tile_bytes,
-                                      xcd_segments=xcd_segments)
+                layer.forward_indices(bound, out=out, tile_bytes=tile, xcd_segments=xcd_segments)
             total_ns += _timed_launches(
-                lambda: layer.forward_indices(bound, out=out, tile_bytes=tile_bytes,
+                lambda: layer.forward_indices(bound, out=out, tile_bytes=tile,
                                               xcd_segments=xcd_segments), repeats)
         _write_atomically(output_path, str(total_ns))
         return total_ns
@@ -414,10 +415,11 @@ def measure_feature_ticks(librecom_path: str, table_shapes: Sequence[Tuple[int, 
         for k in range(len(per_feat[0])):
             bound = layer.bind_inputs([torch.from_numpy(b[k][0]).to(dev) for b in per_feat],
                                       [torch.from_numpy(b[k][1]).to(dev) for b in per_feat])
-            out = layer.forward_indices(bound, tile_bytes=tile_bytes, xcd_segments=xcd_segments)
+            tile = launch_tile_bytes(layer.lib, [b[k][1] for b in per_feat], tile_bytes)
+            out = layer.forward_indices(bound, tile_bytes=tile, xcd_segments=xcd_segments)
             acc = np.zeros(len(per_feat), dtype=np.float64)
             for _ in range(repeats):
-                _, ticks = layer.forward_indices(bound, timing=True, out=out, tile_bytes=tile_bytes,
+                _, ticks = layer.forward_indices(bound, timing=True, out=out, tile_bytes=tile,
                                                  xcd_segments=xcd_segments)
                 acc += ticks.numpy()
             total += acc / repeats
@@ -555,6 +557,18 @@ def capped_tile_bytes(built: int, total: int, grid_blocks: int) -> int:
 def emitted_tile_bytes(tile_bytes: int) -> int:
     """What ``tiles_per_feature`` takes for a library emitted with ``tile_bytes``."""
     return -tile_bytes if tile_bytes > AUTO_TILE_MIN else tile_bytes
+
+
+def launch_tile_bytes(lib, offsets: Sequence[np.ndarray], tile_bytes: int) -> int:
+    """What to launch ``lib`` (a ``RecomLib``) on a batch with, so that it runs as the same library
+    emitted with ``tile_bytes`` would: a size given with a launch is taken as it is, an emitted one
+    is an upper bound for small batches."""
+    if tile_bytes <= AUTO_TILE_MIN:
+        return tile_bytes
+    from recflex_amd.code_emitter.codegen import BAG_FIXED_BYTES, INDEX_BYTES, LOOKUP_OVERHEAD_BYTES
+    total = batch_traffic(offsets, [b + INDEX_BYTES + LOOKUP_OVERHEAD_BYTES for b in lib.row_strides],
+                          [d * 4 + BAG_FIXED_BYTES for d in lib.embed_dims])
+    return capped_tile_bytes(tile_bytes, total, lib.get_max_concurrent_blocks())
 
 
 def auto_tile_bytes(offsets: Sequence[np.ndarray], lookup_bytes: Sequence[int],

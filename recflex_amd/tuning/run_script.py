@@ -21,6 +21,7 @@ if __name__ == "__main__":
     parser.add_argument("--sample_batch_nums", type=int, required=True)
     parser.add_argument("--seed", type=int, default=0)
     parser.add_argument("--repeats", type=int, default=1)
+    # as if the library had been emitted with it (0: as it was)
     parser.add_argument("--tile_bytes", type=int, default=0)
     parser.add_argument("--xcd_segments", type=int, default=0)
     args = parser.parse_args()
@@ -30,7 +31,7 @@ if __name__ == "__main__":
     from recflex_amd.host import RecomHost
     from recflex_amd.parser import parse_raw_data_batches, parse_table_dtypes, parse_table_shapes
     from recflex_amd.rec_modules import FeatEmbed
-    from recflex_amd.tuning.measure import load_batches, make_table
+    from recflex_amd.tuning.measure import launch_tile_bytes, load_batches, make_table
 
     table_shapes = parse_table_shapes(args.table_config_fname)
     data_types = parse_table_dtypes(args.table_config_fname)
@@ -53,14 +54,15 @@ if __name__ == "__main__":
     device_batches = []
     for k in range(len(per_feat[0])):
         device_batches.append(([torch.from_numpy(b[k][0]).to(dev) for b in per_feat],
-                               [torch.from_numpy(b[k][1]).to(dev) for b in per_feat]))
+                               [torch.from_numpy(b[k][1]).to(dev) for b in per_feat],
+                               launch_tile_bytes(layer.lib, [b[k][1] for b in per_feat], args.tile_bytes)))
     torch.cuda.synchronize()
 
     prof = HipProfiler()
     prof.start()
     for _ in range(args.repeats):
-        for d_idx, d_off in device_batches:
-            output = layer.forward_indices(d_idx, d_off, tile_bytes=args.tile_bytes,
+        for d_idx, d_off, tile_bytes in device_batches:
+            output = layer.forward_indices(d_idx, d_off, tile_bytes=tile_bytes,
                                            xcd_segments=args.xcd_segments)
     torch.cuda.synchronize()
     prof.stop()

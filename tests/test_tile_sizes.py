@@ -141,3 +141,40 @@ def test_tiles_of_a_library_emitted_with_large_tiles():
     cfg = TuneConfig(occupancies=[5], gpu_ids=[0], sm_count=256)
     tiles = tuner.sample_tiles([(Sched, None)] * 4, 5, 262144, cfg)
     assert tiles.tolist() == tiles_per_feature(*args, 65536, grid_blocks=1280)
+
+
+def test_the_sweep_times_the_library_that_ships(monkeypatch, tmp_path):
+    """A tile size beyond 64 KiB is tried as the library emitted with it would run each batch."""
+    import torch
+    from recflex_amd import rec_modules
+    from recflex_amd.tuning import measure
+    seen = []
+
+    class Layer:
+        class lib:
+            row_strides, embed_dims = [512] * 4, [128] * 4
+            get_max_concurrent_blocks = staticmethod(lambda: 1280)
+
+        def __init__(self, *args, **kwargs):
+            pass
+
+        def bind_inputs(self, indices, offsets):
+            return offsets
+
+        def forward_indices(self, indices, offsets=None, tile_bytes=0, **kwargs):
+            if offsets is None:
+                seen.append((indices[0].numel() - 1, tile_bytes))
+
+    monkeypatch.setattr(rec_modules, "FeatEmbed", Layer)
+    monkeypatch.setattr(measure, "_pin_gpu", lambda gpu_id: None)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(measure, "make_table", lambda *args, **kwargs: None)
+    monkeypatch.setattr(torch.Tensor, "to", lambda self, device: self)
+    monkeypatch.setattr(measure, "_timed_launches", lambda run, repeats: run() or 1.0)
+    small, large = (np.arange(0, n * 10 + 1, 10, dtype=np.int32) for n in (16384, 163840))
+    monkeypatch.setattr(measure, "load_batches", lambda path: [(small, small), (large, large)])
+    out = str(tmp_path / "t.txt")
+    for size in (0, 32768, 262144):
+        seen.clear()
+        measure.measure_kernel_events("lib", [(1, 1)] * 4, ["float"] * 4, ["x"] * 4, out, size, 0, 1, 1)
+        assert set(seen) == {(16384, min(size, 65536)), (163840, size)}
