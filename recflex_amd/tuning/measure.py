@@ -531,6 +531,7 @@ PLENTY_TILES_PER_WORKGROUP = 2                      # rfx::kPlentyTilesPerWorkgr
 AUTO_TILES_PER_WORKGROUP = 64                       # rfx::kAutoTilesPerWorkgroup
 AUTO_TILE_MIN, AUTO_TILE_MAX = 64 * 1024, 256 * 1024    # rfx::kAutoTileMin / kAutoTileMax
 AUTO_TILE_FLOOR = 4 * 1024                              # rfx::kAutoTileFloor
+_DATA_TYPES = {0: "float", 1: "half", 2: "int8"}         # by the library's numbers
 CAPPED_TILES_PER_WORKGROUP = 5                          # rfx::kCappedTilesPerWorkgroup
 
 
@@ -565,9 +566,11 @@ def launch_tile_bytes(lib, offsets: Sequence[np.ndarray], tile_bytes: int) -> in
     is an upper bound for small batches."""
     if tile_bytes <= AUTO_TILE_MIN:
         return tile_bytes
+    from recflex_amd.code_emitter import MetaData
     from recflex_amd.code_emitter.codegen import BAG_FIXED_BYTES, INDEX_BYTES, LOOKUP_OVERHEAD_BYTES
-    total = batch_traffic(offsets, [b + INDEX_BYTES + LOOKUP_OVERHEAD_BYTES for b in lib.row_strides],
-                          [d * 4 + BAG_FIXED_BYTES for d in lib.embed_dims])
+    metas = [MetaData(d, _DATA_TYPES[t]) for d, t in zip(lib.embed_dims, lib.dtypes)]
+    total = batch_traffic(offsets, [m.row_bytes + INDEX_BYTES + LOOKUP_OVERHEAD_BYTES for m in metas],
+                          [m.embed_dim * 4 + BAG_FIXED_BYTES for m in metas])
     return capped_tile_bytes(tile_bytes, total, lib.get_max_concurrent_blocks())
 
 

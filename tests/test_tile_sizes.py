@@ -152,7 +152,7 @@ def test_the_sweep_times_the_library_that_ships(monkeypatch, tmp_path):
 
     class Layer:
         class lib:
-            row_strides, embed_dims = [512] * 4, [128] * 4
+            embed_dims, dtypes = [128] * 4, [0] * 4
             get_max_concurrent_blocks = staticmethod(lambda: 1280)
 
         def __init__(self, *args, **kwargs):
@@ -178,3 +178,20 @@ def test_the_sweep_times_the_library_that_ships(monkeypatch, tmp_path):
         seen.clear()
         measure.measure_kernel_events("lib", [(1, 1)] * 4, ["float"] * 4, ["x"] * 4, out, size, 0, 1, 1)
         assert set(seen) == {(16384, min(size, 65536)), (163840, size)}
+
+
+def test_launch_tile_bytes_counts_as_the_emitter_does():
+    """Rows without the padding of int8 tables, indices, output rows and offsets."""
+    from recflex_amd import prebuilt
+    from recflex_amd.code_emitter.codegen import BAG_FIXED_BYTES, INDEX_BYTES
+    from recflex_amd.librecom import RecomLib
+    from recflex_amd.tuning import measure
+    for name in ("edge", "c5s"):
+        lib = RecomLib(prebuilt.ensure_built(name))
+        lib.get_max_concurrent_blocks = lambda: 3
+        metas = [s.meta for s, _ in prebuilt.model_spec(name).feat_schedules]
+        off = [np.array([0, 70000 + 13 * f, 99991], np.int64) for f in range(len(metas))]
+        total = measure.batch_traffic(off, [m.row_bytes + INDEX_BYTES for m in metas],
+                                      [m.embed_dim * 4 + BAG_FIXED_BYTES for m in metas])
+        assert 5 * 3 * 65536 < total
+        assert measure.launch_tile_bytes(lib, off, 1 << 30) == measure.capped_tile_bytes(1 << 30, total, 3) < 1 << 30
