@@ -13,7 +13,7 @@ forward-mode derivatives, dispatch and function modes).
 import ctypes
 import subprocess
 import warnings
-from typing import List, Optional
+from typing import List, Optional, Sequence
 
 import torch
 import torch.nn as nn
@@ -32,12 +32,33 @@ except (ImportError, AttributeError):
 MAX_LAYERS = 8                      # RECFLEX_MLP_MAX_LAYERS
 TAIL_MAX_UNITS = 128                # RECFLEX_MLP_TAIL_MAX_UNITS
 TAIL_MAX_INPUTS = 1024              # RECFLEX_MLP_TAIL_MAX_INPUTS
-# Beyond this many rows the layers are library products: the first layer alone keeps the device busy,
-# and the library's kernel for large products reaches 140 TFLOP/s where these reach 105.  MLP of
-# 1024, 256 and 128 units on 4 408 / 23 980 inputs, kernels against library, in us: 256 rows 44 / 140
-# against 86 / 383, 512 rows 65 / 238 against 74 / 250, 700 rows 100 / 398 against 90 / 682, 1 024
-# rows 105 / 517 against 106 / 380.
+# Where the kernels pay, against the modules (in us; both called one after another, and in a graph).
+# The library has switches of its own: up to 256 rows its products take 1.2 to 5 times as long as
+# these, beyond them it is now behind and now ahead.
+#  * Up to 512 rows with layers of up to 1 024 units: 1024, 256, 128 on 4 408 inputs, 256 / 384 / 512
+#    rows 44 / 55 / 64 against 107 (graph 86 / 72 / 74); on 23 980 inputs 138 / 194 / 238 against 383 /
+#    362 / 249.  (1024, 512, 128 on 12 000 inputs is the exception: 450 / 512 rows 136 / 141 against
+#    130 / 130.)
+#  * Wider layers up to 256 rows (8192, 512, 128 on 4 408 inputs, 256 rows: 200 against 238), and beyond
+#    as long as there is little to multiply: these products run at 105 TFLOP/s, the library's large
+#    ones at up to 140, and its launches cost some 40 us.  4 408 inputs, first layer and rows: 2 048
+#    and 352 (7.1 GFLOP) 99 against 109 (graph 95), 2 048 and 416 (8.4) 113 and 110, 4 096 and 512
+#    (21) 198 and 180, 8 192 and 512 (41) 373 and 320; 23 980 inputs, 4 096 and 512 (102) 889 and 717.
+#    (Not without exceptions: 23 980 inputs, 1 536 and 512 rows, 353 against 681.)
+#  * Beyond 512 rows the modules: 1024, 256, 128 on 23 980 inputs, 700 / 1 024 / 2 048 rows 345 / 452 /
+#    888 against 679 / 374 / 713, on 4 408 inputs 91 / 103 / 184 against 109 / 110 / 172.
 MAX_BATCH = 512
+ANY_WIDTH_BATCH = 256
+NARROW_UNITS = 1024
+WIDE_MAX_FLOPS = 8e9
+
+
+def _pays(batch: int, units: Sequence[int]) -> bool:
+    """``units``: of the input and of the hidden layers."""
+    if batch > MAX_BATCH:
+        return False
+    return batch <= ANY_WIDTH_BATCH or max(units[1:]) <= NARROW_UNITS \
+        or 2. * batch * sum(a * b for a, b in zip(units, units[1:])) <= WIDE_MAX_FLOPS
 
 
 class _Args(ctypes.Structure):
@@ -181,7 +202,7 @@ def forward(mlp: nn.Module, x: torch.Tensor) -> Optional[torch.Tensor]:
     if linears is None or _observed():
         return None
     if type(x) is not torch.Tensor or x.dim() != 2 or x.dtype is not torch.float32 or not x.is_cuda \
-            or not x.is_contiguous() or not 0 < x.shape[0] <= MAX_BATCH or x.data_ptr() % 16 \
+            or not x.is_contiguous() or x.shape[0] == 0 or x.data_ptr() % 16 \
             or x.device.index != torch.cuda.current_device():
         return None
     params, fan_in = [], x.shape[1]
@@ -195,6 +216,8 @@ def forward(mlp: nn.Module, x: torch.Tensor) -> Optional[torch.Tensor]:
             return None
         params += [w, b]
         fan_in = w.shape[0]
+    if not _pays(x.shape[0], [x.shape[1]] + [m.weight.shape[0] for m in linears[:-1]]):
+        return None
     if _lib is None and (_missing or not try_load_library()):
         return None
     if linears[-1].weight.shape[1] > TAIL_MAX_UNITS or linears[-2].weight.shape[1] > TAIL_MAX_INPUTS:

@@ -131,3 +131,13 @@ def test_mlp_steps_aside():
     assert kernels.forward(mlp, x[:0]) is None
     mlp[0].bias = None
     assert kernels.forward(mlp, x) is None
+
+
+def test_mlp_leaves_large_products_to_the_library():
+    """Wide layers on many rows, where the library's products are the faster ones."""
+    mlp = build((4096, 4096, 64, 16))
+    x = torch.randn(512, 4096, device="cuda")
+    with torch.no_grad():
+        assert kernels.forward(mlp, x) is None
+        got = kernels.forward(mlp, x[:kernels.ANY_WIDTH_BATCH])
+        assert got is not None and rel(got, mlp.double()(x[:kernels.ANY_WIDTH_BATCH].double())) < REL

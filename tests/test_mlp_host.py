@@ -94,3 +94,13 @@ else:
     assert mlp.forward(None, None) is None
 '''
     subprocess.run([sys.executable, "-c", script], check=True, cwd=ROOT, timeout=120)
+
+
+@pytest.mark.parametrize("batch, units, pays", [
+    (512, (4408, 1024, 256, 128), True), (512, (23980, 1024, 256, 128), True), (513, (64, 32, 16), False),
+    (256, (4408, 8192, 512, 128), True), (257, (4408, 8192, 512, 128), False), (512, (4408, 8192, 128), False),
+    (352, (4408, 2048, 512, 128), True), (416, (4408, 2048, 512, 128), False), (512, (512, 2048, 128), True),
+    # a wide layer behind a narrow one
+    (512, (4408, 512, 4096, 1024, 128), False)])
+def test_where_the_mlp_kernels_pay(batch, units, pays):
+    assert kernels._pays(batch, units) is pays
