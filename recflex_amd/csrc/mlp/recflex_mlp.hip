@@ -37,6 +37,7 @@ __device__ __forceinline__ float relu(const float x) { return x <= 0.f ? 0.f : x
 // rows, one per CU.  Such a CU has two wavefronts per SIMD and nothing else to run while they wait,
 // so the wavefronts split the K of a chunk among them, meet once per chunk, and a chunk is asked for
 // two ahead: it goes to LDS while the matrix cores work on the one before.
+// N and K are multiples of 4 (valid): a vector of four units is whole or beyond N.
 // ---------------------------------------------------------------------------------------------
 constexpr int kTileN = 64, kThreads = 512;
 
@@ -157,15 +158,9 @@ gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *_
     float *dst = out + (static_cast<int64_t>(split) * M + m0 + row) * N + n0 + unit;
     if (bias) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) sum[j] = relu(sum[j] + bias[min(n0 + unit + j, N - 1)]);
+      for (int j = 0; j < 4; ++j) sum[j] = relu(sum[j] + bias[n0 + unit + j]);
     }
-    if (N % 4 == 0) {
-      *reinterpret_cast<f32x4 *>(dst) = sum;
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (n0 + unit + j < N) dst[j] = sum[j];
-    }
+    *reinterpret_cast<f32x4 *>(dst) = sum;
   }
 }
 
