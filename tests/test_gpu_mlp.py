@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 # fp32 sums in blocks of at most 128 terms, blocks and splits added in order: errors of a few eps per
 # layer in the 2-norm
 REL = 1e-6
+GRAD_REL = 1e-5
 
 
 def build(units, device="cuda", seed=0):
@@ -25,6 +26,15 @@ def build(units, device="cuda", seed=0):
 
 def rel(got, want):
     return float((got.double().cpu() - want.double().cpu()).norm() / want.double().cpu().norm())
+
+
+def hidden_of(mlp, x):
+    out = []
+    for m in mlp[:-2]:
+        x = m(x)
+        if isinstance(m, nn.ReLU):
+            out.append(x.detach())
+    return out
 
 
 # edges of the tiles (32 and 64 rows, 64 units), of a chunk of K (128), of the tail (16 rows, 128 units,
@@ -51,16 +61,22 @@ def test_mlp_forward_and_gradients(units, batch):
     assert torch.equal(out.detach(), got)
     weight = torch.linspace(0.5, 1.5, batch, device="cuda")[:, None]
     (out * weight).sum().backward()
-    # against the modules: the gradients of the kernels' path are stock products on the kernels' activations.
-    # A unit within rounding of zero may be on for one and off for the other: fp32 rounding of a few
-    # hundred terms puts one unit in a million there, and one such unit of n is sqrt(1 / n) of a norm.
-    stock = build(units)
-    stock.load_state_dict(mlp.state_dict())
-    xs = x.detach().clone().requires_grad_()
-    (stock(xs) * weight).sum().backward()
-    assert rel(x.grad, xs.grad) < 0.02
-    for a, b in zip(mlp.parameters(), stock.parameters()):
-        assert a.grad.shape == b.grad.shape and rel(a.grad, b.grad) < 0.02
+    # the gradients, in 64 bits from the kernels' own activations (against another path's, a unit within
+    # rounding of zero would be on for one and off for the other): stock fp32 products of up to 1 024
+    # terms, a layer's error handed on to the next, some 1e-7 each
+    ws, bs = [m.weight.detach() for m in mlp[::2]], [m.bias.detach() for m in mlp[::2]]
+    out, hidden = kernels._run(x.detach(), ws, bs, True)
+    acts = [x.detach().double()] + [h.double() for h in hidden]
+    for want_h, got_h in zip(hidden_of(exact, xd.detach()), hidden):
+        assert rel(got_h, want_h) < REL
+    g = weight.double() * out.double() * (1 - out.double())
+    for l in range(len(ws) - 1, -1, -1):
+        assert rel(mlp[2 * l].weight.grad, g.t() @ acts[l]) < GRAD_REL
+        assert rel(mlp[2 * l].bias.grad, g.sum(0)) < GRAD_REL
+        g = g @ ws[l].double()
+        if l:
+            g = g * (acts[l] > 0)
+    assert rel(x.grad, g) < GRAD_REL
 
 
 def test_mlp_repeats_bits_and_passes_nan_on():
