@@ -40,7 +40,8 @@ its library is missing.  Names:
                    ``fewbags_unsplit``: the same with one workgroup per bag, for comparison;
                    ``fewbags64`` / ``fewbags128`` / ``fewbags512``: the same lookups as 64 x 4 000,
                    128 x 2 500 and 512 x 1 000
-``fewbags_even``   8 like features x 16 samples x exactly 20 000 lookups, bound once per launch
+``fewbags_even``   8 like features x 16 samples x exactly 20 000 lookups, bound once per launch;
+                   ``fewbags_mixed``: four features of long bags and four of short ones, likewise
 ``manysplit``      17 fp16 features of dim 256 under the split-bag schedule: 36 MB of workspace,
                    more than the static array of ``recom_process_static_workspace`` may hold
 ``refa``, ``reff4`` models shaped like the reference's example models A and a quarter of F (1 000 and
@@ -287,6 +288,17 @@ def _few_even_bags() -> ModelSpec:
     return ModelSpec(wl, fs, 8, dict(bind_once=True))
 
 
+def _few_mixed_bags() -> ModelSpec:
+    """Four features whose bags may be split and four whose schedules don't, bound once per launch."""
+    feats = tuple(FeatureSpec(5000, d, "float", m, False, 0.0, 1.0)
+                  for d, m in zip((32, 128, 64, 256, 64, 128, 32, 64),
+                                  (20000.0, 3.0, 20000.0, 20000.0, 40.0, 20000.0, 1.0, 200.0)))
+    wl = Workload("fewbags_mixed", 16, 79, feats, "integer")
+    fs = default_feat_schedules(metas_of(wl), [f.mean_bag for f in feats], BLOCK_THREADS)
+    assert sum(isinstance(s, SplitBagSchedule) for s, _ in fs) == 4
+    return ModelSpec(wl, fs, 8, dict(bind_once=True))
+
+
 def _many_split() -> ModelSpec:
     """More split-bag workspace than a library's static device array may hold (32 MiB)."""
     feats = tuple(FeatureSpec(5000 + f, 256, "half", 3000.0, False, 0.0, 1.0) for f in range(17))
@@ -391,6 +403,7 @@ _SPECS: Dict[str, Callable[[], ModelSpec]] = {
     "fewbags64": lambda: _few_bags(True, 64, 4000.0),
     "fewbags128": lambda: _few_bags(True, 128, 2500.0),
     "fewbags_even": _few_even_bags,
+    "fewbags_mixed": _few_mixed_bags,
     "fewbags512": lambda: _few_bags(True, 512, 1000.0),
     "manysplit": _many_split,
     "wide": _wide,

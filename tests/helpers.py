@@ -1,7 +1,9 @@
 """Shared pieces of the parity tests: run a prebuilt model through the C ABI on the GPU and
 compare with the CPU oracle."""
 
+import ctypes
 import os
+import subprocess
 import sys
 
 import numpy as np
@@ -45,3 +47,30 @@ def check_against_oracle(wl, got: np.ndarray, want: np.ndarray):
             failures.append((f, spec, max_abs, max_rel))
         col += spec.dim
     return failures
+
+
+PART_COST = 35 * 1024           # rfx::kSplitPartCost
+
+
+def build_tile_model(lib: str) -> ctypes.CDLL:
+    """``tests/cpu/tile_sizes_model.cpp`` built as ``lib``: the binding's tile sizes on the CPU."""
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-shared", "-fPIC", "-ffp-contract=off",
+                    f"-I{ROOT}/recflex_amd/csrc/include", os.path.join(ROOT, "tests", "cpu", "tile_sizes_model.cpp"),
+                    "-o", lib], check=True)
+    return ctypes.CDLL(lib)
+
+
+def bind_tiles_on_cpu(model, cost, gran, batch, grid, tile_size) -> dict:
+    """Part size, tiles per feature and the price of a round-by-round walk over them, as the binding
+    chooses them and as its plain rule would (``rule``, ``rule_price``); ``counted``: the tiles the
+    search counted, -1 where it was not due."""
+    n = len(cost)
+    cost, gran = np.asarray(cost, np.float32), np.asarray(gran, np.int32)
+    tiles, rule_tiles, out = np.zeros(n, np.int32), np.zeros(n, np.int32), np.zeros(3, np.int64)
+    longest, rule_longest = np.zeros(1, np.float32), np.zeros(1, np.float32)
+    ptr = [a.ctypes.data_as(ctypes.c_void_p) for a in (cost, gran, tiles, longest, rule_tiles, rule_longest, out)]
+    model.model_bind(n, batch, grid, tile_size, *ptr)
+    price = [-(-int(t.sum()) // grid) * (float(l[0]) + PART_COST)
+             for t, l in ((tiles, longest), (rule_tiles, rule_longest))]
+    return dict(unit=int(out[0]), counted=int(out[1]), rule=int(out[2]), tiles=tiles, price=price[0],
+                rule_price=price[1])

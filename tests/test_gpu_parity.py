@@ -1,10 +1,12 @@
 """GPU parity: the HIP fused kernel, called through the C ABI of a prebuilt librecom.so, against
 the CPU oracle on identical seeded inputs."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
-from helpers import check_against_oracle, oracle_output, require_lib
+from helpers import bind_tiles_on_cpu, build_tile_model, check_against_oracle, oracle_output, require_lib
 
 pytestmark = pytest.mark.gpu
 
@@ -707,40 +709,63 @@ def test_smaller_tiles_of_small_batches_change_no_bit(batch):
         assert torch.equal(layer.forward_indices(bound, tile_bytes=tile_bytes), got)
 
 
-@pytest.mark.parametrize("bags, mean, grid", [(16, 4000, 64), (150, 300, 40), (3, 9000, 7), (48, 900, 0),
-                                              (1, 30000, 3), (2049, 40, 12), (33, 2000, 16)])
-def test_part_sizes_that_fill_rounds_of_the_grid(bags, mean, grid):
-    """Models of up to 16 features choose the part size whose tiles fill whole rounds of the grid,
-    where a workgroup's share of the batch is beyond 256 KiB: small grids bring small batches there.
-    Bags of unequal length, empty ones among them; integer-valued tables, so any split gives the same
-    bits; two launches, since the arrival counters must be back at zero."""
-    import torch
-    from recflex_amd import prebuilt
-    from recflex_amd.rec_modules import FeatEmbed
-    from recflex_amd.workloads import gen_inputs, gen_tables
-    wl = prebuilt.model_spec("fewbags").workload
-    wl = wl._replace(batch=bags, table_values="integer", features=tuple(
-        f._replace(rows=5000, mean_bag=float(mean), len_sigma=0.7 if k % 2 else 0.0, empty_frac=0.1)
-        for k, f in enumerate(wl.features)))
-    print("[case] fewbags", bags, mean, grid, flush=True)
-    dev = torch.device("cuda", 0)
-    tables = gen_tables(wl, dev)
-    indices, offsets = gen_inputs(wl)
-    layer = FeatEmbed(dev, embed_tables=tables, librecom=require_lib("fewbags"))
-    bound = layer.bind_inputs([torch.from_numpy(i).to(dev) for i in indices],
-                              [torch.from_numpy(o).to(dev) for o in offsets])
-    want = oracle_output(wl, [t.cpu().numpy() for t in tables], indices, offsets)
-    for _ in range(2):
-        got = layer.forward_indices(bound, grid_blocks=grid).cpu().numpy()
-        assert np.array_equal(got, want)
-
-
 def _bound_tiles(layer):
     """Tiles per feature of the last launch of a library that is bound once per launch: the binding
     kernel's table (prefix[F + 1], bags_per_tile[F], cand[F]) ends the workspace."""
     n = layer.lib.num_features
     table = layer.workspace.cpu().numpy()[-(3 * n + 1):]
     return np.diff(table[:n + 1])
+
+
+@pytest.fixture(scope="module")
+def tile_model(tmp_path_factory):
+    return build_tile_model(str(tmp_path_factory.mktemp("tile_sizes") / "model.so"))
+
+
+@pytest.mark.parametrize("name", ["fewbags", "fewbags_even", "fewbags_mixed"])
+@pytest.mark.parametrize("bags, mean, share", [(16, 4000, 540), (150, 300, 410), (3, 9000, 720), (48, 900, 300),
+                                               (1, 30000, 620), (2049, 40, 350), (33, 2000, 870), (700, 110, 500)])
+def test_part_sizes_that_fill_rounds_of_the_grid(tile_model, name, bags, mean, share):
+    """Models of up to 16 features choose the part size by the rounds of the grid that its tiles take,
+    where a workgroup's share of the batch is between 256 KiB and 1 MiB (``share``, in KiB, gives
+    the grid).  Bags of unequal length, empty ones among them, beside features whose schedules
+    don't split; one bag, more bags than any may be split of.  Integer-valued tables, so any split
+    gives the same bits; two launches, since the arrival counters must be back at zero.  Where the
+    binding leaves its table in the workspace, the tiles are those that the CPU counts with the
+    device's own arithmetic (a correctly rounded reciprocal where the device's is one unit off
+    moves no bag of these inputs over an edge)."""
+    import torch
+    from recflex_amd import prebuilt
+    from recflex_amd.code_emitter.codegen import BAG_FIXED_BYTES, INDEX_BYTES
+    from recflex_amd.rec_modules import FeatEmbed
+    from recflex_amd.workloads import gen_inputs, gen_tables
+    spec = prebuilt.model_spec(name)
+    wl = spec.workload
+    wl = wl._replace(batch=bags, table_values="integer", features=tuple(
+        f._replace(rows=5000, mean_bag=float(mean) if f.mean_bag > 1000 else f.mean_bag, fixed_len=False,
+                   len_sigma=0.7 if k % 2 else 0.0, empty_frac=0.1) for k, f in enumerate(wl.features)))
+    print("[case]", name, bags, mean, share, flush=True)
+    dev = torch.device("cuda", 0)
+    tables = gen_tables(wl, dev)
+    indices, offsets = gen_inputs(wl)
+    layer = FeatEmbed(dev, embed_tables=tables, librecom=require_lib(name))
+    bound = layer.bind_inputs([torch.from_numpy(i).to(dev) for i in indices],
+                              [torch.from_numpy(o).to(dev) for o in offsets])
+    metas = [s.meta for s, _ in spec.feat_schedules]
+    cost = [int(o[-1]) * (m.row_bytes + INDEX_BYTES) + bags * (m.embed_dim * 4 + BAG_FIXED_BYTES)
+            for o, m in zip(offsets, metas)]
+    grid = max(1, sum(cost) // (share * 1024))
+    assert 256 * 1024 < sum(cost) / grid < 1024 * 1024
+    tile_size = tile_model.model_auto_tile_size(ctypes.c_longlong(sum(cost)), grid)
+    expect = bind_tiles_on_cpu(tile_model, cost, [s.TileGranularity(p) for s, p in spec.feat_schedules], bags, grid,
+                               tile_size)
+    assert expect["counted"] >= 0               # the part size was searched
+    want = oracle_output(wl, [t.cpu().numpy() for t in tables], indices, offsets)
+    for _ in range(2):
+        got = layer.forward_indices(bound, grid_blocks=grid).cpu().numpy()
+        assert np.array_equal(got, want)
+        if spec.emit_kwargs.get("bind_once"):
+            assert _bound_tiles(layer).tolist() == expect["tiles"].tolist()
 
 
 def test_bags_of_one_cost_fill_one_round_of_the_grid():

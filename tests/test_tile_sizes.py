@@ -3,38 +3,16 @@ is counted with is what the batch is cut into, models of equal features fill the
 grid, and no size is chosen that is dearer, by the same count, than the plain rule's."""
 
 import ctypes
-import os
-import subprocess
 
 import numpy as np
 import pytest
 
-from helpers import ROOT
-
-PART_COST = 35 * 1024           # rfx::kSplitPartCost
-MIN_UNIT = 256 * 1024           # rfx::kSplitMinUnit
+from helpers import PART_COST, bind_tiles_on_cpu, build_tile_model
 
 
 @pytest.fixture(scope="module")
 def model(tmp_path_factory):
-    lib = str(tmp_path_factory.mktemp("tile_sizes") / "model.so")
-    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-shared", "-fPIC", "-ffp-contract=off",
-                    f"-I{ROOT}/recflex_amd/csrc/include", os.path.join(ROOT, "tests", "cpu", "tile_sizes_model.cpp"),
-                    "-o", lib], check=True)
-    return ctypes.CDLL(lib)
-
-
-def bind(model, cost, gran, batch, grid, tile_size):
-    n = len(cost)
-    cost, gran = np.asarray(cost, np.float32), np.asarray(gran, np.int32)
-    tiles, rule_tiles, out = np.zeros(n, np.int32), np.zeros(n, np.int32), np.zeros(3, np.int64)
-    longest, rule_longest = np.zeros(1, np.float32), np.zeros(1, np.float32)
-    ptr = [a.ctypes.data_as(ctypes.c_void_p) for a in (cost, gran, tiles, longest, rule_tiles, rule_longest, out)]
-    model.model_bind(n, batch, grid, tile_size, *ptr)
-    price = [-(-int(t.sum()) // grid) * (float(l[0]) + PART_COST)
-             for t, l in ((tiles, longest), (rule_tiles, rule_longest))]
-    return dict(unit=int(out[0]), counted=int(out[1]), rule=int(out[2]), tiles=tiles, price=price[0],
-                rule_price=price[1])
+    return build_tile_model(str(tmp_path_factory.mktemp("tile_sizes") / "model.so"))
 
 
 def split_cost(batch, lookups, dim):
@@ -49,7 +27,7 @@ def split_cost(batch, lookups, dim):
 def test_equal_features_fill_their_rounds(model, features, dim, batch, lookups, grid):
     """Bags of one cost: the parts of a round are at most ``grid // bags`` per bag, and no size leaves
     a round that a share of the batch in that many rounds would fill."""
-    got = bind(model, [split_cost(batch, lookups, dim)] * features, [-1] * features, batch, grid, 65536)
+    got = bind_tiles_on_cpu(model, [split_cost(batch, lookups, dim)] * features, [-1] * features, batch, grid, 65536)
     if got["counted"] < 0:
         assert got["unit"] == got["rule"]
         return
@@ -75,7 +53,7 @@ def test_random_models_count_what_they_bind_and_never_lose(model):
         weight = rng.random(n) + 0.05 if rng.random() < 0.7 else np.ones(n)
         cost = share * grid * weight / weight.sum()
         gran = np.where(rng.random(n) < 0.75, -1, rng.choice([1, 4, 16, 64], n))
-        got = bind(model, cost, gran, batch, grid, tile_size)
+        got = bind_tiles_on_cpu(model, cost, gran, batch, grid, tile_size)
         case = (n, grid, batch, tile_size, cost.tolist(), gran.tolist(), got)
         if got["counted"] < 0:
             assert got["unit"] == got["rule"], case
@@ -91,7 +69,7 @@ def test_bags_just_below_the_split_limit_do_not_cost_rounds(model):
     """878 bags of a quarter of a megabyte in eight features: left whole in four rounds of 527 KB by a
     search that does not price the plain rule, five rounds of 263 KB by the rule."""
     for mean in range(1000, 2200, 50):
-        got = bind(model, [split_cost(878, mean, 64)] * 8, [-1] * 8, 878, 2048, 65536)
+        got = bind_tiles_on_cpu(model, [split_cost(878, mean, 64)] * 8, [-1] * 8, 878, 2048, 65536)
         assert got["price"] <= got["rule_price"] * (1 + 1e-6)
 
 
