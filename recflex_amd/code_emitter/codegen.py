@@ -581,9 +581,12 @@ extern "C" __global__ void __launch_bounds__(rfx::kFindThreads) OutlierKnl(
   // of the binding.
   const rfx::TailDraw d_tickets{{d_outliers, xcd}};
   __shared__ int s_ticket[2];
-  // A workgroup's first tile is dealt in any case: it is there without a draw, and a batch of one
-  // pass or less draws nothing (every workgroup asking for a ticket to learn that there are no
-  // tiles left: 1 000 features, one sample 13.1 us, 37 samples 28.4; without 9.2 and 20.8 us).
+  // Where only the last passes are drawn, a workgroup's first tile is dealt in any case: it is there
+  // without a draw, and a batch of one pass or less draws nothing (every workgroup asking for a
+  // ticket to learn that there are no tiles left: 1 000 features, one sample 13.1 us, 37 samples
+  // 28.4; without 9.2 and 20.8 us).  Where every tile is drawn, every workgroup draws, for one
+  // sample too, and its first ticket, asked for above, counts towards the counter's last one: it
+  // has to come to the ticket's loop below whatever the batch holds.
   const int static_last = DRAWN_TAIL >= RFX_DRAWN_ALL ? 0 :
       static_cast<int>(max(static_cast<long long>(min(walk_last, walk_step)),
                            walk_last - static_cast<long long>(DRAWN_TAIL) * walk_step));
@@ -596,7 +599,7 @@ extern "C" __global__ void __launch_bounds__(rfx::kFindThreads) OutlierKnl(
         at = walk;
         walk += walk_step;
       }} else {{
-        if (static_last >= walk_last) break;
+        if (DRAWN_TAIL < RFX_DRAWN_ALL && static_last >= walk_last) break;
         drawing = true;
         if (threadIdx.x == 0)
           s_ticket[0] = DRAWN_TAIL >= RFX_DRAWN_ALL ? first_ticket : rfx::draw_tail_ticket(d_tickets, xcd);

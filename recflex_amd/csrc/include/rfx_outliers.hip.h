@@ -227,7 +227,8 @@ template <typename Space> __device__ __forceinline__ void no_outliers(Space *sp)
 // N + W - 1 knows that nobody draws any more.  (A counter of finished workgroups told the same
 // before: one device-scope add per workgroup to a single address, 11 ns each one after the
 // other, 14 us for 1 280 workgroups -- most of a small batch's kernel: 100 features, 8 samples
-// 22.7 us with it, 11.1 us without; 2 048 samples 126.0 and 123.2 us.)
+// 22.7 us with it, 11.1 us without.  A full batch does not show it: its workgroups end at different
+// times, 2 048 samples 121.9 and 121.3 us.)
 // ---------------------------------------------------------------------------------------------
 struct TailTickets {
   int next[8][32];                           // per XCD, each on a cache line of its own
