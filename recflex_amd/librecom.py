@@ -187,7 +187,7 @@ class RecomLib:
                 times: int = 0, stream: int = 0, output_row_stride: int = 0,
                 workspace: int = 0, workspace_bytes: int = 0,
                 static_workspace: bool = False, start_event: int = 0, stop_event: int = 0,
-                lookup_counts: int = 0) -> None:
+                lookup_counts: int = 0, _ints: bool = False) -> None:
         """All pointer arguments are raw device addresses (``tensor.data_ptr()``).  Without a
         ``workspace``, a library that needs one uses ``default_workspace()``.
         ``start_event`` / ``stop_event``: ``hipEvent_t`` handles that receive the begin and end of
@@ -195,7 +195,8 @@ class RecomLib:
         ``lookup_counts``: device int32[F], the lookups of each feature in this batch as far as
         the caller knows (a hint that spares the binding a scattered read per feature).
         ``static_workspace=True`` calls ``recom_process_static_workspace`` instead: no workspace
-        is passed or allocated, the library uses its own static device array."""
+        is passed or allocated, the library uses its own static device array.
+        ``_ints``: the caller vouches that every address is an ``int``."""
         if static_workspace:
             args = RecomProcessArgs(table_ptrs or None, io_ptrs or None, arg_buffers or None,
                                     arg_buffer_offsets or None, output or None, batch, tile_bytes,
@@ -215,7 +216,7 @@ class RecomLib:
         packed = None
         # (struct takes anything with an __index__, a one-element tensor in place of its address
         # among them; ctypes wants an address to be an int)
-        if {type(table_ptrs), type(io_ptrs), type(arg_buffers), type(arg_buffer_offsets), type(output),
+        if _ints or {type(table_ptrs), type(io_ptrs), type(arg_buffers), type(arg_buffer_offsets), type(output),
                 type(schedule_choice), type(times), type(stream), type(workspace), type(start_event),
                 type(stop_event), type(lookup_counts)} == _ADDRESS_TYPES:
             try:

@@ -58,10 +58,13 @@ def _resolve_lib(librecom: Union[None, str, RecomLib]) -> RecomLib:
     return _current_lib
 
 
-def _stream_of(device: torch.device) -> int:
-    if _RAW_STREAM is None:
+if _RAW_STREAM is not None:
+    def _stream_of(device: torch.device) -> int:
+        index = device.index
+        return _RAW_STREAM(torch.cuda.current_device() if index is None else index)
+else:
+    def _stream_of(device: torch.device) -> int:
         return torch.cuda.current_stream(device).cuda_stream
-    return _RAW_STREAM(torch.cuda.current_device() if device.index is None else device.index)
 
 
 class FeatPreprocess(nn.Module):
@@ -211,6 +214,8 @@ class FeatEmbed(nn.Module):
         stream = _stream_of(self.device)
         if kernel_events is not None:
             inputs.update(start_event=kernel_events[0].handle, stop_event=kernel_events[1].handle)
+        elif type(self.lib) is RecomLib:
+            inputs["_ints"] = True              # every address comes from data_ptr()
         if self.workspace is not None:
             inputs.update(workspace=self.workspace.data_ptr(),
                           workspace_bytes=self.workspace.numel() * 4)
