@@ -4,10 +4,10 @@ eight of the same ``nn.Sequential`` run layer by layer.
 
 ``forward(mlp, x)`` returns ``None`` where the kernels don't apply, and the caller then runs the
 modules: other layers than ``RecomModel`` builds, hooks on any of them, parameters that are not
-plain fp32 tensors on the current device, sizes outside the kernels' range, no library and no
-compiler to build it, and whatever wants to
-see the single operations (autocast, tracing, compiling, vmap and the other function transforms,
-forward-mode derivatives, dispatch and function modes).
+plain fp32 tensors on the current device, sizes outside the kernels' range or where the modules
+are the faster ones, no library and no compiler to build it, and whatever wants to see the single
+operations (autocast, tracing, compiling, vmap and the other function transforms, forward-mode
+derivatives, dispatch and function modes).
 """
 
 import ctypes
