@@ -201,11 +201,13 @@ def forward(mlp: nn.Module, x: torch.Tensor) -> Optional[torch.Tensor]:
     linears = _linears(mlp)
     if linears is None or _observed():
         return None
-    if type(x) is not torch.Tensor or x.dim() != 2 or x.dtype is not torch.float32 or not x.is_cuda \
-            or not x.is_contiguous() or x.shape[0] == 0 or x.data_ptr() % 16 \
-            or x.device.index != torch.cuda.current_device():
+    if type(x) is not torch.Tensor or x.dim() != 2:
         return None
-    params, fan_in = [], x.shape[1]
+    batch, fan_in = x.shape
+    if not 0 < batch <= MAX_BATCH or x.dtype is not torch.float32 or not x.is_cuda or not x.is_contiguous() \
+            or x.data_ptr() % 16 or x.device.index != torch.cuda.current_device():
+        return None
+    params, units = [], [fan_in]
     hidden = len(linears) - 1
     if hidden > MAX_LAYERS or linears[-1].weight.shape[0] != 1:
         return None
@@ -216,11 +218,10 @@ def forward(mlp: nn.Module, x: torch.Tensor) -> Optional[torch.Tensor]:
             return None
         params += [w, b]
         fan_in = w.shape[0]
-    if not _pays(x.shape[0], [x.shape[1]] + [m.weight.shape[0] for m in linears[:-1]]):
+        units.append(fan_in)
+    if units[-2] > TAIL_MAX_UNITS or units[-3] > TAIL_MAX_INPUTS or not _pays(batch, units[:-1]):
         return None
     if _lib is None and (_missing or not try_load_library()):
-        return None
-    if linears[-1].weight.shape[1] > TAIL_MAX_UNITS or linears[-2].weight.shape[1] > TAIL_MAX_INPUTS:
         return None
     if torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in params)):
         return _Mlp.apply(x, *params)[0]
