@@ -65,9 +65,55 @@ template <int VB> __device__ __forceinline__ Vec<VB> load_vec(const char *__rest
   return r;
 }
 
-// scale (x) and bias (y) of an I8 row, stored as two fp16 right after the codes
-template <int D> __device__ __forceinline__ f32x2 load_scale_bias(const char *__restrict__ row) {
-  return unpack_half2(*reinterpret_cast<const uint32_t *>(row + D));
+// r * STRIDE in 32 bits (modulo 2^32) without the multiplication at quarter rate where shifts do
+template <int STRIDE> __device__ __forceinline__ int row_offset(const int r) {
+  constexpr int LOW = STRIDE & -STRIDE, ODD = STRIDE / LOW;
+  if constexpr (ODD == 3 || ODD == 5 || ODD == 9) {
+    int t;
+    asm("v_lshl_add_u32 %0, %1, %2, %1" : "=v"(t) : "v"(r), "n"(ODD == 3 ? 1 : (ODD == 5 ? 2 : 3)));
+    return static_cast<int>(static_cast<unsigned>(t) * LOW);
+  } else {
+    return static_cast<int>(static_cast<unsigned>(r) * STRIDE);
+  }
+}
+
+// A window of a table as a buffer resource: rows are loaded by 32-bit byte offsets, one register where a
+// 64-bit address takes two and several instructions, and a lane without a lookup passes row -1, which
+// lies beyond the window: it reads zeros and touches no memory.  Window w starts at row w * ROWS (a
+// table of less than 4 GB has one).
+template <typename R> struct RowWindow {
+  static constexpr unsigned SLACK = R::STRIDE > 4096 ? R::STRIDE : 4096;
+  static constexpr int ROWS = static_cast<int>((0x100000000ull - SLACK) / R::STRIDE);
+  __amdgpu_buffer_rsrc_t rsrc;
+
+  __device__ __forceinline__ RowWindow(const char *table, const int w)
+      : rsrc(__builtin_amdgcn_make_buffer_rsrc(
+            const_cast<char *>(table) + static_cast<int64_t>(w) * ROWS * R::STRIDE, 0,
+            static_cast<int>(static_cast<unsigned>(ROWS) * R::STRIDE), 0x00020000)) {}
+  // row r of the table as a row of window w (-1: not in it)
+  static __device__ __forceinline__ int local(const int r, const int w) {
+    const int l = r - w * ROWS;
+    return r >= 0 && l >= 0 && l < ROWS ? l : -1;
+  }
+  template <int VB> __device__ __forceinline__ Vec<VB> load(const int at, const int plus) const {
+    Vec<VB> r;
+    if constexpr (VB == 16) {
+      const u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(rsrc, at + plus, 0, 0);
+      r.w[0] = t.x; r.w[1] = t.y; r.w[2] = t.z; r.w[3] = t.w;
+    } else if constexpr (VB == 8) {
+      const u32x2 t = __builtin_amdgcn_raw_buffer_load_b64(rsrc, at + plus, 0, 0);
+      r.w[0] = t.x; r.w[1] = t.y;
+    } else {
+      r.w[0] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, at + plus, 0, 0);
+    }
+    return r;
+  }
+};
+
+// scale (low half) and bias (high half) of an I8 row, stored as two fp16 right after the codes: taken
+// apart where they are used, so that a row's loads do not wait for them
+template <int D> __device__ __forceinline__ uint32_t load_scale_bias(const char *__restrict__ row) {
+  return *reinterpret_cast<const uint32_t *>(row + D);
 }
 
 // acc[0..EPV) += decode(v).  For I8 only code*scale is added here; the bias is summed once per
@@ -83,6 +129,20 @@ template <int HI> __device__ __forceinline__ float add_half(float acc, uint32_t 
   else
     asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(acc) : "v"(w));
   return acc;
+}
+
+// acc + (the fp16 value in the low or high half of w) * s, rounded once
+template <int HI> __device__ __forceinline__ float fma_half(const uint32_t w, const float s, float acc) {
+  if constexpr (HI == 0)
+    asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel_hi:[1,0,0]" : "+v"(acc) : "v"(w), "v"(s));
+  else
+    asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(acc) : "v"(w), "v"(s));
+  return acc;
+}
+
+// what accumulate multiplies the codes of an I8 row by: its scale, for codes that are read as halves
+__device__ __forceinline__ float code_scale(const uint32_t scale_bias) {
+  return unpack_half2(scale_bias).x * 16777216.f;
 }
 
 template <int DT, int VB>
@@ -105,13 +165,16 @@ __device__ __forceinline__ void accumulate(float *acc, const Vec<VB> &v, float s
 #endif
     }
   } else {
+    // A code in the low bits of a half is the subnormal code * 2^-24, which v_fma_mix_f32 takes as it
+    // is: two instructions bring the four codes of a dword into place, where a conversion of each
+    // takes four at half rate.  Same products, same rounding.
 #pragma unroll
     for (int i = 0; i < VB / 4; ++i) {
-      const uint32_t w = v.w[i];
-      acc[4 * i + 0] = fmaf(static_cast<float>(w & 0xffu), scale, acc[4 * i + 0]);
-      acc[4 * i + 1] = fmaf(static_cast<float>((w >> 8) & 0xffu), scale, acc[4 * i + 1]);
-      acc[4 * i + 2] = fmaf(static_cast<float>((w >> 16) & 0xffu), scale, acc[4 * i + 2]);
-      acc[4 * i + 3] = fmaf(static_cast<float>(w >> 24), scale, acc[4 * i + 3]);
+      const uint32_t even = v.w[i] & 0x00ff00ffu, odd = __builtin_amdgcn_perm(0u, v.w[i], 0x0c030c01u);
+      acc[4 * i + 0] = fma_half<0>(even, scale, acc[4 * i + 0]);
+      acc[4 * i + 1] = fma_half<0>(odd, scale, acc[4 * i + 1]);
+      acc[4 * i + 2] = fma_half<1>(even, scale, acc[4 * i + 2]);
+      acc[4 * i + 3] = fma_half<1>(odd, scale, acc[4 * i + 3]);
     }
   }
 }

@@ -134,6 +134,159 @@ __device__ __forceinline__ void mid_queue_walk_done(MidBagQueue *q) {
 
 __device__ __forceinline__ bool mid_queue_open(MidBagQueue *q) { return mid_queue_open<LdsMem>(q); }
 
+// The value that lane j of every group of X consecutive lanes holds, in all lanes of the group (X a
+// power of two, j the same in all lanes).
+template <int X> __device__ __forceinline__ int group_lane(const int v, const int j, const int lane) {
+  if constexpr (X == 1) {
+    return v;
+  } else if constexpr (X == 64) {
+    return __builtin_amdgcn_readlane(v, j);
+  } else {
+    return __builtin_amdgcn_ds_bpermute(((lane & (63 & ~(X - 1))) + j) << 2, v);
+  }
+}
+
+// Largest v (>= 0) over the wavefront, as a scalar.
+__device__ __forceinline__ int wave_max(int v) {
+  v = max(v, dpp_or_zero<0x111, 0xf>(v));
+  v = max(v, dpp_or_zero<0x112, 0xf>(v));
+  v = max(v, dpp_or_zero<0x114, 0xf>(v));
+  v = max(v, dpp_or_zero<0x118, 0xf>(v));
+  v = max(v, dpp_or_zero<0x142, 0xa>(v));
+  v = max(v, dpp_or_zero<0x143, 0xc>(v));
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
+// How many windows of the table (RowWindow) the rows that a wavefront holds lie in, the same in every lane.
+template <typename R> __device__ __forceinline__ int windows_of(const int row) {
+  if (__builtin_amdgcn_ballot_w64(row >= RowWindow<R>::ROWS) == 0) return 1;
+  return wave_max(row >= 0 ? row / RowWindow<R>::ROWS : 0) + 1;
+}
+
+// ---------------------------------------------------------------------------------------------
+// sum_lookups: the lookups [beg[i], end[i]) of UB bags per team of X*Y lanes, added onto acc (and, for
+// int8 rows, the biases onto bias_acc), row vectors v0 .. v0 + VPP - 1 of every lane.  Called by a whole
+// wavefront; len_most is the longest of its bags, the same in every lane.
+//
+// What bounds it: with every table in the L1 (30 rows each) the 200-feature int8 batch took 1 220 us of its
+// 1 566, the 400-feature fp16 batch 3 315 of 4 120 and the 100-feature fp32 batch 66 of 121.  The rows'
+// way through the vector L1 (64 bytes a clock, in order) and the instructions around it are the larger
+// part, not the memory behind.  So the loop spends as little as it can on a lookup besides its row:
+//  * The indices come in chunks, one lane per lookup of the team, and are handed to the lookup's X lanes
+//    across the wavefront: one load per T lookups where every lane asked for every index by itself (on
+//    the 100 features 1.55 M vector loads instead of 2.42 M).
+//  * A row is addressed by one 32-bit offset into a window of its table (RowWindow), and a lane without
+//    a lookup reads zeros from beyond it: a round is straight-line code whether its bags are full,
+//    partial or empty, the loop's control is scalar, and there is one copy of the body.  (Rounds with a
+//    branch around each load and each add, for int8 rows with a wait for the row's scale in each of
+//    them, were most of the rounds of teams that share a wavefront.)
+//  * Codes of int8 rows are multiplied as they lie (accumulate).
+// Measured, same bits: 200 int8 features (16 384 samples) 1 560 -> 1 405 us, 400 fp16 (8 192) 4 115 -> 4 015,
+// 100 fp32 features (tuned, 2 048) 121.4 -> 118.9, (default schedules, 1 337) 94.0 -> 90.1, 2 500 (256)
+// 178.3 -> 175.9.  The registers go from 96 and 4 spilled to 74, from 109 to 79 and from 96 to 82: room for
+// more workgroups on a CU, or more rows in flight.
+// ---------------------------------------------------------------------------------------------
+template <int DT, int D, int X, int Y, int U, int UB, int VPP, int EPV>
+__device__ __forceinline__ void
+sum_lookups(float (&acc)[UB][VPP][EPV], float (&bias_acc)[UB], const char *__restrict__ table,
+            const int *__restrict__ indices, const int (&beg)[UB], const int (&end)[UB], const int len_most,
+            const int v0, const int x, const int y, const int lane) {
+  using R = Row<DT, D>;
+  // The lanes that share an index fetch: the X lanes of a lookup where a round (U of them) and a chunk are
+  // multiples of one another, each lane for itself otherwise.
+  constexpr int G = X % U == 0 || U % X == 0 ? X : 1;
+  constexpr int NC = U > G ? U / G : 1;         // chunks of G*Y indices a round takes
+  constexpr int VB = R::VB;
+  static_assert(EPV == R::EPV, "one accumulator per column of a lane's vector");
+  constexpr int VPL = ceil_div(R::V, X);
+  // every lane has a vector of the row in every pass over it
+  constexpr bool WHOLE = R::V % X == 0;
+
+  // The bag's next lookups: chunk c, lane (g, y) holds position (c*G + g)*Y + y (negative: beyond the bag).
+  int held[UB][NC], coming[UB][NC];
+  const int g = G == X ? x : 0;
+  auto fetch = [&](int (&to)[UB][NC], const int from) {
+#pragma unroll
+    for (int i = 0; i < UB; ++i)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int p = beg[i] + from + (c * G + g) * Y + y;
+        to[i][c] = -1;
+        if (p < end[i]) to[i][c] = indices[p];
+      }
+  };
+  fetch(held, 0);
+  int at = 0;                 // the chunk's next lookup of every lookup lane (G > U: several rounds)
+  int windows = 1;            // of the table, that this chunk's rows lie in
+
+  for (int base = 0; base < len_most; base += U * Y) {
+    const bool chunk_begins = G <= U || at == 0;
+    if (chunk_begins) {
+      windows = 1;
+#pragma unroll
+      for (int i = 0; i < UB; ++i)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          // (here and not as it is fetched: the rows in flight would wait for it)
+          held[i][c] = max(held[i][c], -1);
+          windows = max(windows, windows_of<R>(held[i][c]));
+        }
+    }
+    int idx[UB][U];
+#pragma unroll
+    for (int i = 0; i < UB; ++i)
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        idx[i][u] = group_lane<G>(held[i][u / G], (G > U ? at : 0) + u % G, lane);
+    if constexpr (G > U) at = at + U == G ? 0 : at + U;
+
+    int w = 0;
+    do {
+      const RowWindow<R> window(table, w);
+      Vec<VB> buf[UB][U][VPP];
+      uint32_t sb[UB][U];
+#pragma unroll
+      for (int i = 0; i < UB; ++i)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          int r = idx[i][u];
+          if (__builtin_expect(windows > 1, 0)) {
+            r = window.local(r, w);
+            asm volatile("" : "+v"(r));         // (keeps it a branch: nearly every table has one window)
+          }
+          const int row = row_offset<R::STRIDE>(r);
+#pragma unroll
+          for (int v = 0; v < VPP; ++v) {
+            const int c = x + (v0 + v) * X;
+            if (v0 + v < VPL && (WHOLE || c < R::V))
+              buf[i][u][v] = window.template load<VB>(row + x * VB, (v0 + v) * X * VB);
+          }
+          if constexpr (DT == I8) sb[i][u] = window.template load<4>(row, D).w[0];
+        }
+      // the next chunk, behind the first rows of this one
+      if (chunk_begins && w == 0) fetch(coming, base + NC * G * Y);
+#pragma unroll
+      for (int i = 0; i < UB; ++i)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const float scale = DT == I8 ? code_scale(sb[i][u]) : 1.f;
+#pragma unroll
+          for (int v = 0; v < VPP; ++v) {
+            const int c = x + (v0 + v) * X;
+            if (v0 + v < VPL && (WHOLE || c < R::V)) accumulate<DT, VB>(acc[i][v], buf[i][u][v], scale);
+          }
+          if constexpr (DT == I8) bias_acc[i] = add_half<1>(bias_acc[i], sb[i][u]);
+        }
+    } while (__builtin_expect(++w < windows, 0));
+    if (G <= U || at == 0) {
+#pragma unroll
+      for (int i = 0; i < UB; ++i)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) held[i][c] = coming[i][c];
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------------------------
 // wave_bag: one bag summed by a whole wavefront, whatever the feature's schedule -- the way out
 // for a bag far longer than its feature's schedule was chosen for.  A team of T lanes with U
@@ -187,7 +340,7 @@ wave_bag(const char *__restrict__ table, const int *__restrict__ indices, const 
   }
   for (int base = beg; base < end; base += UW * YW) {
     Vec<VB> buf[UW][VPL];
-    f32x2 sb[UW];
+    uint32_t sb[UW];
 #pragma unroll
     for (int u = 0; u < UW; ++u)
       if (idx[u] >= 0) {
@@ -211,9 +364,9 @@ wave_bag(const char *__restrict__ table, const int *__restrict__ indices, const 
 #pragma unroll
         for (int v = 0; v < VPL; ++v) {
           const int c = x + v * XW;
-          if (c < R::V) accumulate<DT, VB>(acc[v], buf[u][v], DT == I8 ? sb[u].x : 1.f);
+          if (c < R::V) accumulate<DT, VB>(acc[v], buf[u][v], DT == I8 ? code_scale(sb[u]) : 1.f);
         }
-        if constexpr (DT == I8) bias_acc += sb[u].y;
+        if constexpr (DT == I8) bias_acc = add_half<1>(bias_acc, sb[u]);
       }
 #pragma unroll
     for (int u = 0; u < UW; ++u) idx[u] = nidx[u];
@@ -335,6 +488,7 @@ team_bags(f32x4 *__restrict__ stage, const char *__restrict__ table,
     int len_max = 0;
 #pragma unroll
     for (int i = 0; i < UB; ++i) len_max = max(len_max, end[i] - beg[i]);
+    const int len_most = T < 64 ? wave_max(len_max) : __builtin_amdgcn_readfirstlane(len_max);
 
 #pragma unroll
     for (int v0 = 0; v0 < VPL; v0 += VPP) {
@@ -349,114 +503,7 @@ team_bags(f32x4 *__restrict__ stage, const char *__restrict__ table,
           for (int e = 0; e < EPV; ++e) acc[i][v][e] = 0.f;
       }
 
-      // index of the lookup each (bag, unroll slot) will read next; -1 = none
-      int idx[UB][U];
-#pragma unroll
-      for (int i = 0; i < UB; ++i)
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int p = beg[i] + u * Y + y;
-          idx[i][u] = p < end[i] ? indices[p] : -1;
-        }
-
-      for (int base = 0; base < len_max; base += U * Y) {
-        Vec<VB> buf[UB][U][VPP];
-        f32x2 sb[UB][U];
-        const int nbase = base + U * Y;
-
-        // A round in which every lane of the wavefront has all its U lookups: straight-line
-        // code, every load issued before the first add.
-        bool full = true;
-#pragma unroll
-        for (int i = 0; i < UB; ++i) full = full && (beg[i] + nbase <= end[i]);
-        if (__builtin_amdgcn_ballot_w64(!full) == 0) {
-#pragma unroll
-          for (int i = 0; i < UB; ++i)
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-              const char *row = table + static_cast<int64_t>(idx[i][u]) * R::STRIDE;
-#pragma unroll
-              for (int v = 0; v < VPP; ++v) {
-                const int c = x + (v0 + v) * X;
-                if (v0 + v < VPL && c < R::V) buf[i][u][v] = load_vec<VB>(row + c * VB);
-              }
-              if constexpr (DT == I8) sb[i][u] = load_scale_bias<D>(row);
-            }
-          // next round's indices: the address is clamped into the bag, the value dropped if
-          // the position lies beyond it
-          int nidx[UB][U];
-#pragma unroll
-          for (int i = 0; i < UB; ++i)
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-              const int p = beg[i] + nbase + u * Y + y;
-              nidx[i][u] = indices[p < end[i] ? p : end[i] - 1];
-            }
-#pragma unroll
-          for (int i = 0; i < UB; ++i)
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-#pragma unroll
-              for (int v = 0; v < VPP; ++v) {
-                const int c = x + (v0 + v) * X;
-                if (v0 + v < VPL && c < R::V)
-                  accumulate<DT, VB>(acc[i][v], buf[i][u][v], DT == I8 ? sb[i][u].x : 1.f);
-              }
-              if constexpr (DT == I8) bias_acc[i] += sb[i][u].y;
-            }
-#pragma unroll
-          for (int i = 0; i < UB; ++i)
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-              const int p = beg[i] + nbase + u * Y + y;
-              idx[i][u] = p < end[i] ? nidx[i][u] : -1;
-            }
-          continue;
-        }
-
-#pragma unroll
-        for (int i = 0; i < UB; ++i)
-#pragma unroll
-          for (int u = 0; u < U; ++u)
-            if (idx[i][u] >= 0) {
-              const char *row = table + static_cast<int64_t>(idx[i][u]) * R::STRIDE;
-#pragma unroll
-              for (int v = 0; v < VPP; ++v) {
-                const int c = x + (v0 + v) * X;
-                if (v0 + v < VPL && c < R::V) buf[i][u][v] = load_vec<VB>(row + c * VB);
-              }
-              if constexpr (DT == I8) sb[i][u] = load_scale_bias<D>(row);
-            }
-
-        // fetch the next round of indices while the rows are in flight
-        int nidx[UB][U];
-#pragma unroll
-        for (int i = 0; i < UB; ++i)
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const int p = beg[i] + nbase + u * Y + y;
-            nidx[i][u] = p < end[i] ? indices[p] : -1;
-          }
-
-#pragma unroll
-        for (int i = 0; i < UB; ++i)
-#pragma unroll
-          for (int u = 0; u < U; ++u)
-            if (idx[i][u] >= 0) {
-#pragma unroll
-              for (int v = 0; v < VPP; ++v) {
-                const int c = x + (v0 + v) * X;
-                if (v0 + v < VPL && c < R::V)
-                  accumulate<DT, VB>(acc[i][v], buf[i][u][v], DT == I8 ? sb[i][u].x : 1.f);
-              }
-              if constexpr (DT == I8) bias_acc[i] += sb[i][u].y;
-            }
-
-#pragma unroll
-        for (int i = 0; i < UB; ++i)
-#pragma unroll
-          for (int u = 0; u < U; ++u) idx[i][u] = nidx[i][u];
-      }
+      sum_lookups<DT, D, X, Y, U, UB, VPP>(acc, bias_acc, table, indices, beg, end, len_most, v0, x, y, tid & 63);
 
       if constexpr (Y > 1) {
 #pragma unroll
@@ -614,7 +661,7 @@ onehot_bags(f32x4 *__restrict__ stage, const char *__restrict__ table,
     }
     // the rows
     Vec<VB> buf[UB][VPL];
-    f32x2 sb[UB];
+    uint32_t sb[UB];
 #pragma unroll
     for (int u = 0; u < UB; ++u)
       if (idx[u] >= 0) {
@@ -639,10 +686,10 @@ onehot_bags(f32x4 *__restrict__ stage, const char *__restrict__ table,
 #pragma unroll
         for (int e = 0; e < EPV; ++e) acc[e] = 0.f;
         if (idx[u] >= 0) {
-          accumulate<DT, VB>(acc, buf[u][v], DT == I8 ? sb[u].x : 1.f);
+          accumulate<DT, VB>(acc, buf[u][v], DT == I8 ? code_scale(sb[u]) : 1.f);
           if constexpr (DT == I8) {
 #pragma unroll
-            for (int e = 0; e < EPV; ++e) acc[e] += sb[u].y;
+            for (int e = 0; e < EPV; ++e) acc[e] = add_half<1>(acc[e], sb[u]);
           }
         }
         store_floats<EPV, OVEC>(dst + c * EPV, acc);
@@ -735,7 +782,7 @@ block_sum_range(BlockBagStorage<BT, DT, D, X, CHUNK> &s, const char *__restrict_
         for (int e = 0; e < EPV; ++e) sum[v][e] = 0.f;
       for (int base = first; base < stop; base += U * Y) {
         Vec<VB> buf[U][VPL];
-        f32x2 sb[U];
+        uint32_t sb[U];
         bool ok[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -757,9 +804,9 @@ block_sum_range(BlockBagStorage<BT, DT, D, X, CHUNK> &s, const char *__restrict_
 #pragma unroll
             for (int v = 0; v < VPL; ++v) {
               const int c = x + v * X;
-              if (c < R::V) accumulate<DT, VB>(sum[v], buf[u][v], DT == I8 ? sb[u].x : 1.f);
+              if (c < R::V) accumulate<DT, VB>(sum[v], buf[u][v], DT == I8 ? code_scale(sb[u]) : 1.f);
             }
-            if constexpr (DT == I8) bias_sum += sb[u].y;
+            if constexpr (DT == I8) bias_sum = add_half<1>(bias_sum, sb[u]);
           }
       }
 #pragma unroll

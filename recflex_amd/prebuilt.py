@@ -48,6 +48,8 @@ its library is missing.  Names:
                    2 500 small features, batch 256; ``workloads.REF_SHAPED``), default schedules;
                    ``refa_tuned`` / ``reff4_tuned``: with ``tuned/refa_schedule.json`` /
                    ``tuned/reff4_schedule.json`` if that file exists
+``bigtables``      tables of more than 4 GB under every template that walks bags, with lookups that do not
+                   share their lanes' rounds evenly (three in flight)
 ``wide``           1 500 small features (several binding rounds per thread)
 ``wider``          2 500 small features (bound once per launch by the binding kernel)
 ``widest``         4 500 small features (more than 64 chunks of 64 features: the prefix sum's second
@@ -299,6 +301,26 @@ def _few_mixed_bags() -> ModelSpec:
     return ModelSpec(wl, fs, 8, dict(bind_once=True))
 
 
+def _big_tables() -> ModelSpec:
+    """Tables beyond the reach of 32-bit offsets (up to 10 GB), one per template and element type."""
+    combos = [("float", 128, 20_000_000, 120.0, WavefrontPerBagSchedule, dict(lanes_x=8, items_per_thread=4)),
+              ("half", 64, 40_000_000, 20.0, SubWavefrontPerBagSchedule,
+               dict(lanes_x=8, lanes_y=1, items_per_thread=4, bags_per_team=1)),
+              ("int8", 128, 31_000_000, 30.0, SubWavefrontPerBagSchedule,
+               dict(lanes_x=8, lanes_y=4, items_per_thread=2, bags_per_team=1)),
+              ("float", 32, 36_000_000, 9.0, SubWavefrontPerBagSchedule,
+               dict(lanes_x=8, lanes_y=1, items_per_thread=3, bags_per_team=1)),
+              ("float", 4, 300_000_000, 6.0, ThreadPerBagSchedule, {}),
+              ("float", 128, 9_000_000, 700.0, BlockPerBagSchedule, {})]
+    feats, scheds = [], []
+    for data_type, dim, rows, mean, cls, want in combos:
+        sched = cls(MetaData(dim, data_type), BLOCK_THREADS)
+        params = sched.GenParamCandidates()[0]
+        scheds.append((sched, params._replace(vectors_per_pass=1, **want) if want else params))
+        feats.append(FeatureSpec(rows, dim, data_type, mean, False, 0.1, 0.0))
+    return ModelSpec(Workload("bigtables", 70, 2718, tuple(feats), "integer"), scheds, DEFAULT_OCCUPANCY)
+
+
 def _many_split() -> ModelSpec:
     """More split-bag workspace than a library's static device array may hold (32 MiB)."""
     feats = tuple(FeatureSpec(5000 + f, 256, "half", 3000.0, False, 0.0, 1.0) for f in range(17))
@@ -406,6 +428,7 @@ _SPECS: Dict[str, Callable[[], ModelSpec]] = {
     "fewbags_mixed": _few_mixed_bags,
     "fewbags512": lambda: _few_bags(True, 512, 1000.0),
     "manysplit": _many_split,
+    "bigtables": _big_tables,
     "wide": _wide,
     "wider": lambda: _wide(2500, "wider"),
     "widest": lambda: _wide(4500, "widest"),
