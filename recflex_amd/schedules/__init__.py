@@ -49,10 +49,13 @@ def default_schedule(meta: MetaData, mean_bag_len: float = 1.0, block_threads: i
     (``one_hot``: no bag of the feature is known to hold more than one lookup -- the row-copy
     template): enough
     column lanes that a lane owns one or two 16-byte vectors, lookup lanes only for long bags,
-    and two to four independent row loads in flight per lane -- fewer for fp16 and int8 rows,
-    whose 8 or 16 fp32 accumulators per 16-byte vector would otherwise push the fused kernel past
-    the registers that four or five workgroups per CU leave it (measured on C4 and C5: 2 % and
-    17 % faster than with four loads in flight everywhere)."""
+    and eight row vectors in flight per lane, four for fp16 and int8 rows with their 8 or 16
+    accumulators per vector, half as many where the bags hold few lookups (measured at four
+    workgroups per CU, us per launch with half as many in flight and with these: 1 000 fp32
+    features 85 and 79 at 256 samples, 31.9 and 27.6 at 64; 100 fp32 features 318 and 313 at
+    6 000; 200 int8 features 1 529 and 1 404 at 16 384, 17.1 and 14.7 at 64.  Eight for fp16
+    rows: 400 features 388 instead of 394 at 512 samples, but 4 624 instead of 4 299 at 8 192;
+    for int8 rows 13.7 and 1 461)."""
     if one_hot:
         sched = OneHotBagSchedule(meta, block_threads)
         return sched, sched.default_params()
@@ -71,7 +74,6 @@ def default_schedule(meta: MetaData, mean_bag_len: float = 1.0, block_threads: i
             return WavefrontPerBagSchedule(meta, block_threads), WavefrontPerBagParams(64, 1, vpl)
         return (SubWavefrontPerBagSchedule(meta, block_threads),
                 SubWavefrontPerBagParams(x, 1, 1, bags, vpl))
-    items = 4 if acc_floats <= 8 else 2
     if mean_bag_len >= 96 and meta.payload_bytes >= 512 and vpl * meta.elems_per_vector < 16:
         # long bags of wide rows: fewer column lanes, each with 16 accumulators (4 fp32 or 2 fp16
         # vectors), so that four (two) times as many lookups are in flight per wavefront -- the
@@ -79,7 +81,6 @@ def default_schedule(meta: MetaData, mean_bag_len: float = 1.0, block_threads: i
         vpl = max(1, 16 // meta.elems_per_vector)
         x = max(1, next_pow2(v) // vpl)
         vpl = -(-v // x)
-        items = 2
     if mean_bag_len < 24:
         y = 1
     elif mean_bag_len < 96:
@@ -93,6 +94,10 @@ def default_schedule(meta: MetaData, mean_bag_len: float = 1.0, block_threads: i
         return (SplitBagSchedule(meta, block_threads),
                 BlockPerBagParams(min(64, next_pow2(v)), 4 if meta.elems_per_vector <= 4 else 2,
                                   4 * block_threads))
+    items = max(1, (8 if meta.elems_per_vector <= 4 else 4) // vpl)
+    items = 1 << (items.bit_length() - 1)
+    if items * y >= 2 * mean_bag_len and meta.elems_per_vector != 8:
+        items = max(1, items // 2)
     team = x * y
     if team == 1:
         return ThreadPerBagSchedule(meta, block_threads), ThreadPerBagParams(items, 1, vpl)
