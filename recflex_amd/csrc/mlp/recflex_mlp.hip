@@ -5,9 +5,9 @@
 //
 // A batch of 512 through 4408 -> 1024 -> 256 -> 128 -> 1 is 5 GFLOP, 32 us at the rate a large fp32
 // product reaches here (154 TFLOP/s), and most of it the first layer.  Library products with
-// activations between them are eight launches and, one after the other in a graph, 73 us; batches
-// of 1, 37 and 256 take 50, 49 and 86 us.  Here they are three launches (four where the first
-// layer's K is split) and 65 us; 22, 29 and 44 us for the smaller batches:
+// activations between them are eight launches and, one after the other in a graph, 75 us; batches
+// of 1, 64 and 256 take 49, 50 and 86 us.  Here they are three launches (four where the first
+// layer's K is split) and 54 us; 19, 26 and 39 us for the smaller batches:
 //   gemm_nt    a layer: X [M, K] times W [N, K] transposed, bias and ReLU on the way out;
 //   tail       the last hidden layer, its ReLU, the dot product with the last layer's row and
 //              the sigmoid, and ahead of them the sum of the K-splits of the layer before.
@@ -28,39 +28,61 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 __device__ __forceinline__ float relu(const float x) { return x <= 0.f ? 0.f : x; }
 
 // ---------------------------------------------------------------------------------------------
-// gemm_nt: a workgroup of eight wavefronts computes a tile of 32 or 64 rows x 64 units.  Bound by the
-// matrix cores: 2 048 cycles of them per chunk (32 rows, 128 of K, or 64 rows, 64 of K) for 48 or 32 KB
-// read, of the 128 KB that the L2 delivers to a CU meanwhile.  They are busy 62 to 68 % of the time
-// (batch 512, K 23 980: 105 TFLOP/s; the library's kernel 72 %); tiles of 64 x 64 and 128 x 64 by four
-// or eight wavefronts, chunks of 32 to 128 and one to eight splits all end within 7 % of each other.
-// The tiles are small for the number of them: a batch of 512 and 1 024 units give 256 tiles of 32
-// rows, one per CU.  Such a CU has two wavefronts per SIMD and nothing else to run while they wait,
-// so the wavefronts split the K of a chunk among them, meet once per chunk, and a chunk is asked for
-// two ahead: it goes to LDS while the matrix cores work on the one before.
+// gemm_nt: a workgroup of eight wavefronts computes a tile of 32 or 64 rows x 64 units of fp32 products on
+// the bf16 matrix cores: every operand is the sum of three bf16 numbers (8 + 8 + 8 bits with their signs
+// hold the 24 exactly), and of their nine products the six are formed that reach the last bit (the others
+// are below 2^-26 of the product).  16 of K take 6 x 15 ns of a SIMD that way and 8 x 27 ns as fp32 products.
+// Errors against 64 bits, 2-norm, first hidden layer, 4 408 inputs: 2.5e-7 and 5.7e-7 at 512 rows, 1.4e-7 and
+// 1.8e-7 at one (23 980 inputs: 4.7e-7 and 6.9e-7, 2.7e-7 and 3.6e-7): what counts is how often a sum is
+// rounded, and a product of 16 of K rounds it once where two of K did.
+// The wavefronts split K among them, each with the whole tile to itself: no operand is taken apart twice
+// and they meet once, to add up their sums.  A step's operands go through the wavefront's own LDS (as
+// loaded: rows of 64 or 128 bytes; as read: a lane's eight of a row) and are taken apart in registers, in
+// 400 ns of vector instructions beside 360 ns of products (64 x 64, 16 of K).
+// 512 rows, 4 408 -> 1 024 units: 57 us as fp32 products, 38 now (122 TFLOP/s).  What bounds it now is the
+// operands' way to the CU: 64 KB per round of the wavefronts in 1.9 us.  Asking for them two or three steps
+// ahead, products and vector instructions interleaved by hand, and LDS without bank conflicts left that
+// time where it is; steps of 32 (whole cache lines by one wavefront) took 9 % off it at 23 980 inputs
+// and added 4 % at 4 408, whose steps they divide less evenly.
 // N and K are multiples of 4 (valid): a vector of four units is whole or beyond N.
 // ---------------------------------------------------------------------------------------------
-constexpr int kTileN = 64, kThreads = 512;
+constexpr int kTileN = 64, kThreads = 512, kWaves = kThreads / 64;
+constexpr int kRedRow = kTileN + 4;
+// from this K on a step is 32 of K instead of 16
+constexpr int kLongK = 8192;
 
-// TM x 64 tile: a wavefront sums WM blocks of 32 x 32 over its share of a chunk's K
-template <int TM, int KC, int WM> struct Tile {
-  static constexpr int kM = TM, kChunk = KC;
-  static constexpr int kRow = KC + 4;          // LDS row, in floats: 16-byte reads of 8 rows spread over all banks
-  static constexpr int kRows = TM + kTileN;
-  static constexpr int kVecs = KC / 4;         // 16-byte vectors of a row
-  static constexpr int kRowsPerLoad = kThreads / kVecs;
-  static constexpr int kLoads = kRows / kRowsPerLoad;
-  static constexpr int kKGroups = kThreads / 64 / (TM / 32 / WM * 2);       // wavefronts that share a tile's K
-  static constexpr int kRedRow = kTileN + 4;
-  static_assert(TM % kRowsPerLoad == 0 && kTileN % kRowsPerLoad == 0, "a load instruction stays within X or within W");
-  static_assert(kKGroups * TM * kRedRow <= 2 * kRows * kRow, "the sums fit where the chunks were");
-};
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-template <int TM, int KC, int WM>
+// eight fp32 numbers as high + middle + low, exactly (numbers beyond the largest bf16 become infinite,
+// and their products with the other parts NaN: see below)
+struct Parts { bf16x8 high, middle, low; };
+__device__ __forceinline__ Parts parts_of(const f32x4 v0, const f32x4 v1) {
+  u32x4 part[3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float x = i < 2 ? v0[2 * i] : v1[2 * i - 4], y = i < 2 ? v0[2 * i + 1] : v1[2 * i - 3];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      uint32_t w;                                // (the compiler would round x once more to have it by itself)
+      asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(w) : "v"(x), "v"(y));
+      part[p][i] = w;
+      x -= __uint_as_float(w << 16);
+      y -= __uint_as_float(w & 0xffff0000u);
+    }
+  }
+  return {__builtin_bit_cast(bf16x8, part[0]), __builtin_bit_cast(bf16x8, part[1]), __builtin_bit_cast(bf16x8, part[2])};
+}
+
+// TM rows, steps of STEP of K
+template <int TM, int STEP>
 __global__ void __launch_bounds__(kThreads)
 gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
         float *__restrict__ out, const int M, const int N, const int K, const int splits) {
-  using T = Tile<TM, KC, WM>;
-  __shared__ float lds[2 * T::kRows * T::kRow];
+  constexpr int ROWS = TM + kTileN, LANES = STEP / 4, LOADS = ROWS * LANES / 64, WM = TM / 32, WN = kTileN / 32;
+  constexpr int ROW = STEP + 4;                  // LDS row, in floats: 16-byte reads of 8 rows spread over all banks
+  constexpr int LDS = kWaves * ROWS * ROW > kWaves * TM * kRedRow ? kWaves * ROWS * ROW : kWaves * TM * kRedRow;
+  __shared__ float lds[LDS];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tiles_n = (N + kTileN - 1) / kTileN;
@@ -69,92 +91,118 @@ gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *_
   // consecutive workgroups (one XCD each) take the units of the same rows: an XCD keeps to an
   // eighth of the weights, the larger operand
   const int m0 = tile / tiles_n * TM, n0 = tile % tiles_n * kTileN;
-  const int chunks = (K + KC - 1) / KC;
-  const int per_split = (chunks + splits - 1) / splits;
-  const int first = split * per_split, last = min(chunks, first + per_split);
+  const int steps = (K + STEP - 1) / STEP;
+  const int per_split = (steps + splits - 1) / splits;
+  const int first = split * per_split, last = min(steps, first + per_split);
 
   // rows beyond M or N repeat the last one (their sums are not stored); K beyond the end reads 0
-  const int col = tid % T::kVecs * 4;
-  const float *src[T::kLoads];
+  const int col = lane % LANES * 4;
+  const float *src[LOADS];
 #pragma unroll
-  for (int i = 0; i < T::kLoads; ++i) {
-    const int row = i * T::kRowsPerLoad + tid / T::kVecs;
-    src[i] = (i * T::kRowsPerLoad < TM
-                  ? x + static_cast<int64_t>(min(m0 + row, M - 1)) * K
-                  : w + static_cast<int64_t>(min(n0 + row - TM, N - 1)) * K) + col;
+  for (int i = 0; i < LOADS; ++i) {
+    const int row = (i * 64 + lane) / LANES;
+    src[i] = (i * 64 / LANES < TM ? x + static_cast<int64_t>(min(m0 + row, M - 1)) * K
+                          : w + static_cast<int64_t>(min(n0 + row - TM, N - 1)) * K) + col;
   }
-  f32x4 next[T::kLoads];
-  auto request = [&](const int c) {
-    const int k = min(c * KC, K - 4 - col);      // stays within the row
+  f32x4 next[LOADS];
+  auto request = [&](const int step) {
+    const int k = min(step * STEP, K - 4 - col);      // stays within the row
 #pragma unroll
-    for (int i = 0; i < T::kLoads; ++i) next[i] = *reinterpret_cast<const f32x4 *>(src[i] + k);
+    for (int i = 0; i < LOADS; ++i) next[i] = *reinterpret_cast<const f32x4 *>(src[i] + k);
   };
-  auto put = [&](float *buf, const int c) {
-    if (c * KC + KC > K) {                       // the last chunk's surplus
-      const bool in = c * KC + col < K;
+  float *mine = lds + wave * (ROWS * ROW);
+  auto put = [&](const int step) {
+    if (step * STEP + STEP > K) {              // the last step's surplus
+      const bool in = step * STEP + col < K;
 #pragma unroll
-      for (int i = 0; i < T::kLoads; ++i)
+      for (int i = 0; i < LOADS; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) next[i][j] = in ? next[i][j] : 0.f;
     }
 #pragma unroll
-    for (int i = 0; i < T::kLoads; ++i)
-      *reinterpret_cast<f32x4 *>(buf + (i * T::kRowsPerLoad + tid / T::kVecs) * T::kRow + col) = next[i];
+    for (int i = 0; i < LOADS; ++i)
+      *reinterpret_cast<f32x4 *>(mine + (i * 64 + lane) / LANES * ROW + col) = next[i];
   };
 
-  f32x16 acc[WM];
+  f32x16 acc[WM][WN];
 #pragma unroll
-  for (int v = 0; v < WM; ++v)
+  for (int m = 0; m < WM; ++m)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[v][r] = 0.f;
-  const int half_n = wave & 1, part_m = (wave >> 1) % (TM / 32 / WM), kgroup = wave / (TM / 32 / WM * 2);
-  // lane (i, h) of a 32x32x2 product holds row i at two values of k, one per h; which two does not
-  // matter as long as both operands agree, so a lane reads four consecutive ones at once
-  const int frag = (lane & 31) * T::kRow + kgroup * (KC / T::kKGroups) + (lane >> 5) * 4;
-  if (first < last) {
-    request(first);
-    put(lds, first);
-    if (first + 1 < last) request(first + 1);
-  }
-  __syncthreads();
-  for (int c = first; c < last; ++c) {
-    // chunk c + 1, requested a chunk ago, goes to the other buffer (every wavefront is past the
-    // barrier behind its last reads of it) while the matrix cores are busy with chunk c
-    if (c + 1 < last) put(lds + ((c + 1 - first) & 1) * (T::kRows * T::kRow), c + 1);
-    if (c + 2 < last) request(c + 2);
-    const float *buf = lds + ((c - first) & 1) * (T::kRows * T::kRow);
-    const float *xs = buf + part_m * 32 * WM * T::kRow + frag, *ws = buf + (TM + half_n * 32) * T::kRow + frag;
+    for (int n = 0; n < WN; ++n)
 #pragma unroll
-    for (int s = 0; s < KC / T::kKGroups / 8; ++s) {
-      f32x4 a[WM];
+      for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
+  // lane (i, h) of a 32x32x16 product holds row i at eight values of k, one set per h
+  const float *frag = mine + (lane & 31) * ROW + (lane >> 5) * 8;
+  auto operand = [&](const int block, const int sub) {
+    const float *at = frag + block * 32 * ROW + sub * 16;
+    return parts_of(*reinterpret_cast<const f32x4 *>(at), *reinterpret_cast<const f32x4 *>(at + 4));
+  };
+  if (first + wave < last) request(first + wave);
+  for (int step = first + wave; step < last; step += kWaves) {
+    put(step);
+    if (step + kWaves < last) request(step + kWaves);
+    // the wavefront's own LDS: its writes before its reads
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-      for (int v = 0; v < WM; ++v) a[v] = *reinterpret_cast<const f32x4 *>(xs + v * 32 * T::kRow + s * 8);
-      const f32x4 b = *reinterpret_cast<const f32x4 *>(ws + s * 8);
+    for (int sub = 0; sub < STEP / 16; ++sub) {
+      Parts b[WN];
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int n = 0; n < WN; ++n) b[n] = operand(WM + n, sub);
 #pragma unroll
-        for (int v = 0; v < WM; ++v)
-          acc[v] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[v][j], b[j], acc[v], 0, 0, 0);
+      for (int m = 0; m < WM; ++m) {
+        const Parts a = operand(m, sub);
+#pragma unroll
+        for (int n = 0; n < WN; ++n) {             // smallest first
+          f32x16 c = acc[m][n];
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.middle, b[n].middle, c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.high, b[n].low, c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.low, b[n].high, c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.high, b[n].middle, c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.middle, b[n].high, c, 0, 0, 0);
+          acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.high, b[n].high, c, 0, 0, 0);
+        }
+      }
     }
-    __syncthreads();
+    // ... and these reads before the next step's writes
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
 
   // the wavefronts' shares of K, added in order
+  __syncthreads();
 #pragma unroll
-  for (int v = 0; v < WM; ++v)
+  for (int m = 0; m < WM; ++m)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = (part_m * WM + v) * 32 + 8 * (r / 4) + 4 * (lane >> 5) + r % 4;
-      lds[(kgroup * TM + row) * T::kRedRow + half_n * 32 + (lane & 31)] = acc[v][r];
-    }
+    for (int n = 0; n < WN; ++n)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = m * 32 + 8 * (r / 4) + 4 * (lane >> 5) + r % 4;
+        lds[(wave * TM + row) * kRedRow + n * 32 + (lane & 31)] = acc[m][n][r];
+      }
   __syncthreads();
   for (int at = tid; at < TM * (kTileN / 4); at += kThreads) {
     const int row = at / (kTileN / 4), unit = at % (kTileN / 4) * 4;
-    f32x4 sum = *reinterpret_cast<const f32x4 *>(lds + row * T::kRedRow + unit);
+    f32x4 sum = *reinterpret_cast<const f32x4 *>(lds + row * kRedRow + unit);
 #pragma unroll
-    for (int g = 1; g < T::kKGroups; ++g)
-      sum += *reinterpret_cast<const f32x4 *>(lds + (g * TM + row) * T::kRedRow + unit);
+    for (int g = 1; g < kWaves; ++g)
+      sum += *reinterpret_cast<const f32x4 *>(lds + (g * TM + row) * kRedRow + unit);
     if (m0 + row >= M || n0 + unit >= N) continue;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      // An infinity's parts are infinity and NaN, so its products are NaN where fp32 has an infinity, and of
+      // numbers below 1e-33 the low part is lost among the subnormals: a sum that such operands may have
+      // made (not finite, or all but zero) is formed again, term by term.
+      const float size = fabsf(sum[j]);
+      if (!(size <= 3.4028234e38f) || (size < 1e-25f && size > 0.f)) {
+        const float *xs = x + static_cast<int64_t>(m0 + row) * K, *ws = w + static_cast<int64_t>(n0 + unit + j) * K;
+        float t = 0.f;
+        for (int k = first * STEP; k < min(K, last * STEP); ++k) t = fmaf(xs[k], ws[k], t);
+        sum[j] = t;
+      }
+    }
     float *dst = out + (static_cast<int64_t>(split) * M + m0 + row) * N + n0 + unit;
     if (bias) {
 #pragma unroll
@@ -292,22 +340,22 @@ tail(const float *__restrict__ parts, const int splits, const float *__restrict_
 
 int ceil_div(const int64_t a, const int64_t b) { return static_cast<int>((a + b - 1) / b); }
 
-// How a layer is cut: tiles of 32 or 64 rows, and its K into splits.  What a CU takes for a chunk was
-// measured at a batch of 512 and K 23 980: 1.35 us (32 rows), 1.25 us (64 rows, one workgroup on the
-// CU) and 1.18 us (64 rows, two); two more chunks' time for the first loads and the last sums.  Splits
-// cost their traffic and, ahead of any layer but the tail, a kernel that adds them up.
+// How a layer is cut: tiles of 32 or 64 rows, and its K into splits.  What a CU takes for a chunk (16 of K for
+// every wavefront) with all CUs at work: 1.2 us (32 rows) and 1.9 us (64 rows), at 256, 512 and 2 048 rows
+// alike; another 3 us for the first loads and the last sums.  Splits cost their traffic and, ahead of any
+// layer but the tail, a kernel that adds them up.
 struct Plan { int rows, splits; };
 Plan plan_of(const int M, const int N, const int K, const int cus, const bool feeds_tail) {
   Plan best{32, 1};
   double best_us = 1e30;
   for (int rows = 32; rows <= 64; rows += 32) {
     const int64_t tiles = static_cast<int64_t>(ceil_div(M, rows)) * ceil_div(N, kTileN);
-    const int chunks = ceil_div(K, rows == 32 ? 128 : 64);
+    const int chunks = ceil_div(K, kWaves * 16);
     for (int s = 1; s <= RECFLEX_MLP_MAX_SPLITS && s <= chunks; ++s) {
       const int per_split = ceil_div(chunks, s);
       if (static_cast<int64_t>(per_split) * (s - 1) >= chunks) continue;            // an empty split
-      const double chunk_us = rows == 32 ? 1.35 : (tiles * s > cus ? 1.18 : 1.25);
-      double us = chunk_us * ceil_div(tiles * s, cus) * (per_split + 2);
+      const double chunk_us = rows == 32 ? 1.2 : 1.9;
+      double us = (chunk_us * per_split + 3.) * ceil_div(tiles * s, cus);
       if (s > 1) us += (feeds_tail ? 0. : 3.) + 2. * s * M * N * 4 / 4e6;
       if (us < best_us * 0.98) { best = {rows, s}; best_us = us; }
     }
@@ -386,8 +434,10 @@ extern "C" int recflex_mlp_forward(const recflex_mlp_args *a) {
     float *out = direct ? a->hidden[l] : a->workspace;
     void *args[] = {&x, &w, &bias, &out, &M, &N, &K, &splits};
     const int64_t tiles = static_cast<int64_t>(ceil_div(M, plan.rows)) * ceil_div(N, kTileN);
-    const void *kernel = plan.rows == 32 ? reinterpret_cast<const void *>(&gemm_nt<32, 128, 1>)
-                                         : reinterpret_cast<const void *>(&gemm_nt<64, 64, 2>);
+    const void *kernel = K < kLongK ? (plan.rows == 32 ? reinterpret_cast<const void *>(&gemm_nt<32, 16>)
+                                                       : reinterpret_cast<const void *>(&gemm_nt<64, 16>))
+                                    : (plan.rows == 32 ? reinterpret_cast<const void *>(&gemm_nt<32, 32>)
+                                                       : reinterpret_cast<const void *>(&gemm_nt<64, 32>));
     e = launch(kernel, tiles * splits, kThreads, args);
     if (e != hipSuccess) return static_cast<int>(e);
     if (!direct && !feeds_tail) {

@@ -32,21 +32,14 @@ except (ImportError, AttributeError):
 MAX_LAYERS = 8                      # RECFLEX_MLP_MAX_LAYERS
 TAIL_MAX_UNITS = 128                # RECFLEX_MLP_TAIL_MAX_UNITS
 TAIL_MAX_INPUTS = 1024              # RECFLEX_MLP_TAIL_MAX_INPUTS
-# Where the kernels pay, against the modules (in us; both called one after another, and in a graph).
-# The library has switches of its own: up to 256 rows its products take 1.2 to 5 times as long as
-# these, beyond them it is now behind and now ahead.
-#  * Up to 512 rows with layers of up to 1 024 units: 1024, 256, 128 on 4 408 inputs, 256 / 384 / 512
-#    rows 44 / 55 / 64 against 107 (graph 86 / 72 / 74); on 23 980 inputs 138 / 194 / 238 against 383 /
-#    362 / 249.  (1024, 512, 128 on 12 000 inputs is the exception: 450 / 512 rows 136 / 141 against
-#    130 / 130.)
-#  * Wider layers up to 256 rows (8192, 512, 128 on 4 408 inputs, 256 rows: 200 against 238), and beyond
-#    as long as there is little to multiply: these products run at 105 TFLOP/s, the library's large
-#    ones at up to 140, and its launches cost some 40 us.  4 408 inputs, first layer and rows: 2 048
-#    and 352 (7.1 GFLOP) 99 against 109 (graph 95), 2 048 and 416 (8.4) 113 and 110, 4 096 and 512
-#    (21) 198 and 180, 8 192 and 512 (41) 373 and 320; 23 980 inputs, 4 096 and 512 (102) 889 and 717.
-#    (Not without exceptions: 23 980 inputs, 1 536 and 512 rows, 353 against 681.)
-#  * Beyond 512 rows the modules: 1024, 256, 128 on 23 980 inputs, 700 / 1 024 / 2 048 rows 345 / 452 /
-#    888 against 679 / 374 / 713, on 4 408 inputs 91 / 103 / 184 against 109 / 110 / 172.
+# Where the kernels serve, against the modules (in us; both in a graph, where the library's launches cost
+# least).  Up to 256 rows always: the library's products take 1.1 to 5 times as long as these.  Beyond, up to
+# 512 rows: 1024, 256, 128 units on 4 408 inputs, 384 / 512 rows 52 / 57 against 74 / 76, on 23 980 inputs 162 /
+# 197 against 364 / 269, on 512 inputs 24 / 25 against 42 / 43; wider layers gain less (4096, 512, 128 on 4 408
+# inputs, 512 rows, 20 GFLOP: 169 against 185) and lose with much to multiply (8192, 512, 128 on 23 980 inputs,
+# 384 rows, 151 GFLOP: 1 185 against 1 154): beyond 8 GFLOP they are left to the modules.  Beyond 512 rows the
+# modules serve, though up to some 80 GFLOP these would be the faster ones there too (1024, 256, 128 on 4 408
+# inputs, 1 024 / 2 048 rows 88 / 158 against 109 / 174, on 23 980 inputs 381 / 723 against 415 / 734).
 MAX_BATCH = 512
 ANY_WIDTH_BATCH = 256
 NARROW_UNITS = 1024

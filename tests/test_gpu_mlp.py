@@ -157,3 +157,19 @@ def test_mlp_leaves_large_products_to_the_library():
         assert kernels.forward(mlp, x) is None
         got = kernels.forward(mlp, x[:kernels.ANY_WIDTH_BATCH])
         assert got is not None and rel(got, mlp.double()(x[:kernels.ANY_WIDTH_BATCH].double())) < REL
+
+
+# what three bf16 numbers per operand can and cannot hold: numbers whose low parts are subnormal, numbers near
+# the largest; K of the long steps and its remainders, tiles of 64 rows without splits
+@pytest.mark.parametrize("units, batch, scale", [
+    ((260, 96, 32), 70, 1e-36), ((260, 96, 32), 70, 1e-30), ((260, 96, 32), 70, 1e30), ((8196, 64, 16), 40, 1.),
+    ((8224, 100, 16), 65, 1.), ((1000, 1024, 128), 1025, 1.)])
+def test_mlp_products_of_parts(units, batch, scale):
+    print("[case] mlp", units, batch, scale, flush=True)
+    mlp = build(units)
+    for m in mlp[::2]:
+        m.bias.data.zero_()
+    x = torch.randn(batch, units[0], device="cuda") * scale
+    ws, bs = [m.weight.detach() for m in mlp[::2]], [m.bias.detach() for m in mlp[::2]]
+    hidden = kernels._run(x, ws, bs, True)[1][0]
+    assert rel(hidden / scale, torch.relu(x.double() @ ws[0].double().t()) / scale) < REL
