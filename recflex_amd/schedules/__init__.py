@@ -90,9 +90,11 @@ def default_schedule(meta: MetaData, mean_bag_len: float = 1.0, block_threads: i
     if mean_bag_len >= 512 and next_pow2(v) >= 4:
         # the whole workgroup on one bag, one row vector per lane -- and several workgroups per
         # bag when the batch holds so few bags that one of them is a good part of a workgroup's
-        # share (8 features x 64 bags x 4 000 lookups: 105 us against 203 us with a team per bag)
+        # share (8 features x 64 bags x 4 000 lookups: 105 us against 203 us with a team per bag);
+        # eight fp32 vectors in flight per lane (8 features, 1 bag of 28 000 lookups 17.8 us with
+        # four and 16.0, 16 of 20 000 73.5 and 72.2, 128 of 2 000 61.4 and 60.9)
         return (SplitBagSchedule(meta, block_threads),
-                BlockPerBagParams(min(64, next_pow2(v)), 4 if meta.elems_per_vector <= 4 else 2,
+                BlockPerBagParams(min(64, next_pow2(v)), 8 if meta.elems_per_vector <= 4 else 2,
                                   4 * block_threads))
     items = max(1, (8 if meta.elems_per_vector <= 4 else 4) // vpl)
     items = 1 << (items.bit_length() - 1)
