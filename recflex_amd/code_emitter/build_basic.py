@@ -11,6 +11,7 @@ import hashlib
 import os
 import shutil
 import subprocess
+import sysconfig
 from typing import List
 
 import recflex_amd
@@ -26,6 +27,7 @@ class BasicBuilder:
         # include/recflex_hip.h sits at the repository root, beside the package
         self.abi_include = os.path.join(os.path.dirname(self.package_dir), "include")
         self.host_source = os.path.join(self.csrc_dir, "host", "recflex_host.cpp")
+        self.strings_source = os.path.join(self.csrc_dir, "host", "recflex_strings.cpp")
         self.hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
         self.cxx = shutil.which("g++") or "g++"
         # gfx950 only; packed fp32 instructions are disabled on purpose
@@ -54,6 +56,14 @@ class BasicBuilder:
             os.makedirs(os.path.dirname(lib), exist_ok=True)
             tmp = lib + f".tmp{os.getpid()}"
             cmd = [self.cxx, *self.host_flags, "-O3", f"-I{self.abi_include}", self.host_source, "-o", tmp]
+            # the reader of Python's own strings, where its headers are installed
+            python_include = sysconfig.get_paths()["include"]
+            if os.path.exists(os.path.join(python_include, "Python.h")) and os.path.exists(self.strings_source):
+                with_strings = subprocess.run([*cmd, self.strings_source, f"-I{python_include}"],
+                                              stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+                if with_strings.returncode == 0:
+                    os.replace(tmp, lib)
+                    return lib
             subprocess.run(cmd, check=True)
             os.replace(tmp, lib)
         return lib

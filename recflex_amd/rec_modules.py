@@ -75,30 +75,39 @@ class FeatPreprocess(nn.Module):
         self.output_units = output_units
 
     def forward(self, raw_data: List[List[str]], max_concurrent_blocks: int = 0):
-        # (a RecomHost as it is hands the packed buffer over: the arrays of data are not needed)
         host = self.recom_host
-        whole = type(host) is not RecomHost or "preprocess" in vars(host)
-        (data_buffer_offsets, output_offsets, extra_buffer_offsets, task_mapping, task_tiles, data,
-         scala_data) = host.preprocess(raw_data, max_concurrent_blocks) if whole else host._preprocess(raw_data, False)
+        if type(host) is RecomHost and "preprocess" not in vars(host):
+            # a RecomHost as it is hands arrays over: the packed buffer without the arrays of data, the
+            # offsets without a list in between, and no tasks and extra buffers (all zeros)
+            byte_offsets, output_size, scala = host.preprocess_packed(raw_data)
+            num_feats = len(raw_data)
+            arg_buffers = torch.from_numpy(host.packed).to(self.device)
+            data_buffer_offsets = torch.from_numpy(byte_offsets).to(self.device)
+            scala_args = torch.from_numpy(scala).to(self.device)
+            extra_buffers = torch.empty([0], dtype=torch.int8, device=self.device)
+            extra_buffer_offsets = torch.zeros([num_feats + 1], dtype=torch.int32, device=self.device)
+            task_mapping = torch.empty([0, 2], dtype=torch.int32, device=self.device)
+            task_tiles = torch.zeros([num_feats], dtype=torch.int32, device=self.device)
+            task_barriers = torch.zeros([0], dtype=torch.int32, device=self.device)
+        else:
+            (data_buffer_offsets, output_offsets, extra_buffer_offsets, task_mapping, task_tiles, data,
+             scala_data) = host.preprocess(raw_data, max_concurrent_blocks)
+            output_size = output_offsets[-1]
+            extra_buffers = torch.empty([extra_buffer_offsets[-1]], dtype=torch.int8, device=self.device)
+            task_barriers = torch.zeros([len(task_mapping)], dtype=torch.int32, device=self.device)
 
-        output_size: int = output_offsets[-1]
+            packed = getattr(self.recom_host, "packed", None)
+            if packed is None:
+                packed = np.concatenate([np.asarray(d, dtype=np.int32) for d in data]) if data \
+                    else np.zeros(0, np.int32)
+            arg_buffers = torch.from_numpy(packed).to(self.device)
+            data_buffer_offsets = torch.tensor(data_buffer_offsets, dtype=torch.int64, device=self.device)
+            extra_buffer_offsets = torch.tensor(extra_buffer_offsets, dtype=torch.int32, device=self.device)
+            task_mapping = torch.tensor(task_mapping, dtype=torch.int32, device=self.device).reshape(-1, 2)
+            task_tiles = torch.tensor(task_tiles, dtype=torch.int32, device=self.device)
+            scala_args = torch.tensor(scala_data, dtype=torch.int32, device=self.device)
         if output_size == 0 and self.output_units and len(raw_data) > 0:
             output_size = len(raw_data[0]) * self.output_units * 4
-        total_blocks = len(task_mapping)
-
-        extra_buffers = torch.empty([extra_buffer_offsets[-1]], dtype=torch.int8, device=self.device)
-        task_barriers = torch.zeros([total_blocks], dtype=torch.int32, device=self.device)
-
-        packed = getattr(self.recom_host, "packed", None)
-        if packed is None:
-            packed = np.concatenate([np.asarray(d, dtype=np.int32) for d in data]) if data \
-                else np.zeros(0, np.int32)
-        arg_buffers = torch.from_numpy(packed).to(self.device)
-        data_buffer_offsets = torch.tensor(data_buffer_offsets, dtype=torch.int64, device=self.device)
-        extra_buffer_offsets = torch.tensor(extra_buffer_offsets, dtype=torch.int32, device=self.device)
-        task_mapping = torch.tensor(task_mapping, dtype=torch.int32, device=self.device).reshape(-1, 2)
-        task_tiles = torch.tensor(task_tiles, dtype=torch.int32, device=self.device)
-        scala_args = torch.tensor(scala_data, dtype=torch.int32, device=self.device)
 
         return (
             arg_buffers,

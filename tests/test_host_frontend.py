@@ -190,3 +190,34 @@ def test_joint_parse_reports_the_first_feature_that_fails(host, bad, message):
     for parse in (host.preprocess, host._parse_each):
         with pytest.raises(RecomHostError, match=message):
             parse(raw)
+
+
+# lists, tuples and what only the joined text can hold; lengths around the eight bytes that are read at a time,
+# numbers of up to ten digits, separators at the ends
+@pytest.mark.parametrize("line", ["", "5", ",", "1234567", "12345678", "1234567,", ",1234567", "123456,89012345", "2147483647",
+                                  "0,00000000007,1", "9;8 7\t6", "12345678,87654321,1", "1,2,3,4,5,6,7,8", "é,1", "1,₂,3"])
+@pytest.mark.parametrize("box", [list, tuple])
+def test_strings_where_they_lie_equal_the_joined_text(host, line, box):
+    raw = box([box([line, "1", line, "", line + line]), box(["7", "", "8,9", line, ""])])
+    if max((len(w) for w in line.replace(";", ",").split(",")), default=0) > 5:
+        raw = box([box([line, "1", line, "", line]), box(["7", "", "8,9", line, ""])])
+    counts, at = np.empty(2, np.int64), np.zeros(3, np.int64)
+    want = host._parse_joined(raw, 5, counts, at)
+    got_counts, got_at = np.empty(2, np.int64), np.zeros(3, np.int64)
+    got = host._parse_strings(raw, 5, got_counts, got_at)
+    if not line.isascii():
+        assert got is None
+    else:
+        assert np.array_equal(got, want) and np.array_equal(got_counts, counts) and np.array_equal(got_at, at)
+    assert np.array_equal(host._parse_packed(list(raw), False)[2], at) and np.array_equal(host.packed, want)
+
+
+def test_strings_that_are_not_plain_are_left_to_the_joined_text(host):
+    class Line(str):
+        pass
+
+    counts, at = np.empty(1, np.int64), np.zeros(2, np.int64)
+    for lines in (["1\n2", "3"], ["2147483648", "1"], ["99999999999", "1"], [Line("1"), "2"], [b"1", "2"], np.array(["1", "2"]),
+                  ["1"], [None, "1"]):
+        assert host._parse_strings([lines], 2, counts, at) is None
+    assert host._parse_strings(np.array([["1", "2"]]), 2, counts, at) is None
