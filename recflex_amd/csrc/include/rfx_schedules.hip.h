@@ -48,7 +48,7 @@ template <int BT> struct TeamStage {
 // loop; given the plain thread index the compiler computes every body's lane decomposition (team,
 // x, y and what follows from them) once before that loop and keeps all of it in registers
 // throughout: 128 registers and a spill for the 100-feature model, against 94 when each body
-// derives its values per tile.  The lane number therefore passes through an empty asm statement,
+// derived its values per tile (both with the teams' loop before sum_lookups; 80 with it).  The lane number therefore passes through an empty asm statement,
 // which nothing can be moved across.  The wavefront number stays a scalar and both ranges stay
 // visible to the compiler (the masks), which the straight-line paths of the bodies rely on.
 template <int BT> __device__ __forceinline__ int body_thread_id() {
@@ -184,7 +184,10 @@ template <typename R> __device__ __forceinline__ int windows_of(const int row) {
 // Measured, same bits: 200 int8 features (16 384 samples) 1 560 -> 1 405 us, 400 fp16 (8 192) 4 115 -> 4 015,
 // 100 fp32 features (tuned, 2 048) 121.4 -> 118.9, (default schedules, 1 337) 94.0 -> 90.1, 2 500 (256)
 // 178.3 -> 175.9.  The registers go from 96 and 4 spilled to 74, from 109 to 79 and from 96 to 82: room for
-// more workgroups on a CU, or more rows in flight.
+// more workgroups on a CU, or more rows in flight, which the schedules take (the first three 1 326, 3 729 and
+// 115 us with them).  A round costs the same however many of its lookups are left; closing a bag with a
+// round of a half, a quarter or an eighth of U gave 1 to 2 % (115.6 -> 114.0, 1 312 -> 1 300) for four more
+// copies of the loop's body in each schedule, and spills where a model has outlier tiles.
 // ---------------------------------------------------------------------------------------------
 template <int DT, int D, int X, int Y, int U, int UB, int VPP, int EPV>
 __device__ __forceinline__ void
@@ -294,8 +297,9 @@ sum_lookups(float (&acc)[UB][VPP][EPV], float (&bias_acc)[UB], const char *__res
 // memory round trip each: a single bag of 2 000 lookups among one-lookup bags (16 lanes per bag,
 // one lookup in flight) held one wavefront for 1.2 ms in a kernel of 124 us, one of 20 000 for
 // 10 ms.  Here all 64 lanes work on the bag: as many column lanes as the row has vectors (at
-// most 64), the rest lookup lanes, four lookups in flight each (eight would push the
-// 100-feature kernel, which inlines this into twenty bodies, over its 96 registers: 8 spills),
+// most 64), the rest lookup lanes, four lookups in flight each (every team body inlines this, twenty
+// times in the 100-feature kernel: with eight it spilled, and through sum_lookups or its row windows it
+// took 117.5-125.9 us instead of 115.5-117.5 on bags that never come here),
 // indices fetched a round ahead, butterfly over the lookup lanes at the end.
 // No LDS and no barrier: only the wavefront that met the bag is involved.
 // ---------------------------------------------------------------------------------------------

@@ -68,7 +68,9 @@ RFX_SIZES_FN int capped_tile_size(const int built, const long long total, const 
 // unsplit at 185 us.)
 // Smallest part: 256 KiB of traffic (with 128 KiB parts the three shapes above take 175 / 108 /
 // 161 us at four workgroups per CU, with 256 KiB parts 142 / 103 / 122 us; at eight workgroups
-// per CU, which these light kernels allow, 138 / 76 / 83 us and 107 / 83 / 96 us).
+// per CU, which these light kernels allow, 138 / 76 / 83 us and 107 / 83 / 96 us.  All of these with a
+// branch around every row load; without it a part's rows come faster, its round trips stay:
+// block_sum_range).
 constexpr int kSplitMinUnit = 256 * 1024;
 // ... unless the batch is so small that parts of that size leave the workgroups with one or two
 // tiles each: then the part size is chosen so that the tiles come out as a whole number per

@@ -276,8 +276,9 @@ def _few_bags(split: bool, bags: int = 16, lookups: float = 20000.0) -> ModelSpe
     assert all(isinstance(s, SplitBagSchedule) for s, _ in fs)
     if not split:
         fs = [(BlockPerBagSchedule(s.meta, BLOCK_THREADS), p) for s, p in fs]
-    # 20 vector registers and 6.5 KB of LDS: eight workgroups per CU cover each other's waits
-    # for index chunks, partial sums and arrival counters (177 -> 156 us at four)
+    # 64 vector registers and 10.7 KB of LDS: eight workgroups per CU cover each other's waits
+    # for index chunks, partial sums and arrival counters (six: 16 bags of 20 000 lookups 72.2 -> 70.0
+    # us, 128 of 2 000 60.9 -> 63.3)
     return ModelSpec(wl, fs, 8)
 
 
