@@ -51,6 +51,8 @@ constexpr int kRedRow = kTileN + 4;
 // from this K on a step is 32 of K instead of 16
 constexpr int kLongK = 8192;
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -64,8 +66,9 @@ __device__ __forceinline__ Parts parts_of(const f32x4 v0, const f32x4 v1) {
     float x = i < 2 ? v0[2 * i] : v1[2 * i - 4], y = i < 2 ? v0[2 * i + 1] : v1[2 * i - 3];
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
-      uint32_t w;                                // (the compiler would round x once more to have it by itself)
-      asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(w) : "v"(x), "v"(y));
+      // (the builtin and not the instruction by hand: its result goes to a matrix instruction, and the
+      // compiler keeps the two wait states between them only where it knows the writer)
+      const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){x, y}, bf16x2));
       part[p][i] = w;
       x -= __uint_as_float(w << 16);
       y -= __uint_as_float(w & 0xffff0000u);

@@ -1,5 +1,7 @@
 """What ``RecomModel`` does around its MLP kernels, as far as that needs no GPU."""
 
+import os
+import re
 import shutil
 import subprocess
 import sys
@@ -104,3 +106,39 @@ else:
     (512, (4408, 512, 4096, 1024, 128), False)])
 def test_where_the_mlp_kernels_pay(batch, units, pays):
     assert kernels._pays(batch, units) is pays
+
+
+def _registers(operand):
+    m = re.fullmatch(r"v\[(\d+):(\d+)\]|v(\d+)", operand)
+    if not m:
+        return range(0)
+    return range(int(m[1]), int(m[2]) + 1) if m[1] else range(int(m[3]), int(m[3]) + 1)
+
+
+def test_mlp_kernels_wait_before_matrix_instructions(tmp_path):
+    """Two wait states lie between a vector instruction and a matrix instruction that reads its result; the
+    compiler sees to it except behind an instruction written in inline assembly."""
+    builder = BasicBuilder()
+    if not os.path.exists(builder.hipcc):
+        pytest.skip("no hipcc")
+    listing = tmp_path / "mlp.s"
+    flags = [f for f in builder.hip_flags if f not in ("-shared", "-fPIC")]
+    subprocess.run([builder.hipcc, *flags, "-O3", "--offload-device-only", "-S",
+                    f"{builder.csrc_dir}/mlp/recflex_mlp.hip", "-o", str(listing)], check=True, stderr=subprocess.DEVNULL)
+    products, since = 0, {}             # wait states since a vector instruction wrote the register
+    for line in listing.read_text().splitlines():
+        op, _, rest = line.split(";")[0].strip().partition(" ")
+        if op.endswith(":"):
+            since = {}
+        if not op or op.endswith(":") or op.startswith("."):
+            continue
+        operands = [o.strip() for o in rest.split(",")]
+        if op.startswith("v_mfma"):
+            products += 1
+            for operand in operands[1:]:
+                assert all(since.get(r, 2) >= 2 for r in _registers(operand)), line
+        states = int(operands[0], 0) + 1 if op == "s_nop" else 1
+        since = {r: n + states for r, n in since.items() if n + states < 2}
+        if op.startswith("v_") and not op.startswith("v_mfma"):
+            since.update(dict.fromkeys(_registers(operands[0]), 0))
+    assert products > 0
