@@ -37,19 +37,15 @@ __device__ __forceinline__ float relu(const float x) { return x <= 0.f ? 0.f : x
 // rounded, and a product of 16 of K rounds it once where two of K did.
 // The wavefronts split K among them, each with the whole tile to itself: no operand is taken apart twice
 // and they meet once, to add up their sums.  A step's operands go through the wavefront's own LDS (as
-// loaded: rows of 64 or 128 bytes; as read: a lane's eight of a row) and are taken apart in registers, in
+// loaded: rows of 64 bytes; as read: a lane's eight of a row) and are taken apart in registers, in
 // 400 ns of vector instructions beside 360 ns of products (64 x 64, 16 of K).
-// 512 rows, 4 408 -> 1 024 units: 57 us as fp32 products, 38 now (122 TFLOP/s).  What bounds it now is the
-// operands' way to the CU: 64 KB per round of the wavefronts in 1.9 us.  Asking for them two or three steps
-// ahead, products and vector instructions interleaved by hand, and LDS without bank conflicts left that
-// time where it is; steps of 32 (whole cache lines by one wavefront) took 9 % off it at 23 980 inputs
-// and added 4 % at 4 408, whose steps they divide less evenly.
+// 512 rows, 4 408 -> 1 024 units: 57 us as fp32 products, 38 now (122 TFLOP/s).  Asking for operands two or three
+// steps ahead, products and vector instructions interleaved by hand, and LDS without bank conflicts left that
+// time where it is.
 // N and K are multiples of 4 (valid): a vector of four units is whole or beyond N.
 // ---------------------------------------------------------------------------------------------
-constexpr int kTileN = 64, kThreads = 512, kWaves = kThreads / 64;
+constexpr int kTileN = 64, kThreads = 512, kWaves = kThreads / 64, kStep = 16;
 constexpr int kRedRow = kTileN + 4;
-// from this K on a step is 32 of K instead of 16
-constexpr int kLongK = 8192;
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -77,13 +73,13 @@ __device__ __forceinline__ Parts parts_of(const f32x4 v0, const f32x4 v1) {
   return {__builtin_bit_cast(bf16x8, part[0]), __builtin_bit_cast(bf16x8, part[1]), __builtin_bit_cast(bf16x8, part[2])};
 }
 
-// TM rows, steps of STEP of K
-template <int TM, int STEP>
+// TM rows
+template <int TM>
 __global__ void __launch_bounds__(kThreads)
 gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
         float *__restrict__ out, const int M, const int N, const int K, const int splits) {
-  constexpr int ROWS = TM + kTileN, LANES = STEP / 4, LOADS = ROWS * LANES / 64, WM = TM / 32, WN = kTileN / 32;
-  constexpr int ROW = STEP + 4;                  // LDS row, in floats: 16-byte reads of 8 rows spread over all banks
+  constexpr int ROWS = TM + kTileN, LANES = kStep / 4, LOADS = ROWS * LANES / 64, WM = TM / 32, WN = kTileN / 32;
+  constexpr int ROW = kStep + 4;                  // LDS row, in floats: 16-byte reads of 8 rows spread over all banks
   constexpr int LDS = kWaves * ROWS * ROW > kWaves * TM * kRedRow ? kWaves * ROWS * ROW : kWaves * TM * kRedRow;
   __shared__ float lds[LDS];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -94,7 +90,7 @@ gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *_
   // consecutive workgroups (one XCD each) take the units of the same rows: an XCD keeps to an
   // eighth of the weights, the larger operand
   const int m0 = tile / tiles_n * TM, n0 = tile % tiles_n * kTileN;
-  const int steps = (K + STEP - 1) / STEP;
+  const int steps = (K + kStep - 1) / kStep;
   const int per_split = (steps + splits - 1) / splits;
   const int first = split * per_split, last = min(steps, first + per_split);
 
@@ -109,14 +105,14 @@ gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *_
   }
   f32x4 next[LOADS];
   auto request = [&](const int step) {
-    const int k = min(step * STEP, K - 4 - col);      // stays within the row
+    const int k = min(step * kStep, K - 4 - col);      // stays within the row
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) next[i] = *reinterpret_cast<const f32x4 *>(src[i] + k);
   };
   float *mine = lds + wave * (ROWS * ROW);
   auto put = [&](const int step) {
-    if (step * STEP + STEP > K) {              // the last step's surplus
-      const bool in = step * STEP + col < K;
+    if (step * kStep + kStep > K) {              // the last step's surplus
+      const bool in = step * kStep + col < K;
 #pragma unroll
       for (int i = 0; i < LOADS; ++i)
 #pragma unroll
@@ -136,8 +132,8 @@ gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *_
       for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
   // lane (i, h) of a 32x32x16 product holds row i at eight values of k, one set per h
   const float *frag = mine + (lane & 31) * ROW + (lane >> 5) * 8;
-  auto operand = [&](const int block, const int sub) {
-    const float *at = frag + block * 32 * ROW + sub * 16;
+  auto operand = [&](const int block) {
+    const float *at = frag + block * 32 * ROW;
     return parts_of(*reinterpret_cast<const f32x4 *>(at), *reinterpret_cast<const f32x4 *>(at + 4));
   };
   if (first + wave < last) request(first + wave);
@@ -148,24 +144,21 @@ gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *_
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    Parts b[WN];
 #pragma unroll
-    for (int sub = 0; sub < STEP / 16; ++sub) {
-      Parts b[WN];
+    for (int n = 0; n < WN; ++n) b[n] = operand(WM + n);
 #pragma unroll
-      for (int n = 0; n < WN; ++n) b[n] = operand(WM + n, sub);
+    for (int m = 0; m < WM; ++m) {
+      const Parts a = operand(m);
 #pragma unroll
-      for (int m = 0; m < WM; ++m) {
-        const Parts a = operand(m, sub);
-#pragma unroll
-        for (int n = 0; n < WN; ++n) {             // smallest first
-          f32x16 c = acc[m][n];
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.middle, b[n].middle, c, 0, 0, 0);
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.high, b[n].low, c, 0, 0, 0);
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.low, b[n].high, c, 0, 0, 0);
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.high, b[n].middle, c, 0, 0, 0);
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.middle, b[n].high, c, 0, 0, 0);
-          acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.high, b[n].high, c, 0, 0, 0);
-        }
+      for (int n = 0; n < WN; ++n) {               // smallest first
+        f32x16 c = acc[m][n];
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.middle, b[n].middle, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.high, b[n].low, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.low, b[n].high, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.high, b[n].middle, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.middle, b[n].high, c, 0, 0, 0);
+        acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.high, b[n].high, c, 0, 0, 0);
       }
     }
     // ... and these reads before the next step's writes
@@ -202,7 +195,7 @@ gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *_
       if (!(size <= 3.4028234e38f) || (size < 1e-25f && size > 0.f)) {
         const float *xs = x + static_cast<int64_t>(m0 + row) * K, *ws = w + static_cast<int64_t>(n0 + unit + j) * K;
         float t = 0.f;
-        for (int k = first * STEP; k < min(K, last * STEP); ++k) t = fmaf(xs[k], ws[k], t);
+        for (int k = first * kStep; k < min(K, last * kStep); ++k) t = fmaf(xs[k], ws[k], t);
         sum[j] = t;
       }
     }
@@ -353,7 +346,7 @@ Plan plan_of(const int M, const int N, const int K, const int cus, const bool fe
   double best_us = 1e30;
   for (int rows = 32; rows <= 64; rows += 32) {
     const int64_t tiles = static_cast<int64_t>(ceil_div(M, rows)) * ceil_div(N, kTileN);
-    const int chunks = ceil_div(K, kWaves * 16);
+    const int chunks = ceil_div(K, kWaves * kStep);
     for (int s = 1; s <= RECFLEX_MLP_MAX_SPLITS && s <= chunks; ++s) {
       const int per_split = ceil_div(chunks, s);
       if (static_cast<int64_t>(per_split) * (s - 1) >= chunks) continue;            // an empty split
@@ -437,10 +430,8 @@ extern "C" int recflex_mlp_forward(const recflex_mlp_args *a) {
     float *out = direct ? a->hidden[l] : a->workspace;
     void *args[] = {&x, &w, &bias, &out, &M, &N, &K, &splits};
     const int64_t tiles = static_cast<int64_t>(ceil_div(M, plan.rows)) * ceil_div(N, kTileN);
-    const void *kernel = K < kLongK ? (plan.rows == 32 ? reinterpret_cast<const void *>(&gemm_nt<32, 16>)
-                                                       : reinterpret_cast<const void *>(&gemm_nt<64, 16>))
-                                    : (plan.rows == 32 ? reinterpret_cast<const void *>(&gemm_nt<32, 32>)
-                                                       : reinterpret_cast<const void *>(&gemm_nt<64, 32>));
+    const void *kernel = plan.rows == 32 ? reinterpret_cast<const void *>(&gemm_nt<32>)
+                                         : reinterpret_cast<const void *>(&gemm_nt<64>);
     e = launch(kernel, tiles * splits, kThreads, args);
     if (e != hipSuccess) return static_cast<int>(e);
     if (!direct && !feeds_tail) {
