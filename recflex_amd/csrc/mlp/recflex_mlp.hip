@@ -30,18 +30,22 @@ __device__ __forceinline__ float relu(const float x) { return x <= 0.f ? 0.f : x
 // ---------------------------------------------------------------------------------------------
 // gemm_nt: a workgroup of eight wavefronts computes a tile of 32 or 64 rows x 64 units of fp32 products on
 // the bf16 matrix cores: every operand is the sum of three bf16 numbers (8 + 8 + 8 bits with their signs
-// hold the 24 exactly), and of their nine products the six are formed that reach the last bit (the others
-// are below 2^-26 of the product).  16 of K take 6 x 15 ns of a SIMD that way and 8 x 27 ns as fp32 products.
-// Errors against 64 bits, 2-norm, first hidden layer, 4 408 inputs: 2.5e-7 and 5.7e-7 at 512 rows, 1.4e-7 and
-// 1.8e-7 at one (23 980 inputs: 4.7e-7 and 6.9e-7, 2.7e-7 and 3.6e-7): what counts is how often a sum is
-// rounded, and a product of 16 of K rounds it once where two of K did.
+// hold the 24 exactly), and of their nine products all but that of the low parts (at most 2^-34) are formed.
+// Those of the high parts have a sum of their own, in which the others would be cut off: a matrix instruction
+// rounds down what it adds (measured, by up to 0.98 units in the last place).  So one product alone comes out as
+// fp32 rounds it, and long sums are rounded less often than fp32 products would be.
+// Errors against 64 bits, 2-norm, first hidden layer, as fp32 products and so: 4 408 inputs, 512 rows 5.9e-7 and
+// 1.1e-7, one row 2.0e-7 and 1.0e-7; 23 980 inputs, 512 rows 6.9e-7 and 2.3e-7; one active input per row 2.5e-8
+// both, at most 6.0e-8 both.  (With six of the products and one sum: 2.6e-7, 1.4e-7, 6.6e-7, and 3.3e-8, at most
+// 1.6e-7, for 59 us of the whole MLP at 4 408 inputs and 512 rows where this takes 64.)
 // The wavefronts split K among them, each with the whole tile to itself: no operand is taken apart twice
-// and they meet once, to add up their sums.  A step's operands go through the wavefront's own LDS (as
-// loaded: rows of 64 bytes; as read: a lane's eight of a row) and are taken apart in registers, in
-// 400 ns of vector instructions beside 360 ns of products (64 x 64, 16 of K).
-// 512 rows, 4 408 -> 1 024 units: 57 us as fp32 products, 38 now (122 TFLOP/s).  Asking for operands two or three
-// steps ahead, products and vector instructions interleaved by hand, and LDS without bank conflicts left that
-// time where it is.
+// and they meet once, to add up their sums.  A step's operands (16 of K) go through the wavefront's own LDS (as
+// loaded: rows of 64 bytes; as read: a lane's eight of a row) and are taken apart in registers.
+// 512 rows, 4 408 -> 1 024 units: 57 us as fp32 products, 46 and 5 for the sum of two splits so.  The whole MLP at 512
+// rows, 4 408 and 23 980 inputs: 68 and 240 us, 65 and 235 so.
+// Bound by the two kinds of instructions, which hardly overlap: the matrix cores are busy 35 % of the time and the
+// vector units 38 %, of a wavefront's time 15 % goes to waiting for memory (4 408 inputs, 512 rows).  Without the
+// conversions the MLP takes 61 us instead of 66, without the loads 58, with three products of the eight 54.
 // N and K are multiples of 4 (valid): a vector of four units is whole or beyond N.
 // ---------------------------------------------------------------------------------------------
 constexpr int kTileN = 64, kThreads = 512, kWaves = kThreads / 64, kStep = 16;
@@ -123,13 +127,14 @@ gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *_
       *reinterpret_cast<f32x4 *>(mine + (i * 64 + lane) / LANES * ROW + col) = next[i];
   };
 
-  f32x16 acc[WM][WN];
+  // the products of the high parts, and the others
+  f32x16 acc[WM][WN], rest[WM][WN];
 #pragma unroll
   for (int m = 0; m < WM; ++m)
 #pragma unroll
     for (int n = 0; n < WN; ++n)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[m][n][r] = 0.f;
+      for (int r = 0; r < 16; ++r) acc[m][n][r] = rest[m][n][r] = 0.f;
   // lane (i, h) of a 32x32x16 product holds row i at eight values of k, one set per h
   const float *frag = mine + (lane & 31) * ROW + (lane >> 5) * 8;
   auto operand = [&](const int block) {
@@ -144,22 +149,32 @@ gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *_
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    Parts b[WN];
+    Parts a[WM], b[WN];
 #pragma unroll
     for (int n = 0; n < WN; ++n) b[n] = operand(WM + n);
 #pragma unroll
-    for (int m = 0; m < WM; ++m) {
-      const Parts a = operand(m);
+    for (int m = 0; m < WM; ++m) a[m] = operand(m);
+    auto add = [](f32x16 &sum, const bf16x8 p, const bf16x8 q) {
+      sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p, q, sum, 0, 0, 0);
+    };
 #pragma unroll
-      for (int n = 0; n < WN; ++n) {               // smallest first
-        f32x16 c = acc[m][n];
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.middle, b[n].middle, c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.high, b[n].low, c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.low, b[n].high, c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.high, b[n].middle, c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.middle, b[n].high, c, 0, 0, 0);
-        acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.high, b[n].high, c, 0, 0, 0);
-      }
+    for (int m = 0; m < WM; ++m) {             // smallest first, neighbours in the row on different sums
+#pragma unroll
+      for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].middle, b[n].low);
+#pragma unroll
+      for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].low, b[n].middle);
+#pragma unroll
+      for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].middle, b[n].middle);
+#pragma unroll
+      for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].high, b[n].low);
+#pragma unroll
+      for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].low, b[n].high);
+#pragma unroll
+      for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].high, b[n].middle);
+#pragma unroll
+      for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].middle, b[n].high);
+#pragma unroll
+      for (int n = 0; n < WN; ++n) add(acc[m][n], a[m].high, b[n].high);
     }
     // ... and these reads before the next step's writes
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -176,7 +191,7 @@ gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *_
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int row = m * 32 + 8 * (r / 4) + 4 * (lane >> 5) + r % 4;
-        lds[(wave * TM + row) * kRedRow + n * 32 + (lane & 31)] = acc[m][n][r];
+        lds[(wave * TM + row) * kRedRow + n * 32 + (lane & 31)] = acc[m][n][r] + rest[m][n][r];
       }
   __syncthreads();
   for (int at = tid; at < TM * (kTileN / 4); at += kThreads) {
@@ -336,10 +351,12 @@ tail(const float *__restrict__ parts, const int splits, const float *__restrict_
 
 int ceil_div(const int64_t a, const int64_t b) { return static_cast<int>((a + b - 1) / b); }
 
-// How a layer is cut: tiles of 32 or 64 rows, and its K into splits.  What a CU takes for a chunk (16 of K for
-// every wavefront) with all CUs at work: 1.2 us (32 rows) and 1.9 us (64 rows), at 256, 512 and 2 048 rows
-// alike; another 3 us for the first loads and the last sums.  Splits cost their traffic and, ahead of any
-// layer but the tail, a kernel that adds them up.
+// How a layer is cut: tiles of 32 or 64 rows, and its K into splits.  A CU takes 1.4 us (32 rows) or 2.4 us (64 rows)
+// for a chunk (16 of K for every wavefront) with all CUs at work, and 3 us for the first loads and the last sums.
+// Splits cost their traffic and, ahead of any layer but the tail, a kernel that adds them up; that traffic is priced
+// high, so the chunks are priced lower than they measure, in their proportion: over 1 to 512 rows and the first
+// layers 512, 1 000, 4 408, 12 000, 23 980 x 1 024 to 8 192 the better number of rows is taken to within 3 % of the
+// whole MLP (with 1.4 and 2.4 here, 4 408 x 1 024 and 512 rows would go unsplit: 69 us instead of 65).
 struct Plan { int rows, splits; };
 Plan plan_of(const int M, const int N, const int K, const int cus, const bool feeds_tail) {
   Plan best{32, 1};

@@ -9,8 +9,7 @@ from recflex_amd import mlp as kernels
 
 pytestmark = pytest.mark.gpu
 
-# fp32 sums in blocks of at most 128 terms, blocks and splits added in order: errors of a few eps per
-# layer in the 2-norm
+# fp32 sums in one order or another of up to some hundred partial sums: errors of a few eps per layer in the 2-norm
 REL = 1e-6
 GRAD_REL = 1e-5
 
@@ -159,8 +158,7 @@ def test_mlp_leaves_large_products_to_the_library():
         assert got is not None and rel(got, mlp.double()(x[:kernels.ANY_WIDTH_BATCH].double())) < REL
 
 
-# what three bf16 numbers per operand can and cannot hold: numbers whose low parts are subnormal, numbers near
-# the largest; K of the long steps and its remainders, tiles of 64 rows without splits
+# tiny and huge inputs; long K and its remainders, tiles of 64 rows without splits
 @pytest.mark.parametrize("units, batch, scale", [
     ((260, 96, 32), 70, 1e-36), ((260, 96, 32), 70, 1e-30), ((260, 96, 32), 70, 1e30), ((8196, 64, 16), 40, 1.),
     ((8224, 100, 16), 65, 1.), ((1000, 1024, 128), 1025, 1.)])
@@ -173,3 +171,29 @@ def test_mlp_products_of_parts(units, batch, scale):
     ws, bs = [m.weight.detach() for m in mlp[::2]], [m.bias.detach() for m in mlp[::2]]
     hidden = kernels._run(x, ws, bs, True)[1][0]
     assert rel(hidden / scale, torch.relu(x.double() @ ws[0].double().t()) / scale) < REL
+
+
+def first_hidden(x, w, b=None):
+    """The first hidden layer of an MLP whose first weights are ``w``, as the kernels form it."""
+    units = (w.shape[1], w.shape[0], 16)
+    mlp = build(units)
+    ws, bs = [m.weight.detach() for m in mlp[::2]], [m.bias.detach() for m in mlp[::2]]
+    ws[0], bs[0] = w, torch.zeros(w.shape[0], device="cuda") if b is None else b
+    return kernels._run(x, ws, bs, True)[1][0]
+
+
+# with and without splits of K, tiles of 32 and of 64 rows
+SHAPES = [(70, 260, 96), (33, 4408, 64), (512, 4408, 1024), (1025, 1000, 1024)]
+
+
+@pytest.mark.parametrize("batch, inputs, units", SHAPES)
+def test_mlp_single_products_are_fp32_products(batch, inputs, units):
+    """One active input per row: every sum is one product.  Rounded to fp32 it is off by up to 2^-24 of itself; what is
+    cut off ahead of that (parts of it, seven times by up to 2^-30, once by 2^-34) is less than an eighth of this."""
+    print("[case] mlp single products", batch, inputs, units, flush=True)
+    torch.manual_seed(1)
+    at = torch.randint(0, inputs, (batch,), device="cuda")
+    value, w = torch.randn(batch, device="cuda"), torch.randn(units, inputs, device="cuda")
+    x = torch.zeros(batch, inputs, device="cuda").scatter_(1, at[:, None], value[:, None])
+    want = torch.relu(value.double()[:, None] * w.double().t()[at])
+    assert bool(((first_hidden(x, w) - want).abs() <= 2 ** -24 * (1 + 1 / 8) * want).all())
