@@ -1,13 +1,13 @@
 // The MLP behind the fused embedding (RecomModel): Linear + ReLU layers and a last Linear to one
-// unit with a sigmoid, all in fp32 on the matrix cores.
+// unit with a sigmoid, to fp32's precision on the matrix cores.
 //
 // Reference counterpart: the nn.Sequential of RecFlex/rec_modules.py:150-179.
 //
 // A batch of 512 through 4408 -> 1024 -> 256 -> 128 -> 1 is 5 GFLOP, 32 us at the rate a large fp32
 // product reaches here (154 TFLOP/s), and most of it the first layer.  Library products with
-// activations between them are eight launches and, one after the other in a graph, 75 us; batches
-// of 1, 64 and 256 take 49, 50 and 86 us.  Here they are three launches (four where the first
-// layer's K is split) and 54 us; 19, 26 and 39 us for the smaller batches:
+// activations between them are eight launches and, one after the other in a graph, 77 us; batches
+// of 1, 64 and 256 take 55, 54 and 89 us.  Here they are three launches (four where the first
+// layer's K is split) and 64 us; 25, 31 and 46 us for the smaller batches:
 //   gemm_nt    a layer: X [M, K] times W [N, K] transposed, bias and ReLU on the way out;
 //   tail       the last hidden layer, its ReLU, the dot product with the last layer's row and
 //              the sigmoid, and ahead of them the sum of the K-splits of the layer before.
@@ -50,20 +50,29 @@ __device__ __forceinline__ float relu(const float x) { return x <= 0.f ? 0.f : x
 // ---------------------------------------------------------------------------------------------
 constexpr int kTileN = 64, kThreads = 512, kWaves = kThreads / 64, kStep = 16;
 constexpr int kRedRow = kTileN + 4;
+// Of numbers between these (and zeros) the three parts are exact and no product of parts leaves fp32's range or nears
+// its subnormals.  A step with others is left out and taken as fp32 products at the end: at 4 408 inputs and 512
+// rows 98 us for the MLP with such a number in every step, 65 without (fp32 products throughout: 68).  The question
+// costs a vector instruction per number, and three where there are zeros.
+constexpr float kSmallest = 0x1p-60f, kLargest = 0x1p60f;
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// eight fp32 numbers as high + middle + low, exactly (numbers beyond the largest bf16 become infinite,
-// and their products with the other parts NaN: see below)
+struct Eight {
+  f32x4 v[2];
+  __device__ __forceinline__ float operator[](const int i) const { return v[i / 4][i % 4]; }
+};
+
+// eight fp32 numbers as high + middle + low
 struct Parts { bf16x8 high, middle, low; };
-__device__ __forceinline__ Parts parts_of(const f32x4 v0, const f32x4 v1) {
+__device__ __forceinline__ Parts parts_of(const Eight &v) {
   u32x4 part[3];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    float x = i < 2 ? v0[2 * i] : v1[2 * i - 4], y = i < 2 ? v0[2 * i + 1] : v1[2 * i - 3];
+    float x = v[2 * i], y = v[2 * i + 1];
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
       // (the builtin and not the instruction by hand: its result goes to a matrix instruction, and the
@@ -77,13 +86,20 @@ __device__ __forceinline__ Parts parts_of(const f32x4 v0, const f32x4 v1) {
   return {__builtin_bit_cast(bf16x8, part[0]), __builtin_bit_cast(bf16x8, part[1]), __builtin_bit_cast(bf16x8, part[2])};
 }
 
+// the wavefront's own LDS: what it wrote before what it reads next, and the other way round
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // TM rows
 template <int TM>
 __global__ void __launch_bounds__(kThreads)
 gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
         float *__restrict__ out, const int M, const int N, const int K, const int splits) {
   constexpr int ROWS = TM + kTileN, LANES = kStep / 4, LOADS = ROWS * LANES / 64, WM = TM / 32, WN = kTileN / 32;
-  constexpr int ROW = kStep + 4;                  // LDS row, in floats: 16-byte reads of 8 rows spread over all banks
+  constexpr int ROW = kStep + 4;                 // LDS row, in floats: 16-byte reads of 8 rows spread over all banks
   constexpr int LDS = kWaves * ROWS * ROW > kWaves * TM * kRedRow ? kWaves * ROWS * ROW : kWaves * TM * kRedRow;
   __shared__ float lds[LDS];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -109,11 +125,12 @@ gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *_
   }
   f32x4 next[LOADS];
   auto request = [&](const int step) {
-    const int k = min(step * kStep, K - 4 - col);      // stays within the row
+    const int k = min(step * kStep, K - 4 - col);     // stays within the row
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) next[i] = *reinterpret_cast<const f32x4 *>(src[i] + k);
   };
   float *mine = lds + wave * (ROWS * ROW);
+  // what was requested, to LDS; whether the parts hold all of it, the same in every lane
   auto put = [&](const int step) {
     if (step * kStep + kStep > K) {              // the last step's surplus
       const bool in = step * kStep + col < K;
@@ -122,12 +139,30 @@ gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *_
 #pragma unroll
         for (int j = 0; j < 4; ++j) next[i][j] = in ? next[i][j] : 0.f;
     }
+    float least = kLargest, most = 0.f;
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i)
+    for (int i = 0; i < LOADS; ++i) {
       *reinterpret_cast<f32x4 *>(mine + (i * 64 + lane) / LANES * ROW + col) = next[i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        least = fminf(least, fabsf(next[i][j]));
+        most = __builtin_elementwise_maximum(most, fabsf(next[i][j]));        // (a NaN stays)
+      }
+    }
+    bool fits = most < kLargest;
+    if (__builtin_amdgcn_ballot_w64(!(least >= kSmallest)) != 0) {            // zeros, or small numbers
+      unsigned lowest = ~0u;
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)                                           // (a zero becomes the largest)
+          lowest = min(lowest, (__float_as_uint(next[i][j]) << 1) - 1u);
+      fits = fits && lowest >= (__float_as_uint(kSmallest) << 1) - 1u;
+    }
+    return __builtin_amdgcn_ballot_w64(!fits) == 0;
   };
 
-  // the products of the high parts, and the others
+  // the products of the high parts (and fp32 products), and the others
   f32x16 acc[WM][WN], rest[WM][WN];
 #pragma unroll
   for (int m = 0; m < WM; ++m)
@@ -135,52 +170,70 @@ gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *_
     for (int n = 0; n < WN; ++n)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[m][n][r] = rest[m][n][r] = 0.f;
-  // lane (i, h) of a 32x32x16 product holds row i at eight values of k, one set per h
+  // lane (i, h) of a 32x32x16 product holds row i at eight values of k, one set per h (of eight 32x32x2 products
+  // one value each)
   const float *frag = mine + (lane & 31) * ROW + (lane >> 5) * 8;
   auto operand = [&](const int block) {
     const float *at = frag + block * 32 * ROW;
-    return parts_of(*reinterpret_cast<const f32x4 *>(at), *reinterpret_cast<const f32x4 *>(at + 4));
+    return Eight{*reinterpret_cast<const f32x4 *>(at), *reinterpret_cast<const f32x4 *>(at + 4)};
   };
+  bool left_out = false;
   if (first + wave < last) request(first + wave);
   for (int step = first + wave; step < last; step += kWaves) {
-    put(step);
+    const bool fits = put(step);
     if (step + kWaves < last) request(step + kWaves);
-    // the wavefront's own LDS: its writes before its reads
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    Parts a[WM], b[WN];
+    wave_lds_fence();
+    if (__builtin_expect(fits, 1)) {
+      Parts a[WM], b[WN];
 #pragma unroll
-    for (int n = 0; n < WN; ++n) b[n] = operand(WM + n);
+      for (int n = 0; n < WN; ++n) b[n] = parts_of(operand(WM + n));
 #pragma unroll
-    for (int m = 0; m < WM; ++m) a[m] = operand(m);
-    auto add = [](f32x16 &sum, const bf16x8 p, const bf16x8 q) {
-      sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p, q, sum, 0, 0, 0);
-    };
+      for (int m = 0; m < WM; ++m) a[m] = parts_of(operand(m));
+      auto add = [](f32x16 &sum, const bf16x8 p, const bf16x8 q) {
+        sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p, q, sum, 0, 0, 0);
+      };
 #pragma unroll
-    for (int m = 0; m < WM; ++m) {             // smallest first, neighbours in the row on different sums
+      for (int m = 0; m < WM; ++m) {             // smallest first, neighbours in the row on different sums
 #pragma unroll
-      for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].middle, b[n].low);
+        for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].middle, b[n].low);
 #pragma unroll
-      for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].low, b[n].middle);
+        for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].low, b[n].middle);
 #pragma unroll
-      for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].middle, b[n].middle);
+        for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].middle, b[n].middle);
 #pragma unroll
-      for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].high, b[n].low);
+        for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].high, b[n].low);
 #pragma unroll
-      for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].low, b[n].high);
+        for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].low, b[n].high);
 #pragma unroll
-      for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].high, b[n].middle);
+        for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].high, b[n].middle);
 #pragma unroll
-      for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].middle, b[n].high);
+        for (int n = 0; n < WN; ++n) add(rest[m][n], a[m].middle, b[n].high);
 #pragma unroll
-      for (int n = 0; n < WN; ++n) add(acc[m][n], a[m].high, b[n].high);
+        for (int n = 0; n < WN; ++n) add(acc[m][n], a[m].high, b[n].high);
+      }
+    } else {
+      left_out = true;
     }
-    // ... and these reads before the next step's writes
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_fence();
   }
+  // The steps left out: infinities, NaN, numbers beyond kSmallest and kLargest.
+  if (__builtin_expect(left_out, 0))
+    for (int step = first + wave; step < last; step += kWaves) {
+      request(step);
+      if (put(step)) continue;
+      wave_lds_fence();
+#pragma unroll
+      for (int m = 0; m < WM; ++m) {
+        const Eight a = operand(m);
+#pragma unroll
+        for (int n = 0; n < WN; ++n) {
+          const Eight b = operand(WM + n);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], b[j], acc[m][n], 0, 0, 0);
+        }
+      }
+      wave_lds_fence();
+    }
 
   // the wavefronts' shares of K, added in order
   __syncthreads();
@@ -201,19 +254,6 @@ gemm_nt(const float *__restrict__ x, const float *__restrict__ w, const float *_
     for (int g = 1; g < kWaves; ++g)
       sum += *reinterpret_cast<const f32x4 *>(lds + (g * TM + row) * kRedRow + unit);
     if (m0 + row >= M || n0 + unit >= N) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      // An infinity's parts are infinity and NaN, so its products are NaN where fp32 has an infinity, and of
-      // numbers below 1e-33 the low part is lost among the subnormals: a sum that such operands may have
-      // made (not finite, or all but zero) is formed again, term by term.
-      const float size = fabsf(sum[j]);
-      if (!(size <= 3.4028234e38f) || (size < 1e-25f && size > 0.f)) {
-        const float *xs = x + static_cast<int64_t>(m0 + row) * K, *ws = w + static_cast<int64_t>(n0 + unit + j) * K;
-        float t = 0.f;
-        for (int k = first * kStep; k < min(K, last * kStep); ++k) t = fmaf(xs[k], ws[k], t);
-        sum[j] = t;
-      }
-    }
     float *dst = out + (static_cast<int64_t>(split) * M + m0 + row) * N + n0 + unit;
     if (bias) {
 #pragma unroll

@@ -33,13 +33,15 @@ MAX_LAYERS = 8                      # RECFLEX_MLP_MAX_LAYERS
 TAIL_MAX_UNITS = 128                # RECFLEX_MLP_TAIL_MAX_UNITS
 TAIL_MAX_INPUTS = 1024              # RECFLEX_MLP_TAIL_MAX_INPUTS
 # Where the kernels serve, against the modules (in us; both in a graph, where the library's launches cost
-# least).  Up to 256 rows always: the library's products take 1.1 to 5 times as long as these.  Beyond, up to
-# 512 rows: 1024, 256, 128 units on 4 408 inputs, 384 / 512 rows 52 / 57 against 74 / 76, on 23 980 inputs 162 /
-# 197 against 364 / 269, on 512 inputs 24 / 25 against 42 / 43; wider layers gain less (4096, 512, 128 on 4 408
-# inputs, 512 rows, 20 GFLOP: 169 against 185) and lose with much to multiply (8192, 512, 128 on 23 980 inputs,
-# 384 rows, 151 GFLOP: 1 185 against 1 154): beyond 8 GFLOP they are left to the modules.  Beyond 512 rows the
-# modules serve, though up to some 80 GFLOP these would be the faster ones there too (1024, 256, 128 on 4 408
-# inputs, 1 024 / 2 048 rows 88 / 158 against 109 / 174, on 23 980 inputs 381 / 723 against 415 / 734).
+# least).  Up to 256 rows: the library's products take 1.1 to 5 times as long as these (except where there is as much
+# to multiply as in 8192, 512, 128 units on 23 980 inputs, 256 rows, 103 GFLOP: 994 against 857).  Beyond, up to 512
+# rows: 1024, 256, 128 units on 4 408 inputs, 384 / 512 rows 57 / 65 against 76 / 77, on 23 980 inputs 183 / 235 against
+# 360 / 252, on 512 inputs 28 / 29 against 45 / 46; wider layers gain less or lose (4 408 inputs: 2048, 512, 128 units,
+# 384 rows, 8 GFLOP, 96 to 104 against 97 to 101; 4096, 512, 128, 300 / 512 rows, 12 / 21 GFLOP, 149 / 191 against 144 /
+# 185; 8192, 512, 128, 512 rows, 41 GFLOP, 364 against 324): beyond 8 GFLOP they are left to the modules (not without
+# exceptions: 1536, 512, 128 on 23 980 inputs, 512 rows, 346 against 687).  Beyond 512 rows the modules serve: 1024,
+# 256, 128 on 4 408 inputs, 700 / 1 024 / 2 048 rows 86 / 103 / 189 against 93 / 110 / 176, on 23 980 inputs 328 / 451 /
+# 899 against 683 / 379 / 720.
 MAX_BATCH = 512
 ANY_WIDTH_BATCH = 256
 NARROW_UNITS = 1024

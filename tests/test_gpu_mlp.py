@@ -161,7 +161,7 @@ def test_mlp_leaves_large_products_to_the_library():
 # tiny and huge inputs; long K and its remainders, tiles of 64 rows without splits
 @pytest.mark.parametrize("units, batch, scale", [
     ((260, 96, 32), 70, 1e-36), ((260, 96, 32), 70, 1e-30), ((260, 96, 32), 70, 1e30), ((8196, 64, 16), 40, 1.),
-    ((8224, 100, 16), 65, 1.), ((1000, 1024, 128), 1025, 1.)])
+    ((8224, 100, 16), 65, 1.), ((1000, 1024, 128), 1025, 1.), ((4408, 1024, 128), 512, 1e-30)])
 def test_mlp_products_of_parts(units, batch, scale):
     print("[case] mlp", units, batch, scale, flush=True)
     mlp = build(units)
@@ -197,3 +197,34 @@ def test_mlp_single_products_are_fp32_products(batch, inputs, units):
     x = torch.zeros(batch, inputs, device="cuda").scatter_(1, at[:, None], value[:, None])
     want = torch.relu(value.double()[:, None] * w.double().t()[at])
     assert bool(((first_hidden(x, w) - want).abs() <= 2 ** -24 * (1 + 1 / 8) * want).all())
+
+
+@pytest.mark.parametrize("inputs_scale, weights_scale", [(1e-34, 1e12), (1e-36, 1e20), (1e-37, 1e30), (1e20, 1e-36)])
+def test_mlp_tiny_numbers_times_large_ones(inputs_scale, weights_scale):
+    """Numbers whose parts would be subnormal, in products that are not."""
+    print("[case] mlp", inputs_scale, weights_scale, flush=True)
+    torch.manual_seed(2)
+    x, w = torch.randn(70, 260, device="cuda") * inputs_scale, torch.randn(96, 260, device="cuda") * weights_scale
+    scale = inputs_scale * weights_scale
+    assert rel(first_hidden(x, w) / scale, torch.relu(x.double() @ w.double().t()) / scale) < REL
+
+
+@pytest.mark.parametrize("batch, inputs, units", SHAPES)
+def test_mlp_infinities_stay_infinities(batch, inputs, units):
+    """Rows with an infinity of either sign, a NaN, numbers between the largest bf16 and the largest fp32."""
+    print("[case] mlp infinities", batch, inputs, units, flush=True)
+    torch.manual_seed(3)
+    x, w = torch.randn(batch, inputs, device="cuda"), torch.randn(units, inputs, device="cuda") * 1e-3
+    x[3, 5], x[7, inputs - 1], x[11, 0], x[13, 2] = float("inf"), -float("inf"), float("nan"), 3.4e38
+    x[20, 1], x[20, 2] = float("inf"), -float("inf")
+    got = first_hidden(x, w)
+    want = torch.relu(x.double() @ w.double().t())
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isposinf(got), torch.isposinf(want))
+    for row in (3, 7):                  # infinite or, behind the ReLU, zero
+        assert bool((torch.isposinf(got[row]) | (got[row] == 0)).all()) and bool(torch.isposinf(got[row]).any())
+    finite = torch.isfinite(want)
+    for row in (13, 0):
+        assert bool(finite[row].all()) and rel(got[row], want[row]) < REL
+    rest = finite.all(1)
+    rest[13] = False
+    assert rel(got[rest], want[rest]) < REL
