@@ -77,24 +77,18 @@ template <int STRIDE> __device__ __forceinline__ int row_offset(const int r) {
   }
 }
 
-// A window of a table as a buffer resource: rows are loaded by 32-bit byte offsets, one register where a
+// The first 4 GB of a table as a buffer resource: rows are loaded by 32-bit byte offsets, one register where a
 // 64-bit address takes two and several instructions, and a lane without a lookup passes row -1, which
-// lies beyond the window: it reads zeros and touches no memory.  Window w starts at row w * ROWS (a
-// table of less than 4 GB has one).
+// lies beyond the window: it reads zeros and touches no memory.  A round with a row beyond the window (row ROWS
+// and on) is loaded by 64-bit addresses (load_far).
 template <typename R> struct RowWindow {
   static constexpr unsigned SLACK = R::STRIDE > 4096 ? R::STRIDE : 4096;
   static constexpr int ROWS = static_cast<int>((0x100000000ull - SLACK) / R::STRIDE);
   __amdgpu_buffer_rsrc_t rsrc;
 
-  __device__ __forceinline__ RowWindow(const char *table, const int w)
-      : rsrc(__builtin_amdgcn_make_buffer_rsrc(
-            const_cast<char *>(table) + static_cast<int64_t>(w) * ROWS * R::STRIDE, 0,
-            static_cast<int>(static_cast<unsigned>(ROWS) * R::STRIDE), 0x00020000)) {}
-  // row r of the table as a row of window w (-1: not in it)
-  static __device__ __forceinline__ int local(const int r, const int w) {
-    const int l = r - w * ROWS;
-    return r >= 0 && l >= 0 && l < ROWS ? l : -1;
-  }
+  __device__ __forceinline__ explicit RowWindow(const char *table)
+      : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(table), 0,
+                                               static_cast<int>(static_cast<unsigned>(ROWS) * R::STRIDE), 0x00020000)) {}
   template <int VB> __device__ __forceinline__ Vec<VB> load(const int at, const int plus) const {
     Vec<VB> r;
     if constexpr (VB == 16) {
@@ -108,7 +102,23 @@ template <typename R> struct RowWindow {
     }
     return r;
   }
+  // whether a lane of the wavefront holds a row beyond the window, the same in every lane
+  static __device__ __forceinline__ bool beyond(const int row) {
+    return __builtin_amdgcn_ballot_w64(row >= ROWS) != 0;
+  }
 };
+
+// VB bytes of row r at byte `at`, wherever it lies; a lane without a lookup (-1) has its table's first row, whose
+// values zero_far takes out again behind the round's last load
+template <typename R, int VB>
+__device__ __forceinline__ Vec<VB> load_far(const char *__restrict__ table, const int r, int at) {
+  asm volatile("" : "+v"(at));                  // (or the addresses' fixed parts are kept in registers all along)
+  return load_vec<VB>(table + static_cast<int64_t>(max(r, 0)) * R::STRIDE + at);
+}
+template <int VB> __device__ __forceinline__ void zero_far(Vec<VB> &v, const int r) {
+#pragma unroll
+  for (int i = 0; i < VB / 4; ++i) v.w[i] = r < 0 ? 0u : v.w[i];
+}
 
 // scale (low half) and bias (high half) of an I8 row, stored as two fp16 right after the codes: taken
 // apart where they are used, so that a row's loads do not wait for them

@@ -157,12 +157,6 @@ __device__ __forceinline__ int wave_max(int v) {
   return __builtin_amdgcn_readlane(v, 63);
 }
 
-// How many windows of the table (RowWindow) the rows that a wavefront holds lie in, the same in every lane.
-template <typename R> __device__ __forceinline__ int windows_of(const int row) {
-  if (__builtin_amdgcn_ballot_w64(row >= RowWindow<R>::ROWS) == 0) return 1;
-  return wave_max(row >= 0 ? row / RowWindow<R>::ROWS : 0) + 1;
-}
-
 // ---------------------------------------------------------------------------------------------
 // sum_lookups: the lookups [beg[i], end[i]) of UB bags per team of X*Y lanes, added onto acc (and, for
 // int8 rows, the biases onto bias_acc), row vectors v0 .. v0 + VPP - 1 of every lane.  Called by a whole
@@ -179,7 +173,11 @@ template <typename R> __device__ __forceinline__ int windows_of(const int row) {
 //    a lookup reads zeros from beyond it: a round is straight-line code whether its bags are full,
 //    partial or empty, the loop's control is scalar, and there is one copy of the body.  (Rounds with a
 //    branch around each load and each add, for int8 rows with a wait for the row's scale in each of
-//    them, were most of the rounds of teams that share a wavefront.)
+//    them, were most of the rounds of teams that share a wavefront.)  Rounds with a row beyond the window load
+//    by 64-bit addresses, as many loads in the same order, so that the sums wait for the same counts (one
+//    feature, tables of 2 / 5 / 20 / 40 GB: fp32 x 128 13.2 / 13.7 / 13.8 / 13.8 us, fp16 x 64 11.4 / 13.8 / 14.0 /
+//    14.1, int8 x 128 14.4 / 14.6 / 14.8 / 14.7; one window of the table after another, a pass each: fp16 12.3 /
+//    21.0 / 42.6 / 71.3).
 //  * Codes of int8 rows are multiplied as they lie (accumulate).
 // Measured, same bits: 200 int8 features (16 384 samples) 1 560 -> 1 405 us, 400 fp16 (8 192) 4 115 -> 4 015,
 // 100 fp32 features (tuned, 2 048) 121.4 -> 118.9, (default schedules, 1 337) 94.0 -> 90.1, 2 500 (256)
@@ -219,20 +217,21 @@ sum_lookups(float (&acc)[UB][VPP][EPV], float (&bias_acc)[UB], const char *__res
       }
   };
   fetch(held, 0);
+  const RowWindow<R> window(table);
   int at = 0;                 // the chunk's next lookup of every lookup lane (G > U: several rounds)
-  int windows = 1;            // of the table, that this chunk's rows lie in
+  bool far = false;           // a row of this chunk lies beyond the window
 
   for (int base = 0; base < len_most; base += U * Y) {
     const bool chunk_begins = G <= U || at == 0;
     if (chunk_begins) {
-      windows = 1;
+      far = false;
 #pragma unroll
       for (int i = 0; i < UB; ++i)
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
           // (here and not as it is fetched: the rows in flight would wait for it)
           held[i][c] = max(held[i][c], -1);
-          windows = max(windows, windows_of<R>(held[i][c]));
+          far = far || RowWindow<R>::beyond(held[i][c]);
         }
     }
     int idx[UB][U];
@@ -243,44 +242,63 @@ sum_lookups(float (&acc)[UB][VPP][EPV], float (&bias_acc)[UB], const char *__res
         idx[i][u] = group_lane<G>(held[i][u / G], (G > U ? at : 0) + u % G, lane);
     if constexpr (G > U) at = at + U == G ? 0 : at + U;
 
-    int w = 0;
-    do {
-      const RowWindow<R> window(table, w);
-      Vec<VB> buf[UB][U][VPP];
-      uint32_t sb[UB][U];
+    Vec<VB> buf[UB][U][VPP];
+    uint32_t sb[UB][U];
+    if (__builtin_expect(!far, 1)) {
 #pragma unroll
       for (int i = 0; i < UB; ++i)
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          int r = idx[i][u];
-          if (__builtin_expect(windows > 1, 0)) {
-            r = window.local(r, w);
-            asm volatile("" : "+v"(r));         // (keeps it a branch: nearly every table has one window)
-          }
-          const int row = row_offset<R::STRIDE>(r);
+          const int row = row_offset<R::STRIDE>(idx[i][u]);
 #pragma unroll
           for (int v = 0; v < VPP; ++v) {
             const int c = x + (v0 + v) * X;
             if (v0 + v < VPL && (WHOLE || c < R::V))
               buf[i][u][v] = window.template load<VB>(row + x * VB, (v0 + v) * X * VB);
           }
-          if constexpr (DT == I8) sb[i][u] = window.template load<4>(row, D).w[0];
+          if constexpr (DT == I8) {
+            sb[i][u] = window.template load<4>(row, D).w[0];
+            __builtin_amdgcn_sched_barrier(0);
+          }
         }
-      // the next chunk, behind the first rows of this one
-      if (chunk_begins && w == 0) fetch(coming, base + NC * G * Y);
+    } else {
 #pragma unroll
       for (int i = 0; i < UB; ++i)
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const float scale = DT == I8 ? code_scale(sb[i][u]) : 1.f;
 #pragma unroll
           for (int v = 0; v < VPP; ++v) {
             const int c = x + (v0 + v) * X;
-            if (v0 + v < VPL && (WHOLE || c < R::V)) accumulate<DT, VB>(acc[i][v], buf[i][u][v], scale);
+            if (v0 + v < VPL && (WHOLE || c < R::V)) buf[i][u][v] = load_far<R, VB>(table, idx[i][u], c * VB);
           }
-          if constexpr (DT == I8) bias_acc[i] = add_half<1>(bias_acc[i], sb[i][u]);
+          if constexpr (DT == I8) sb[i][u] = load_far<R, 4>(table, idx[i][u], D).w[0];
         }
-    } while (__builtin_expect(++w < windows, 0));
+    }
+    // the next chunk, behind the first rows of this one
+    if (chunk_begins) fetch(coming, base + NC * G * Y);
+    if (__builtin_expect(far, 0)) {
+#pragma unroll
+      for (int i = 0; i < UB; ++i)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+          for (int v = 0; v < VPP; ++v)
+            if (v0 + v < VPL && (WHOLE || x + (v0 + v) * X < R::V)) zero_far(buf[i][u][v], idx[i][u]);
+          if constexpr (DT == I8) sb[i][u] = idx[i][u] < 0 ? 0u : sb[i][u];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < UB; ++i)
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float scale = DT == I8 ? code_scale(sb[i][u]) : 1.f;
+#pragma unroll
+        for (int v = 0; v < VPP; ++v) {
+          const int c = x + (v0 + v) * X;
+          if (v0 + v < VPL && (WHOLE || c < R::V)) accumulate<DT, VB>(acc[i][v], buf[i][u][v], scale);
+        }
+        if constexpr (DT == I8) bias_acc[i] = add_half<1>(bias_acc[i], sb[i][u]);
+      }
     if (G <= U || at == 0) {
 #pragma unroll
       for (int i = 0; i < UB; ++i)
@@ -740,6 +758,7 @@ block_sum_range(BlockBagStorage<BT, DT, D, X, CHUNK> &s, const char *__restrict_
   const int x = tid - y * X;
   const int wave = tid / 64;
   const int lane = tid - wave * 64;
+  const RowWindow<R> window(table);
 
   float acc[VPL][EPV];
   float bias_acc = 0.f;
@@ -797,20 +816,21 @@ block_sum_range(BlockBagStorage<BT, DT, D, X, CHUNK> &s, const char *__restrict_
           idx[u] = p < n ? max(chunk[p], -1) : -1;
           highest = max(highest, idx[u]);
         }
-        const int windows = windows_of<R>(highest);
-        int w = 0;
-        do {
-          const RowWindow<R> window(table, w);
-          Vec<VB> buf[U][VPL];
-          uint32_t sb[U];
+        Vec<VB> buf[U][VPL];
+        uint32_t sb[U];
+        auto add = [&](const int u) {
+          const float scale = DT == I8 ? code_scale(sb[u]) : 1.f;
+#pragma unroll
+          for (int v = 0; v < VPL; ++v) {
+            const int c = x + v * X;
+            if (WHOLE || c < R::V) accumulate<DT, VB>(sum[v], buf[u][v], scale);
+          }
+          if constexpr (DT == I8) bias_sum = add_half<1>(bias_sum, sb[u]);
+        };
+        if (__builtin_expect(!RowWindow<R>::beyond(highest), 1)) {
 #pragma unroll
           for (int u = 0; u < U; ++u) {
-            int r = idx[u];
-            if (__builtin_expect(windows > 1, 0)) {
-              r = window.local(r, w);
-              asm volatile("" : "+v"(r));       // (keeps it a branch)
-            }
-            const int row = row_offset<R::STRIDE>(r);
+            const int row = row_offset<R::STRIDE>(idx[u]);
 #pragma unroll
             for (int v = 0; v < VPL; ++v) {
               const int c = x + v * X;
@@ -819,16 +839,35 @@ block_sum_range(BlockBagStorage<BT, DT, D, X, CHUNK> &s, const char *__restrict_
             if constexpr (DT == I8) sb[u] = window.template load<4>(row, D).w[0];
           }
 #pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const float scale = DT == I8 ? code_scale(sb[u]) : 1.f;
+          for (int u = 0; u < U; ++u) add(u);
+        } else {
+          // (four at a time, their indices read again: a round of eight leaves no registers for 64-bit addresses; one
+          // feature, tables of 2 / 5 / 20 / 40 GB 18.2 / 19.0 / 20.0 / 19.9 us)
+          constexpr int FEW = U % 4 == 0 ? 4 : U;
+#pragma unroll 1
+          for (int u0 = 0; u0 < U; u0 += FEW) {
+            int r[FEW];
 #pragma unroll
-            for (int v = 0; v < VPL; ++v) {
-              const int c = x + v * X;
-              if (WHOLE || c < R::V) accumulate<DT, VB>(sum[v], buf[u][v], scale);
+            for (int f = 0; f < FEW; ++f) {
+              const int p = base + (u0 + f) * Y + y;
+              r[f] = p < n ? chunk[p] : -1;
+#pragma unroll
+              for (int v = 0; v < VPL; ++v) {
+                const int c = x + v * X;
+                if (WHOLE || c < R::V) buf[f][v] = load_far<R, VB>(table, r[f], c * VB);
+              }
+              if constexpr (DT == I8) sb[f] = load_far<R, 4>(table, r[f], D).w[0];
             }
-            if constexpr (DT == I8) bias_sum = add_half<1>(bias_sum, sb[u]);
+#pragma unroll
+            for (int f = 0; f < FEW; ++f) {
+#pragma unroll
+              for (int v = 0; v < VPL; ++v)
+                if (WHOLE || x + v * X < R::V) zero_far(buf[f][v], r[f]);
+              if constexpr (DT == I8) sb[f] = r[f] < 0 ? 0u : sb[f];
+              add(f);
+            }
           }
-        } while (__builtin_expect(++w < windows, 0));
+        }
       }
 #pragma unroll
       for (int v = 0; v < VPL; ++v)

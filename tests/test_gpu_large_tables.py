@@ -1,5 +1,6 @@
-"""Tables of more than 4 GB, whose rows 32-bit offsets do not reach from the table's start: the bodies
-take them in windows (rfx::RowWindow).  Integer-valued rows, so that sums are exact in any order."""
+"""Tables of more than 4 GB, whose rows 32-bit offsets do not reach from the table's start: rounds with a row
+beyond the first 4 GB (rfx::RowWindow) load by 64-bit addresses.  Integer-valued rows, so that sums are exact in any
+order."""
 
 import numpy as np
 import pytest
@@ -15,7 +16,7 @@ def _window_rows(stride: int) -> int:
 
 
 def _rows_to_look_up(spec, stride, rng):
-    """Rows around the ends of the table and of every window, and some anywhere."""
+    """Rows around the ends of the table and of every 4 GB of it, and some anywhere."""
     edges = [0, 1, spec.rows - 2, spec.rows - 1]
     window = _window_rows(stride)
     assert spec.rows > window
