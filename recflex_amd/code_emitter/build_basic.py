@@ -49,6 +49,14 @@ class BasicBuilder:
     def host_lib_path(self, dirname: str = "build") -> str:
         return os.path.join(self.csrc_dir, dirname, "librecflex_host.so")
 
+    def strings_build(self) -> List[str]:
+        """What the reader of Python's own strings adds to the compiler's arguments; nothing where this
+        interpreter's headers are not installed."""
+        include = sysconfig.get_paths()["include"]
+        if not os.path.exists(os.path.join(include, "Python.h")) or not os.path.exists(self.strings_source):
+            return []
+        return [self.strings_source, f"-I{include}"]
+
     def build(self, dirname: str = "build", force: bool = False) -> str:
         """Build ``librecflex_host.so`` if missing (or ``force``); returns its path."""
         lib = self.host_lib_path(dirname)
@@ -56,11 +64,9 @@ class BasicBuilder:
             os.makedirs(os.path.dirname(lib), exist_ok=True)
             tmp = lib + f".tmp{os.getpid()}"
             cmd = [self.cxx, *self.host_flags, "-O3", f"-I{self.abi_include}", self.host_source, "-o", tmp]
-            # the reader of Python's own strings, where its headers are installed
-            python_include = sysconfig.get_paths()["include"]
-            if os.path.exists(os.path.join(python_include, "Python.h")) and os.path.exists(self.strings_source):
-                with_strings = subprocess.run([*cmd, self.strings_source, f"-I{python_include}"],
-                                              stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+            strings = self.strings_build()
+            if strings:
+                with_strings = subprocess.run([*cmd, *strings], stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
                 if with_strings.returncode == 0:
                     os.replace(tmp, lib)
                     return lib

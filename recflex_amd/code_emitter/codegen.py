@@ -1100,6 +1100,7 @@ extern "C" int recom_host_preprocess_feat(
         add_subdirs = '\n'.join(f"add_subdirectory({subdir})" for subdir in subdirs)
         # the device side is header-only: a change of a schedule template rebuilds the library
         device_headers = " ".join(basic.device_headers())
+        strings = basic.strings_build()
 
         recom = f'''
 add_custom_command(
@@ -1115,9 +1116,9 @@ add_custom_target(recom ALL DEPENDS ${{CMAKE_BINARY_DIR}}/librecom.so)
 add_custom_command(
   OUTPUT ${{CMAKE_BINARY_DIR}}/recom_host.so
   COMMAND {basic.cxx} {" ".join(basic.host_flags)} {opt} {inc_flags}
-          ${{CMAKE_SOURCE_DIR}}/{host_fname} {basic.host_source} {host_link_flags}
+          ${{CMAKE_SOURCE_DIR}}/{host_fname} {basic.host_source} {" ".join(strings)} {host_link_flags}
           -o ${{CMAKE_BINARY_DIR}}/recom_host.so
-  DEPENDS ${{CMAKE_SOURCE_DIR}}/{host_fname} {basic.host_source}
+  DEPENDS ${{CMAKE_SOURCE_DIR}}/{host_fname} {basic.host_source} {" ".join(strings[:1])}
   VERBATIM)
 add_custom_target(recom_host ALL DEPENDS ${{CMAKE_BINARY_DIR}}/recom_host.so)
 ''' if host_fname else ''

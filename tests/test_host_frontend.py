@@ -5,8 +5,11 @@ import numpy as np
 import pytest
 
 from helpers import oracle
+from recflex_amd.code_emitter import CodeEmitter, MetaData
 from recflex_amd.code_emitter.build_basic import BasicBuilder
 from recflex_amd.host import RecomHost, RecomHostError
+from recflex_amd.model_build import default_feat_schedules
+from recflex_amd.utils import compile_build
 
 
 @pytest.fixture(scope="module")
@@ -221,3 +224,19 @@ def test_strings_that_are_not_plain_are_left_to_the_joined_text(host):
                   ["1"], [None, "1"]):
         assert host._parse_strings([lines], 2, counts, at) is None
     assert host._parse_strings(np.array([["1", "2"]]), 2, counts, at) is None
+
+
+def test_a_generated_library_reads_the_strings_where_they_lie(tmp_path, host):
+    """``recom_host.so`` as a model's CMake project builds it, the library that the examples load."""
+    if not BasicBuilder().strings_build():
+        pytest.skip("no Python headers")
+    fs = default_feat_schedules([MetaData(8, "float"), MetaData(16, "half")], [3.0, 5.0])
+    emitter = CodeEmitter(fs)
+    emitter.emit_host(str(tmp_path / "preprocess.cpp"))
+    emitter.emit_cmake_list(str(tmp_path / "CMakeLists.txt"), code_fname=None, host_fname="preprocess.cpp")
+    compile_build(str(tmp_path / "build"))
+    generated = RecomHost(str(tmp_path / "build" / "recom_host.so"))
+    raw = [["1,2", "", "3"], ["4", "5,6,7", ""]]
+    counts, at = np.empty(2, np.int64), np.zeros(3, np.int64)
+    got = generated._parse_strings(raw, 3, counts, at)
+    assert got is not None and np.array_equal(got, host._parse_joined(raw, 3, counts.copy(), at.copy()))
