@@ -11,7 +11,9 @@ import hashlib
 import os
 import shutil
 import subprocess
+import sys
 import sysconfig
+import warnings
 from typing import List
 
 import recflex_amd
@@ -58,35 +60,39 @@ class BasicBuilder:
         return [self.strings_source, f"-I{include}"]
 
     def build(self, dirname: str = "build", force: bool = False) -> str:
-        """Build ``librecflex_host.so`` if missing (or ``force``); returns its path."""
+        """Build ``librecflex_host.so`` if it is missing or was built from other sources, with other flags or
+        for another interpreter's strings (or ``force``); returns its path."""
         lib = self.host_lib_path(dirname)
-        if force or not os.path.exists(lib):
-            os.makedirs(os.path.dirname(lib), exist_ok=True)
-            tmp = lib + f".tmp{os.getpid()}"
-            cmd = [self.cxx, *self.host_flags, "-O3", f"-I{self.abi_include}", self.host_source, "-o", tmp]
-            strings = self.strings_build()
+        strings = self.strings_build()
+        sources = [self.host_source, self.strings_source, os.path.join(self.abi_include, "recflex_hip.h")]
+        flags = [*self.host_flags, "-O3"]
+        interpreter = [sys.implementation.cache_tag or "", *strings[1:]] if strings else []
+
+        def compile_to(tmp):
+            cmd = [self.cxx, *flags, f"-I{self.abi_include}", self.host_source, "-o", tmp]
             if strings:
-                with_strings = subprocess.run([*cmd, *strings], stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
-                if with_strings.returncode == 0:
-                    os.replace(tmp, lib)
-                    return lib
+                done = subprocess.run([*cmd, *strings], stdout=subprocess.DEVNULL, stderr=subprocess.PIPE, text=True)
+                if done.returncode == 0:
+                    return
+                warnings.warn("the reader of Python's strings does not compile, sample lines are joined first:\n"
+                              + done.stderr[-2000:], RuntimeWarning, stacklevel=3)
             subprocess.run(cmd, check=True)
-            os.replace(tmp, lib)
-        return lib
 
-    def mlp_lib_path(self, dirname: str = "build") -> str:
-        return os.path.join(self.csrc_dir, dirname, "librecflex_mlp.so")
+        try:
+            return self._build_from(lib, sources, [*flags, *interpreter], force, compile_to)
+        except (OSError, subprocess.SubprocessError) as e:      # no compiler, nowhere to write, ...
+            if force or not os.path.exists(lib):
+                raise
+            warnings.warn(f"{lib} was built from other sources and could not be built again: {e}", RuntimeWarning,
+                          stacklevel=2)
+            return lib
 
-    def build_mlp(self, dirname: str = "build", force: bool = False) -> str:
-        """Build ``librecflex_mlp.so`` (the kernels of ``RecomModel``'s MLP, model independent) if it is
-        missing or was built from another source or with other flags (or ``force``); returns its path."""
-        lib = self.mlp_lib_path(dirname)
-        sources = [os.path.join(self.csrc_dir, "mlp", n) for n in ("recflex_mlp.hip", "recflex_mlp.h")]
+    def _build_from(self, lib: str, sources: List[str], flags: List[str], force: bool, compile_to) -> str:
+        """``lib``, made anew by ``compile_to(path)`` unless it is there, from these sources and flags."""
         if not force and os.path.exists(lib) and not all(map(os.path.exists, sources)):
             return lib                              # a package without its sources
-        flags = [*self.hip_flags, "-O3"]
         key = hashlib.sha256(" ".join(flags).encode())
-        for path in sources:
+        for path in filter(os.path.exists, sources):
             with open(path, "rb") as f:
                 key.update(f.read())
         built_from = lib + ".from"                  # what the library beside it was built from
@@ -97,9 +103,20 @@ class BasicBuilder:
         if force or current != key.hexdigest():
             os.makedirs(os.path.dirname(lib), exist_ok=True)
             tmp = lib + f".tmp{os.getpid()}"
-            subprocess.run([self.hipcc, *flags, sources[0], "-o", tmp], check=True)
+            compile_to(tmp)
             os.replace(tmp, lib)
             with open(tmp, "w") as f:
                 f.write(key.hexdigest())
             os.replace(tmp, built_from)
         return lib
+
+    def mlp_lib_path(self, dirname: str = "build") -> str:
+        return os.path.join(self.csrc_dir, dirname, "librecflex_mlp.so")
+
+    def build_mlp(self, dirname: str = "build", force: bool = False) -> str:
+        """Build ``librecflex_mlp.so`` (the kernels of ``RecomModel``'s MLP, model independent) if it is
+        missing or was built from another source or with other flags (or ``force``); returns its path."""
+        sources = [os.path.join(self.csrc_dir, "mlp", n) for n in ("recflex_mlp.hip", "recflex_mlp.h")]
+        flags = [*self.hip_flags, "-O3"]
+        return self._build_from(self.mlp_lib_path(dirname), sources, flags, force,
+                                lambda tmp: subprocess.run([self.hipcc, *flags, sources[0], "-o", tmp], check=True))

@@ -1,6 +1,10 @@
 """CPU text front end (librecflex_host.so, recom_host_* in include/recflex_hip.h) against the
 oracle's restatement of the reference's line splitter, plus the packed-buffer layout."""
 
+import os
+import shutil
+import sys
+
 import numpy as np
 import pytest
 
@@ -240,3 +244,50 @@ def test_a_generated_library_reads_the_strings_where_they_lie(tmp_path, host):
     counts, at = np.empty(2, np.int64), np.zeros(3, np.int64)
     got = generated._parse_strings(raw, 3, counts, at)
     assert got is not None and np.array_equal(got, host._parse_joined(raw, 3, counts.copy(), at.copy()))
+
+
+@pytest.fixture
+def builder(tmp_path):
+    b = BasicBuilder()
+    (tmp_path / "host").mkdir()
+    for name in ("host_source", "strings_source"):
+        setattr(b, name, shutil.copy(getattr(b, name), tmp_path / "host"))
+    b.csrc_dir = str(tmp_path)
+    return b
+
+
+def test_host_library_follows_its_sources(builder, monkeypatch):
+    """Built when it is missing, kept as long as sources, flags and interpreter are what it was built from."""
+    def edit(path):
+        with open(path, "a") as f:
+            f.write("\n// edited\n")
+
+    lib = builder.build()
+    steps = [(lambda: None, False), (lambda: edit(builder.host_source), True), (lambda: None, False),
+             (lambda: builder.host_flags.append("-DX"), True)]
+    if builder.strings_build():
+        steps += [(lambda: edit(builder.strings_source), True),
+                  (lambda: monkeypatch.setattr(sys.implementation, "cache_tag", "cpython-000"), True)]
+    for change, again in steps + [(lambda: None, False)]:
+        change()
+        built = os.stat(lib).st_ino
+        assert builder.build() == lib and (os.stat(lib).st_ino != built) is again
+    os.unlink(lib + ".from")                        # a library of before this was kept
+    built = os.stat(lib).st_ino
+    builder.build()
+    assert os.stat(lib).st_ino != built
+    builder.cxx = "/no/such/compiler"
+    builder.build()
+    builder.host_flags.append("-DY")
+    with pytest.warns(RuntimeWarning, match="could not be built again"):
+        assert builder.build() == lib
+
+
+def test_a_string_reader_that_does_not_compile_is_named(builder):
+    if not builder.strings_build():
+        pytest.skip("no Python headers")
+    with open(builder.strings_source, "a") as f:
+        f.write("not c++\n")
+    with pytest.warns(RuntimeWarning, match="not c"):
+        host = RecomHost(builder.build())
+    assert host._strings is None and np.array_equal(host.parse_lines(["1,2"])[0], [1, 2])
