@@ -124,8 +124,16 @@ template <typename Body> void for_all_features(int32_t num_features, int64_t lin
 
 extern "C" {
 
-// The interpreter whose objects this was built to read: PY_MAJOR_VERSION * 256 + PY_MINOR_VERSION.
-int recom_host_strings_python() { return PY_MAJOR_VERSION * 256 + PY_MINOR_VERSION; }
+// The interpreter whose objects this was built to read: PY_MAJOR_VERSION * 256 + PY_MINOR_VERSION, and 65536
+// more where objects begin with the links of Py_TRACE_REFS.
+int recom_host_strings_python() {
+#ifdef Py_TRACE_REFS
+  constexpr int links = 65536;
+#else
+  constexpr int links = 0;
+#endif
+  return links + PY_MAJOR_VERSION * 256 + PY_MINOR_VERSION;
+}
 
 // raw: num_features lists (or tuples) of `batch` str each, in one.  num_indices_out[f]: the indices
 // of feature f.  0, or 1 where something is not plain.

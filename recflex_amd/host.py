@@ -56,7 +56,8 @@ def _string_reader(path: str):
     lib = ctypes.PyDLL(path)
     if sys.implementation.name != "cpython" or not hasattr(lib, "recom_host_parse_strings") \
             or getattr(sys, "_is_gil_enabled", lambda: True)() is False \
-            or lib.recom_host_strings_python() != sys.version_info[0] * 256 + sys.version_info[1]:
+            or lib.recom_host_strings_python() != sys.version_info[0] * 256 + sys.version_info[1] \
+            + (65536 if hasattr(sys, "getobjects") else 0):
         return None
     lib.recom_host_count_strings.restype = ctypes.c_int
     lib.recom_host_count_strings.argtypes = [ctypes.py_object, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p]

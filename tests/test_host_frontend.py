@@ -293,3 +293,15 @@ def test_a_string_reader_that_does_not_compile_is_named(builder):
     with pytest.warns(RuntimeWarning, match="not c"):
         host = RecomHost(builder.build())
     assert host._strings is None and np.array_equal(host.parse_lines(["1,2"])[0], [1, 2])
+
+
+def test_another_interpreters_strings_are_not_read(host, monkeypatch):
+    """Of another version, or with other objects (sys.getobjects is there if they begin with links)."""
+    if host._strings is None:
+        pytest.skip("no reader of strings for this interpreter")
+    assert RecomHost(host.path)._strings is not None
+    with monkeypatch.context() as m:
+        m.setattr(sys, "getobjects", lambda n: [], raising=False)
+        assert RecomHost(host.path)._strings is None
+    monkeypatch.setattr(sys, "version_info", (3, 99, 0))
+    assert RecomHost(host.path)._strings is None
