@@ -179,6 +179,11 @@ class ScheduleBase(ABC):
     def GenParamCandidates(self, stats: InputStats = None) -> List:
         pass
 
+    def GenFurtherCandidates(self) -> List:
+        """More parameters to try, proposed behind the candidates of all of a feature's templates: the numbers
+        that a tuning directory's files know those by stay what they were."""
+        return []
+
     def UsedArgCounts(self) -> Tuple[int, int]:
         # data vectors: offsets, indices; scalars: num_inputs, num_segments
         # (same counts as the reference's bag schedules, warp_per_sample.py:78-81)

@@ -66,6 +66,12 @@ class BlockPerBagSchedule(ScheduleBase):
         return 1
 
     def GenParamCandidates(self, stats: InputStats = None) -> List[BlockPerBagParams]:
+        return self._with_items((1, 2, 4))
+
+    def GenFurtherCandidates(self) -> List[BlockPerBagParams]:
+        return self._with_items((8,))
+
+    def _with_items(self, in_flight) -> List[BlockPerBagParams]:
         m = self.meta
         out = []
         vmax = next_pow2(m.row_vectors)
@@ -75,7 +81,7 @@ class BlockPerBagSchedule(ScheduleBase):
                 continue
             if x * 4 < min(64, vmax):   # keep to the widest few column splits
                 continue
-            for items in (1, 2, 4):
+            for items in in_flight:
                 if items * vpl * m.vec_bytes // 4 > MAX_INFLIGHT_DWORDS:
                     continue
                 out.append(BlockPerBagParams(x, items, 4 * self.block_threads))

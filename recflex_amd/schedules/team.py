@@ -151,6 +151,12 @@ class ThreadPerBagSchedule(TeamScheduleBase):
                         out.append(p)
         return out
 
+    def GenFurtherCandidates(self) -> List[ThreadPerBagParams]:
+        """Eight lookups in flight, for one bag per lane."""
+        m = self.meta
+        eight = [ThreadPerBagParams(8, 1, vpp) for vpp in passes_for(m.row_vectors, m)]
+        return [p for p in eight if m.payload_bytes <= 256 and fits_registers(m, self.team_params(p))]
+
 
 class SubWavefrontPerBagSchedule(TeamScheduleBase):
     """2..32 lanes per bag."""

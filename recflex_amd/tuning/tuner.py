@@ -268,6 +268,9 @@ class Tuner:
             for schedule in self.feat_schedules[feat_id]:
                 for params in schedule.GenParamCandidates():
                     self.feat_sched_param_candidates[feat_id].append([schedule, params])
+            for schedule in self.feat_schedules[feat_id]:
+                for params in schedule.GenFurtherCandidates():
+                    self.feat_sched_param_candidates[feat_id].append([schedule, params])
             if not self.feat_sched_param_candidates[feat_id]:
                 # e.g. a template whose parameter space has no member for rows this wide: tune
                 # nothing for this feature, run the default schedule
@@ -870,7 +873,10 @@ class Tuner:
             for occupancy in tune_config.occupancies:
                 output_dir, build_dir = self.get_output_build_dir(feat_id, occupancy)
                 with open(f"{output_dir}/result.txt") as f:     # absent if the worker failed
-                    results[feat_id][occupancy] = list(map(float, f.read().strip().split(' ')))
+                    times = list(map(float, f.read().strip().split(' ')))
+                # (fewer in a file from before there were as many candidates)
+                missing = len(self.feat_sched_param_candidates[feat_id]) - len(times)
+                results[feat_id][occupancy] = times + [float("inf")] * missing
         return results
 
     def cluster_validation(self, occupancy: int, tune_config: TuneConfig) -> dict:

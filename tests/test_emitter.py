@@ -7,6 +7,8 @@ import re
 import pytest
 
 from recflex_amd.code_emitter import CodeEmitter, MetaData, ScheduleBase
+from recflex_amd.model_build import feat_schedules_from_entries
+from recflex_amd.prebuilt import TUNED_DIR
 from recflex_amd.schedules import (SCHEDULE_MAPPING, BlockPerBagParams, BlockPerBagSchedule,
                                    SubWavefrontPerBagParams, SubWavefrontPerBagSchedule,
                                    ThreadPerBagSchedule, WavefrontPerBagParams,
@@ -50,7 +52,7 @@ def test_candidates_are_valid_and_emit(dt, dim):
     total = 0
     for cls in (ThreadPerBagSchedule, SubWavefrontPerBagSchedule, WavefrontPerBagSchedule, BlockPerBagSchedule):
         sched = cls(meta, 256)
-        for p in sched.GenParamCandidates():
+        for p in sched.GenParamCandidates() + sched.GenFurtherCandidates():
             body = sched.EmitScheduleBody(p)          # raises on invalid parameters
             assert "rfx::" in body
             g = sched.TileGranularity(p)
@@ -61,6 +63,22 @@ def test_candidates_are_valid_and_emit(dt, dim):
                 assert tp.lanes_x * tp.lanes_y <= 64
             total += 1
     assert 4 <= total <= 200
+
+
+@pytest.mark.parametrize("dt", ["float", "half", "int8"])
+def test_the_tuner_can_propose_the_default_schedules(dt):
+    for dim in (4, 8, 16, 32, 64, 96, 128, 192, 256, 512):
+        for mean in (0.5, 2, 4, 8, 16, 23, 30, 64, 95, 96, 200, 511, 512, 5000):
+            sched, params = default_schedule(MetaData(dim, dt), mean, 256)
+            assert params in sched.GenParamCandidates() + sched.GenFurtherCandidates(), (dim, mean, type(sched).__name__, params)
+
+
+@pytest.mark.parametrize("name", ["c2", "c3", "c4", "c5", "refa", "reff4"])
+def test_the_tuner_can_propose_the_tuned_schedules(name):
+    with open(os.path.join(TUNED_DIR, f"{name}_schedule.json")) as f:
+        entries = json.load(f)["schedules"]
+    for sched, params in feat_schedules_from_entries(entries):
+        assert params in sched.GenParamCandidates() + sched.GenFurtherCandidates(), (type(sched).__name__, sched.meta, params)
 
 
 def test_invalid_params_rejected():

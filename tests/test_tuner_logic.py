@@ -11,7 +11,8 @@ import pytest
 
 from helpers import oracle
 from recflex_amd.code_emitter import MetaData
-from recflex_amd.schedules import SCHEDULE_MAPPING, WarpPerSampleSchedule, OneHotSchedule
+from recflex_amd.schedules import (SCHEDULE_MAPPING, BlockPerBagSchedule, OneHotSchedule, SubWavefrontPerBagSchedule,
+                                   ThreadPerBagSchedule, WarpPerSampleSchedule)
 from recflex_amd.tuning import BasicConfig, TuneConfig, Tuner
 from recflex_amd.tuning.tuner import padded_sched_num
 from recflex_amd.tuning.measure import load_batches, tiles_per_feature
@@ -42,6 +43,27 @@ def test_padding_matches_reference_rule(tmp_path):
     cands = t.feat_sched_param_candidates[0]
     padded = t.pad_sched_params(cands, 2 * len(cands) + 3)
     assert padded == oracle.pad_sched_params(cands, 2 * len(cands) + 3)
+
+
+def test_further_candidates_come_behind_all_others(tmp_path):
+    """The numbers that a tuning directory's files know candidates by do not move, and a result file with fewer
+    numbers than there are candidates knows nothing of the others."""
+    t = _tiny_tuner(tmp_path, feats=1)
+    t.feat_schedules[0] = [cls(t.metas[0], 256) for cls in (ThreadPerBagSchedule, SubWavefrontPerBagSchedule,
+                                                            BlockPerBagSchedule)]
+    t.gen_feat_sched_param_candidates()
+    cands = t.feat_sched_param_candidates[0]
+    first = [(s, p) for s in t.feat_schedules[0] for p in s.GenParamCandidates()]
+    assert [tuple(c) for c in cands[:len(first)]] == first
+    assert {type(s).__name__ for s, _ in cands[len(first):]} == {"ThreadPerBagSchedule", "BlockPerBagSchedule"}
+    cfg = TuneConfig(occupancies=[4], gpu_ids=[0], sm_count=4, num_processes=1, in_process=True,
+                     interference="replicate")
+    t.compile_local = lambda cfg: None
+    out, _ = t.get_output_build_dir(0, 4)
+    os.makedirs(out)
+    with open(f"{out}/result.txt", "w") as f:
+        f.write(" ".join(["2.0"] * len(first)))
+    assert t.tune(cfg)[0][4] == [2.0] * len(first) + [float("inf")] * (len(cands) - len(first))
 
 
 def test_selection_is_argmin_per_occupancy(tmp_path):
