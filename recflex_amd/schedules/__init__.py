@@ -91,11 +91,13 @@ def default_schedule(meta: MetaData, mean_bag_len: float = 1.0, block_threads: i
         # the whole workgroup on one bag, one row vector per lane -- and several workgroups per
         # bag when the batch holds so few bags that one of them is a good part of a workgroup's
         # share (8 features x 64 bags x 4 000 lookups: 105 us against 203 us with a team per bag);
-        # eight fp32 vectors in flight per lane (8 features, 1 bag of 28 000 lookups 17.8 us with
-        # four and 16.0, 16 of 20 000 73.5 and 72.2, 128 of 2 000 61.4 and 60.9)
-        return (SplitBagSchedule(meta, block_threads),
-                BlockPerBagParams(min(64, next_pow2(v)), 8 if meta.elems_per_vector <= 4 else 2,
-                                  4 * block_threads))
+        # eight lookups in flight per lane for fp32 rows (8 features, 1 bag of 28 000 lookups 17.8 us
+        # with four and 16.0, 16 of 20 000 73.5 and 72.2, 128 of 2 000 61.4 and 60.9), four where a
+        # lane has more than two vectors of them: eight spill (8 features, 16 bags of 4 000: 512
+        # columns 154 us either way, 768 247 with four and 261, 1 024 340 and 382)
+        lanes = min(64, next_pow2(v))
+        items = 2 if meta.elems_per_vector > 4 else (8 if v <= 2 * lanes else 4)
+        return SplitBagSchedule(meta, block_threads), BlockPerBagParams(lanes, items, 4 * block_threads)
     items = max(1, (8 if meta.elems_per_vector <= 4 else 4) // vpl)
     items = 1 << (items.bit_length() - 1)
     if items * y >= 2 * mean_bag_len and meta.elems_per_vector != 8:

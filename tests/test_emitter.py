@@ -67,7 +67,7 @@ def test_candidates_are_valid_and_emit(dt, dim):
 
 @pytest.mark.parametrize("dt", ["float", "half", "int8"])
 def test_the_tuner_can_propose_the_default_schedules(dt):
-    for dim in (4, 8, 16, 32, 64, 96, 128, 192, 256, 512):
+    for dim in (4, 8, 16, 32, 64, 96, 128, 192, 256, 512, 768, 1024):
         for mean in (0.5, 2, 4, 8, 16, 23, 30, 64, 95, 96, 200, 511, 512, 5000):
             sched, params = default_schedule(MetaData(dim, dt), mean, 256)
             assert params in sched.GenParamCandidates() + sched.GenFurtherCandidates(), (dim, mean, type(sched).__name__, params)
