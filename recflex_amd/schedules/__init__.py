@@ -50,12 +50,14 @@ def default_schedule(meta: MetaData, mean_bag_len: float = 1.0, block_threads: i
     template): enough
     column lanes that a lane owns one or two 16-byte vectors, lookup lanes only for long bags,
     and eight row vectors in flight per lane, four for fp16 and int8 rows with their 8 or 16
-    accumulators per vector, half as many where the bags hold few lookups (measured at four
-    workgroups per CU, us per launch with half as many in flight and with these: 1 000 fp32
-    features 85 and 79 at 256 samples, 31.9 and 27.6 at 64; 100 fp32 features 318 and 313 at
-    6 000; 200 int8 features 1 529 and 1 404 at 16 384, 17.1 and 14.7 at 64.  Eight for fp16
-    rows: 400 features 388 instead of 394 at 512 samples, but 4 624 instead of 4 299 at 8 192;
-    for int8 rows 13.7 and 1 461)."""
+    accumulators per vector, half as many of fp32 and int8 rows where the bags hold few lookups
+    (measured at four workgroups per CU, us per launch with half as many in flight and with
+    these: 1 000 fp32 features 85 and 79 at 256 samples, 31.9 and 27.6 at 64; 100 fp32 features
+    318 and 313 at 6 000; 200 int8 features 1 529 and 1 404 at 16 384, 17.1 and 14.7 at 64.  Eight
+    for fp16 rows: 400 features 388 instead of 394 at 512 samples, but 4 624 instead of 4 299 at
+    8 192; for int8 rows 13.7 and 1 461.  200 features with bags of 1.8 lookups, 4 096 / 16 384
+    samples, half as many and not: fp16 116 / 405 and 110 / 394, int8 126 / 528 and 129 / 540, fp32
+    134 / 502 and 132 / 495)."""
     if one_hot:
         sched = OneHotBagSchedule(meta, block_threads)
         return sched, sched.default_params()
